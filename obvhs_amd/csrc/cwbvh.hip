@@ -740,7 +740,7 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
                                       items[(level + 1) & 1], in_pre, pres[(level + 1) & 1], level,
                                       order_children ? 1u : 0u, out->nodes.as<CwNode>(),
                                       out->prim_indices.as<uint32_t>(), ncw, n, misc, nullptr);
-        bound *= 8;
+        bound = cap * 8;  // never past 8 * ncw, however deep the tree
     }
     OBVHS_TRY(hipGetLastError(), "cwbvh emit launch");
     // the error word and the count of the level below the last (err and level_count are adjacent): one copy
@@ -813,7 +813,7 @@ obvhs_status cwbvh_convert_batch(obvhs_context* ctx, const Node32* nodes, const 
                                       pres[level & 1], pres[(level + 1) & 1], level, order_children ? 1u : 0u,
                                       out_nodes.as<CwNode>(), out_prims.as<uint32_t>(), 0u, 0u, misc,
                                       d_meshes);
-        bound *= 8;
+        bound = capl * 8;
     }
     OBVHS_TRY(hipGetLastError(), "batch cwbvh emit launch");
     uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
