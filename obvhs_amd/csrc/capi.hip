@@ -110,6 +110,7 @@ obvhs_status obvhs_context_destroy(obvhs_context* ctx) {
     S.clusters_b.release();
     S.keys.release();
     S.keys_hi.release();
+    S.tops.release();
     S.vals.release();
     S.merge.release();
     S.blocksums.release();

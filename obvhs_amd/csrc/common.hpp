@@ -25,6 +25,7 @@ enum : uint32_t {
     DERR_CW_PRIMCOUNT = 1u << 5,
     DERR_CW_DEPTH = 1u << 6,
     DERR_CAPACITY = 1u << 7,
+    DERR_RESORT = 1u << 8,  // internal: a build's top-word sort met a long run of equal tops (never a status)
 };
 
 // PLOC working cluster / compact BVH2 node: the obvhs `small_bvh2_node` layout (bvh2/node.rs:12-36), 32 bytes.

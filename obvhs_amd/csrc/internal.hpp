@@ -42,6 +42,7 @@ struct BuildScratch {
     DevBuf clusters_b;  // Node32[n]
     DevBuf keys;        // u64[n]
     DevBuf keys_hi;     // u64[n] high words of SortPrecision::U128 codes
+    DevBuf tops;        // u32[n] top 32 bits of the codes
     DevBuf vals;        // u32[n]
     DevBuf merge;       // i8[n]
     DevBuf blocksums;   // uint2[n/256+1]
@@ -127,6 +128,8 @@ hipError_t launch_iota(uint32_t* p, uint32_t n, hipStream_t stream);
 size_t radix_sort_scratch_bytes(uint32_t n);
 hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                             void* scratch, hipStream_t stream, int items);
+hipError_t radix_sort_pairs32(uint32_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
+                              void* scratch, hipStream_t stream, int items);
 // Size class of n primitives or keys (the tuning table's index).
 inline uint32_t size_class(uint64_t n) { return n < 4096u ? 0u : n < 65536u ? 1u : n < 1048576u ? 2u : 3u; }
 inline int sort_items_for(const obvhs_context* ctx, uint64_t n) { return (int)ctx->tune.sort_items[size_class(n)]; }

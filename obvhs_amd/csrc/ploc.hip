@@ -132,6 +132,13 @@ __global__ void __launch_bounds__(1024) k_reduce_bounds(const uint32_t* __restri
 }
 
 // Triangle::aabb = Aabb::from_points([v0, v1, v2]) (triangle.rs:28-30; aabb.rs:59-66).
+__device__ __forceinline__ Box tri_box(const float4& v0, const float4& v1, const float4& v2) {
+    const Box b{smin(v0.x, v1.x), smin(v0.y, v1.y), smin(v0.z, v1.z), smax(v0.x, v1.x), smax(v0.y, v1.y),
+                smax(v0.z, v1.z)};
+    return Box{smin(b.lx, v2.x), smin(b.ly, v2.y), smin(b.lz, v2.z), smax(b.hx, v2.x), smax(b.hy, v2.y),
+               smax(b.hz, v2.z)};
+}
+
 // iota_out (when the caller gave no indices): primitive_indices = 0..n-1, written here instead of by a launch of its own.
 __global__ void __launch_bounds__(T256) k_leaf_init_tris(const float4* __restrict__ tris,
                                                          const uint32_t* __restrict__ indices, uint32_t n,
@@ -145,11 +152,7 @@ __global__ void __launch_bounds__(T256) k_leaf_init_tris(const float4* __restric
     bool nan = false;
     if (valid) {
         float4 v0 = tris[3 * (size_t)i], v1 = tris[3 * (size_t)i + 1], v2 = tris[3 * (size_t)i + 2];
-        b = Box{v0.x, v0.y, v0.z, v0.x, v0.y, v0.z};
-        b = Box{smin(b.lx, v1.x), smin(b.ly, v1.y), smin(b.lz, v1.z), smax(b.hx, v1.x), smax(b.hy, v1.y),
-                smax(b.hz, v1.z)};
-        b = Box{smin(b.lx, v2.x), smin(b.ly, v2.y), smin(b.lz, v2.z), smax(b.hx, v2.x), smax(b.hy, v2.y),
-                smax(b.hz, v2.z)};
+        b = tri_box(v0, v1, v2);
         nan = box_has_nan(b);
         store_node(&leaves[i], make_node(b, 1u, indices ? indices[i] : i));
     }
@@ -176,7 +179,6 @@ __global__ void __launch_bounds__(T256) k_leaf_init_aabbs(const float4* __restri
     reduce_scene_bounds(valid, b, nan, misc, partials);
 }
 
-// ploc/mod.rs:287-288 and 782-785; morton.rs:55-58.
 // rebuild_from_leaves takes the root's stored box as the scene box (ploc/rebuild.rs:154).
 __global__ void k_bounds_from_node(Misc* misc, const Node32* __restrict__ nodes) {
     if (threadIdx.x == 0) {
@@ -204,28 +206,63 @@ __device__ __forceinline__ bool child_slot(uint32_t v, const uint32_t* __restric
     return true;
 }
 
+// The scene's normalisation to the unit cube (ploc/mod.rs:287-288 and 782-785) from the bounds' order keys.
+struct SceneMap {
+    double sx, sy, sz, ox, oy, oz;
+    __device__ __forceinline__ void point(const Box& b, double& px, double& py, double& pz) const {
+        const float cx = (b.hx + b.lx) * 0.5f, cy = (b.hy + b.ly) * 0.5f, cz = (b.hz + b.lz) * 0.5f;
+        px = (double)cx * sx + ox;
+        py = (double)cy * sy + oy;
+        pz = (double)cz * sz + oz;
+    }
+};
+__device__ __forceinline__ SceneMap scene_map(const uint32_t* bounds) {
+    const float mnx = f32_from_order_key(bounds[0]), mny = f32_from_order_key(bounds[1]),
+                mnz = f32_from_order_key(bounds[2]);
+    const float mxx = f32_from_order_key(bounds[3]), mxy = f32_from_order_key(bounds[4]),
+                mxz = f32_from_order_key(bounds[5]);
+    SceneMap m;
+    m.sx = 1.0 / (double)(mxx - mnx);
+    m.sy = 1.0 / (double)(mxy - mny);
+    m.sz = 1.0 / (double)(mxz - mnz);
+    m.ox = -(double)mnx * m.sx;
+    m.oy = -(double)mny * m.sy;
+    m.oz = -(double)mnz * m.sz;
+    return m;
+}
+
+// The 63-bit Morton code of a unit-cube point (morton.rs:35-58).
+__device__ __forceinline__ uint64_t morton64_of_point(double px, double py, double pz) {
+    const double s = 2097152.0;  // 2^21
+    return split_by_3_u64(f64_as_u32(px * s)) | split_by_3_u64(f64_as_u32(py * s)) << 1 |
+           split_by_3_u64(f64_as_u32(pz * s)) << 2;
+}
+
+// The top 32 bits of a 63-bit code, or of a 126-bit code's 62-bit high word.
+__device__ __forceinline__ uint32_t top_of_u64(uint64_t code) { return (uint32_t)(code >> 31); }
+__device__ __forceinline__ uint32_t top_of_u128(uint64_t hi) { return (uint32_t)(hi >> 30); }
+
 // keys_hi = NULL: U64 codes into keys.  Otherwise U128 codes, low words into keys and high words into keys_hi.
+// tops: the codes' top 32 bits (the first sort key).
 __global__ void __launch_bounds__(T256) k_morton(const Node32* __restrict__ leaves, uint32_t n,
                                                  const Misc* __restrict__ misc, uint64_t* __restrict__ keys,
-                                                 uint64_t* __restrict__ keys_hi) {
+                                                 uint64_t* __restrict__ keys_hi, uint32_t* __restrict__ tops) {
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     if (i >= n) return;
-    const float mnx = f32_from_order_key(misc->bounds[0]), mny = f32_from_order_key(misc->bounds[1]),
-                mnz = f32_from_order_key(misc->bounds[2]);
-    const float mxx = f32_from_order_key(misc->bounds[3]), mxy = f32_from_order_key(misc->bounds[4]),
-                mxz = f32_from_order_key(misc->bounds[5]);
-    const double sx = 1.0 / (double)(mxx - mnx), sy = 1.0 / (double)(mxy - mny), sz = 1.0 / (double)(mxz - mnz);
-    const double ox = -(double)mnx * sx, oy = -(double)mny * sy, oz = -(double)mnz * sz;
-    Node32 l = load_node(&leaves[i]);
-    const float cx = (l.maxx + l.minx) * 0.5f, cy = (l.maxy + l.miny) * 0.5f, cz = (l.maxz + l.minz) * 0.5f;
-    const double px = (double)cx * sx + ox, py = (double)cy * sy + oy, pz = (double)cz * sz + oz;
+    const SceneMap map = scene_map(misc->bounds);
+    double px, py, pz;
+    map.point(node_box(load_node(&leaves[i])), px, py, pz);
     if (keys_hi) {
-        morton128_of_point(px, py, pz, keys[i], keys_hi[i]);
+        uint64_t lo, hi;
+        morton128_of_point(px, py, pz, lo, hi);
+        keys[i] = lo;
+        keys_hi[i] = hi;
+        tops[i] = top_of_u128(hi);
         return;
     }
-    const double s = 2097152.0;
-    keys[i] = split_by_3_u64(f64_as_u32(px * s)) | split_by_3_u64(f64_as_u32(py * s)) << 1 |
-              split_by_3_u64(f64_as_u32(pz * s)) << 2;
+    const uint64_t code = morton64_of_point(px, py, pz);
+    keys[i] = code;
+    tops[i] = top_of_u64(code);
 }
 
 __global__ void __launch_bounds__(T256) k_gather_u64(const uint64_t* __restrict__ src,
@@ -242,6 +279,267 @@ __global__ void __launch_bounds__(T256) k_gather(const Node32* __restrict__ leav
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     if (i >= n) return;
     store_node(&out[i], load_node(&leaves[order[i]]));
+}
+
+// The sorted leaves in cluster order from the sort by the codes' top 32 bits (tops and order, stable): a run of equal
+// tops is put in the order of the codes' remaining bits, ties by position (the leaf order, the sort being stable), by
+// ranking each of its members against the others from LDS, so that the result is the order of a stable sort of the
+// whole codes.  Runs are short (the tops are cells of 10 or 11 bits per axis: 1 to 12 leaves a run on the benchmark's
+// heightfields of 1.3M and 17.3M triangles).  A run longer than RUN_MAX (or that long on one side of a member) sets
+// DERR_RESORT and leaves one cluster in the pass state, which turns the passes behind this launch into no-ops; the
+// host then sorts the whole codes.
+// Bound by the random 32-byte leaf reads.  1,288,352 leaves: 23 us against the plain gather's 16, and with it the sort
+// takes 4 passes of 20 bytes per key instead of 8 of 32 (198 -> 98 us).
+// order_out (may be NULL): the final permutation.
+constexpr uint32_t RUN_MAX = 64;
+
+template <bool WIDE>
+__global__ void __launch_bounds__(T256) k_gather_runs(const Node32* __restrict__ leaves,
+                                                      const uint32_t* __restrict__ tops,
+                                                      const uint32_t* __restrict__ order, uint32_t n,
+                                                      const uint64_t* __restrict__ keys,
+                                                      const uint64_t* __restrict__ keys_hi, Misc* misc,
+                                                      Node32* __restrict__ out, uint32_t* __restrict__ order_out) {
+    constexpr uint32_t WIN = T256 + 2 * RUN_MAX;
+    __shared__ uint32_t tk[WIN];
+    __shared__ uint32_t rest[WIN];                  // the bits below the top: 31, or 30 of the high word
+    __shared__ uint64_t low[WIDE ? WIN : 1];        // the low word of a 126-bit code
+    const uint32_t base = blockIdx.x * T256;
+    // window slot w holds sorted position base - RUN_MAX + w
+    const uint32_t w0 = base < RUN_MAX ? RUN_MAX - base : 0u;             // first slot inside the array
+    const uint32_t w1 = min(WIN, n - base + RUN_MAX);                     // end of the slots inside it
+    for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) tk[w] = tops[base + w - RUN_MAX];
+    __syncthreads();
+    for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) {
+        const uint32_t t = tk[w];
+        if ((w > w0 && tk[w - 1] == t) || (w + 1 < w1 && tk[w + 1] == t)) {
+            const uint32_t leaf = order[base + w - RUN_MAX];
+            if (WIDE) {
+                rest[w] = (uint32_t)keys_hi[leaf] & 0x3fffffffu;
+                low[w] = keys[leaf];
+            } else {
+                rest[w] = (uint32_t)keys[leaf] & 0x7fffffffu;
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t i = base + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t leaf = order[i], me = threadIdx.x + RUN_MAX, t = tk[me];
+    uint32_t a = me, b = me;  // the run's first and last slot
+    while (a > w0 && me - a < RUN_MAX && tk[a - 1] == t) --a;
+    while (b + 1 < w1 && b - me < RUN_MAX && tk[b + 1] == t) ++b;
+    if (me - a == RUN_MAX || b - me == RUN_MAX) {
+        atomicOr(&misc->err, DERR_RESORT);
+        misc->state[0].count = 1u;
+        return;
+    }
+    uint32_t rank = 0u;
+    if (a != b) {
+        const uint32_t r = rest[me];
+        const uint64_t l = WIDE ? low[me] : 0ull;
+        for (uint32_t j = a; j <= b; ++j) {
+            const bool same = rest[j] == r;
+            const bool less = rest[j] < r || (same && WIDE && low[j] < l);
+            const bool tie = same && (!WIDE || low[j] == l) && j < me;
+            rank += (less || tie) ? 1u : 0u;
+        }
+    }
+    const uint32_t pos = base + a - RUN_MAX + rank;
+    store_node(&out[pos], load_node(&leaves[leaf]));
+    if (order_out) order_out[pos] = leaf;
+}
+
+// State reset before a build repeats its passes (after DERR_RESORT); the bounds and the codes stay.
+__global__ void k_reset_state(Misc* misc, uint32_t n) {
+    if (threadIdx.x == 0) {
+        misc->err &= ~DERR_RESORT;
+        misc->state[0] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
+        misc->state[1] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
+    }
+}
+
+// The front of a build of at most SMALL_MAX leaves in one workgroup and one launch: leaf boxes, scene bounds, Morton
+// codes, the stable sort (four 8-bit LSD passes over the codes' top 32 bits in LDS, wave multisplit ranking as in
+// sort.hip, then runs of equal tops ranked by the remaining bits) and the sorted leaves as the first clusters.  At
+// these sizes the 29 launches it replaces are 2 to 7 us each whatever they hold (1,501 triangles: 109 us of kernels in
+// 29 launches -> 20 us in one).
+constexpr uint32_t SMALL_MAX = 2048;
+constexpr int SMALL_THREADS = 1024;
+constexpr int SMALL_ITEMS = (int)SMALL_MAX / SMALL_THREADS;
+constexpr int SMALL_WAVES = SMALL_THREADS / 64;
+
+template <bool WIDE>
+__global__ void __launch_bounds__(SMALL_THREADS)
+    k_front_small(const float4* __restrict__ tris, const float4* __restrict__ aabbs,
+                  const uint32_t* __restrict__ indices, uint32_t n, Misc* misc, uint32_t* __restrict__ hist,
+                  uint32_t* __restrict__ iota_out, uint64_t* __restrict__ codes_out,
+                  uint64_t* __restrict__ codes_hi_out, uint32_t* __restrict__ order_out,
+                  Node32* __restrict__ clusters) {
+    __shared__ uint64_t low[SMALL_MAX];                // codes (the low words of 126-bit codes), leaf order
+    __shared__ uint64_t high[WIDE ? SMALL_MAX : 1];
+    __shared__ uint32_t tk[SMALL_MAX];                 // tops in sorted order
+    __shared__ uint16_t tv[SMALL_MAX];                 // leaves in sorted order
+    __shared__ uint32_t whist[SMALL_WAVES][256];
+    __shared__ uint32_t red[6][SMALL_WAVES];
+    __shared__ uint32_t wtot[4];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+
+    // leaf boxes (as k_leaf_init_*) and scene bounds
+    auto leaf_box = [&](uint32_t i) {
+        if (tris) {
+            const float4 v0 = tris[3 * (size_t)i], v1 = tris[3 * (size_t)i + 1], v2 = tris[3 * (size_t)i + 2];
+            return tri_box(v0, v1, v2);
+        }
+        const float4 lo = aabbs[2 * (size_t)i], hi = aabbs[2 * (size_t)i + 1];
+        return Box{lo.x, lo.y, lo.z, hi.x, hi.y, hi.z};
+    };
+    Box box[SMALL_ITEMS];
+    uint32_t k[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
+    bool nan = false;
+#pragma unroll
+    for (int q = 0; q < SMALL_ITEMS; ++q) {
+        const uint32_t i = (uint32_t)q * SMALL_THREADS + tid;
+        box[q] = Box{0, 0, 0, 0, 0, 0};
+        if (i < n) {
+            box[q] = leaf_box(i);
+            nan |= box_has_nan(box[q]);
+            if (iota_out) iota_out[i] = i;
+            const uint32_t kl[3] = {f32_order_key(box[q].lx), f32_order_key(box[q].ly), f32_order_key(box[q].lz)};
+            const uint32_t kh[3] = {f32_order_key(box[q].hx), f32_order_key(box[q].hy), f32_order_key(box[q].hz)};
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                k[a] = min(k[a], min(kl[a], kh[a]));
+                k[3 + a] = max(k[3 + a], max(kl[a], kh[a]));
+            }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        k[a] = wave_min_u32(k[a]);
+        k[3 + a] = wave_max_u32(k[3 + a]);
+        if (lane == 0) {
+            red[a][wave] = k[a];
+            red[3 + a][wave] = k[3 + a];
+        }
+    }
+    const bool any_nan = __syncthreads_or(nan);
+    if (tid == 0) {
+        hist[0] = 2u * n - 1u;
+        misc->err = any_nan ? DERR_NAN_INPUT : 0u;
+        misc->state[0] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
+        misc->state[1] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
+    }
+#pragma unroll
+    for (int w = 0; w < SMALL_WAVES; ++w)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            k[a] = min(k[a], red[a][w]);
+            k[3 + a] = max(k[3 + a], red[3 + a][w]);
+        }
+    const SceneMap map = scene_map(k);
+#pragma unroll
+    for (int q = 0; q < SMALL_ITEMS; ++q) {
+        const uint32_t i = (uint32_t)q * SMALL_THREADS + tid;
+        if (i >= n) continue;
+        double px, py, pz;
+        map.point(box[q], px, py, pz);
+        if (WIDE) {
+            uint64_t lo, hi;
+            morton128_of_point(px, py, pz, lo, hi);
+            low[i] = lo;
+            high[i] = hi;
+            tk[i] = top_of_u128(hi);
+            if (codes_hi_out) codes_hi_out[i] = hi;
+            if (codes_out) codes_out[i] = lo;
+        } else {
+            const uint64_t code = morton64_of_point(px, py, pz);
+            low[i] = code;
+            tk[i] = top_of_u64(code);
+            if (codes_out) codes_out[i] = code;
+        }
+        tv[i] = (uint16_t)i;
+    }
+    __syncthreads();
+
+    // four LSD passes; wave w owns positions [w * 64 * ITEMS, (w + 1) * 64 * ITEMS)
+    const uint64_t lt = lanemask_lt();
+    for (uint32_t shift = 0; shift < 32u; shift += 8u) {
+        uint32_t key[SMALL_ITEMS], rank[SMALL_ITEMS];
+        uint16_t val[SMALL_ITEMS];
+        for (uint32_t d = lane; d < 256u; d += 64u) whist[wave][d] = 0u;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < SMALL_ITEMS; ++j) {
+            const uint32_t p = wave * (64u * SMALL_ITEMS) + (uint32_t)j * 64u + lane;
+            const bool valid = p < n;
+            key[j] = valid ? tk[p] : 0u;
+            val[j] = valid ? tv[p] : (uint16_t)0;
+            const uint32_t d = (key[j] >> shift) & 0xffu;
+            uint64_t peers = ballot64(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bm = ballot64(bit);
+                peers &= bit ? bm : ~bm;
+            }
+            const uint32_t below = (uint32_t)__popcll(peers & lt);
+            uint32_t at = 0u;
+            if (valid) at = whist[wave][d];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0u) whist[wave][d] = at + (uint32_t)__popcll(peers);
+            __builtin_amdgcn_wave_barrier();
+            rank[j] = at + below;
+        }
+        __syncthreads();
+        uint32_t run = 0u, incl = 0u;
+        if (tid < 256u) {  // thread d: prefix of digit d across the waves, then across the digits
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; ++w) {
+                const uint32_t c = whist[w][tid];
+                whist[w][tid] = run;
+                run += c;
+            }
+            incl = wave_inclusive_scan(run);
+            if (lane == 63u) wtot[wave] = incl;
+        }
+        __syncthreads();
+        if (tid < 256u) {
+            uint32_t before = incl - run;
+            for (uint32_t w = 0; w < wave; ++w) before += wtot[w];
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; ++w) whist[w][tid] += before;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SMALL_ITEMS; ++j) {
+            const uint32_t p = wave * (64u * SMALL_ITEMS) + (uint32_t)j * 64u + lane;
+            if (p < n) {
+                const uint32_t to = whist[wave][(key[j] >> shift) & 0xffu] + rank[j];
+                tk[to] = key[j];
+                tv[to] = val[j];
+            }
+        }
+        __syncthreads();
+    }
+
+    // runs of equal tops by the remaining bits, ties by position
+#pragma unroll
+    for (int q = 0; q < SMALL_ITEMS; ++q) {
+        const uint32_t p = (uint32_t)q * SMALL_THREADS + tid;
+        if (p >= n) continue;
+        const uint32_t t = tk[p], leaf = tv[p];
+        uint32_t a = p, rank = 0u;
+        while (a > 0u && tk[a - 1] == t) --a;
+        const uint64_t l = low[leaf], h = WIDE ? high[leaf] : 0ull;
+        for (uint32_t j = a; j < n && tk[j] == t; ++j) {
+            const uint64_t jl = low[tv[j]], jh = WIDE ? high[tv[j]] : 0ull;
+            const bool less = jh < h || (jh == h && (jl < l || (jl == l && j < p)));
+            rank += less ? 1u : 0u;
+        }
+        store_node(&clusters[a + rank], make_node(leaf_box(leaf), 1u, indices ? indices[leaf] : leaf));
+        if (order_out) order_out[a + rank] = leaf;
+    }
 }
 
 // Classification of cluster i (ploc/mod.rs:423-439): `emit` when it goes to the next pass (kept, or the higher
@@ -983,9 +1281,45 @@ static obvhs_status sort_codes(obvhs_context* ctx, uint64_t* keys, const uint64_
     return OBVHS_OK;
 }
 
+// Clusters in Morton order (ploc/mod.rs:811-846) from the codes: the top 32 bits sorted, the runs of equal tops
+// ordered by the gather.  keys and keys_hi keep their leaf order.  order_out (may be NULL): the permutation.
+static obvhs_status sort_gather(obvhs_context* ctx, const Node32* leaves, const uint64_t* keys,
+                                const uint64_t* keys_hi, uint32_t n, Node32* cur, uint32_t* order_out) {
+    hipStream_t st = ctx->stream;
+    BuildScratch& S = ctx->scratch;
+    uint32_t* tops = S.tops.as<uint32_t>();
+    uint32_t* vals = S.vals.as<uint32_t>();
+    Misc* misc = S.misc.as<Misc>();
+    OBVHS_TRY(radix_sort_pairs32(tops, vals, true, n, 32, S.sort_scratch.ptr, st, sort_items_for(ctx, n)),
+              "radix sort (top words)");
+    const uint32_t nblk = (n + T256 - 1) / T256;
+    if (keys_hi)
+        k_gather_runs<true><<<nblk, T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+    else
+        k_gather_runs<false><<<nblk, T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+    OBVHS_TRY(hipGetLastError(), "gather launch");
+    return OBVHS_OK;
+}
+
+// The same by a sort of the whole codes, after sort_gather met a long run (DERR_RESORT): the pass state starts over.
+static obvhs_status resort_gather(obvhs_context* ctx, const Node32* leaves, uint64_t* keys, const uint64_t* keys_hi,
+                                  uint32_t n, Node32* cur, uint32_t* order_out) {
+    hipStream_t st = ctx->stream;
+    BuildScratch& S = ctx->scratch;
+    uint32_t* vals = S.vals.as<uint32_t>();
+    k_reset_state<<<1, 64, 0, st>>>(S.misc.as<Misc>(), n);
+    const obvhs_status ss = sort_codes(ctx, keys, keys_hi, vals, n);
+    if (ss != OBVHS_OK) return ss;
+    if (order_out)
+        OBVHS_TRY(hipMemcpyAsync(order_out, vals, (size_t)n * 4, hipMemcpyDeviceToDevice, st), "copy sorted index");
+    k_gather<<<(n + T256 - 1) / T256, T256, 0, st>>>(leaves, vals, n, cur);
+    OBVHS_TRY(hipGetLastError(), "gather launch");
+    return OBVHS_OK;
+}
+
 // The PLOC passes from the sorted clusters in `cur` to the root (ploc/mod.rs:327-499): grid passes while more than
 // TAIL_MAX clusters remain, then the one-workgroup tail.  `fin`
-// receives the final pass state.
+// receives the final pass state; `resort` is set (and the passes did nothing) when the gather flagged DERR_RESORT.
 // The error word and the pass state of `slot` with one copy (err, pad, state[0], state[1] are adjacent) into the
 // pinned staging area, then a stream synchronisation.
 static hipError_t read_state(const Misc* misc, uint32_t slot, void* pinned, hipStream_t st, PlocState& state,
@@ -1036,7 +1370,8 @@ static void launch_tail(hipStream_t st, const Node32* cur, Misc* misc, uint32_t 
 static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uint32_t n, uint32_t r,
                                uint32_t search_depth_threshold, Node32* bvh_nodes, uint32_t* hist, DpView dp,
                                uint32_t fused, const uint32_t* slot_map, uint32_t vtop, uint32_t map_len,
-                               PlocState& fin) {
+                               PlocState& fin, bool& resort) {
+    resort = false;
     hipStream_t st = ctx->stream;
     BuildScratch& S = ctx->scratch;
     Misc* misc = S.misc.as<Misc>();
@@ -1075,7 +1410,11 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
         OBVHS_TRY(hipGetLastError(), "ploc pass launch");
         uint32_t herr_loop = 0u;
         OBVHS_TRY(read_state(misc, slot, ctx->pinned, st, hstate, herr_loop), "read ploc state");
-        if (herr_loop) return device_error_to_status(herr_loop);
+        if (herr_loop & ~DERR_RESORT) return device_error_to_status(herr_loop);
+        if (herr_loop) {
+            resort = true;
+            return OBVHS_OK;
+        }
         // Every pass merges at least one pair unless costs are NaN; a batch without progress would never end.
         if (hstate.count >= known) return OBVHS_ERR_PLOC_SELF_MERGE;
         known = hstate.count;
@@ -1087,7 +1426,11 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
     OBVHS_TRY(hipGetLastError(), "ploc tail launch");
     uint32_t herr = 0u;
     OBVHS_TRY(read_state(misc, slot, ctx->pinned, st, hstate, herr), "read final ploc state");
-    if (herr) return device_error_to_status(herr);
+    if (herr & ~DERR_RESORT) return device_error_to_status(herr);
+    if (herr) {
+        resort = true;
+        return OBVHS_OK;
+    }
     if (hstate.insert != 1u) return OBVHS_ERR_PLOC_SELF_MERGE;  // ploc/mod.rs:495-497
     fin = hstate;
     return OBVHS_OK;
@@ -1124,6 +1467,7 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
     OBVHS_TRY(S.keys.ensure((size_t)n * 8), "alloc keys");
     if (u128) OBVHS_TRY(S.keys_hi.ensure((size_t)n * 8), "alloc high key words");
     OBVHS_TRY(S.vals.ensure((size_t)n * 4), "alloc vals");
+    OBVHS_TRY(S.tops.ensure((size_t)n * 4), "alloc top key words");
     OBVHS_TRY(S.merge.ensure((size_t)n + 64), "alloc merge");
     const uint32_t nblk = (n + T256 - 1) / T256;
     OBVHS_TRY(S.blocksums.ensure((size_t)nblk * sizeof(uint2) + 64 + (size_t)nblk * 6 * 4), "alloc blocksums");
@@ -1134,7 +1478,6 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
     Node32* bvh_nodes = bvh->nodes.as<Node32>();
     uint64_t* keys = S.keys.as<uint64_t>();
     uint64_t* keys_hi = u128 ? S.keys_hi.as<uint64_t>() : nullptr;
-    uint32_t* vals = S.vals.as<uint32_t>();
     uint32_t* hist = bvh->hist.as<uint32_t>();
     // per-block bound partials share the blocksums allocation (they are dead before the first pass)
     uint32_t* partials = reinterpret_cast<uint32_t*>(S.blocksums.as<char>() + (size_t)nblk * sizeof(uint2) + 64);
@@ -1144,42 +1487,55 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
         OBVHS_TRY(hipMemcpyAsync(bvh->prim_indices.ptr, d_indices, (size_t)n * 4, hipMemcpyDeviceToDevice, st),
                   "copy indices");
     }
-    k_init_misc<<<1, 64, 0, st>>>(misc, n, hist);
     uint32_t* iota_out = d_indices ? nullptr : bvh->prim_indices.as<uint32_t>();  // primitive_indices = 0..n-1
-    if (d_tris) {
-        k_leaf_init_tris<<<nblk, T256, 0, st>>>(reinterpret_cast<const float4*>(d_tris), d_indices, n, leaves,
-                                                misc, partials, iota_out);
-    } else {
-        k_leaf_init_aabbs<<<nblk, T256, 0, st>>>(reinterpret_cast<const float4*>(d_aabbs), d_indices, n, leaves,
-                                                 misc, partials, iota_out);
-    }
-    k_reduce_bounds<<<1, 1024, 0, st>>>(partials, nblk, misc);
-    k_morton<<<nblk, T256, 0, st>>>(leaves, n, misc, keys, keys_hi);
-    OBVHS_TRY(hipGetLastError(), "leaf/morton launch");
     bvh->code_words = u128 ? 2u : 1u;
+    uint64_t *codes = nullptr, *codes_hi = nullptr;  // kept with the sort permutation for parity tests
+    uint32_t* order_out = nullptr;
     if (ctx->keep_trace) {  // low words, then the high words of U128 codes
         OBVHS_TRY(bvh->codes.ensure((size_t)n * 8 * bvh->code_words), "alloc codes");
-        OBVHS_TRY(hipMemcpyAsync(bvh->codes.ptr, keys, (size_t)n * 8, hipMemcpyDeviceToDevice, st), "copy codes");
-        if (u128)
-            OBVHS_TRY(hipMemcpyAsync(bvh->codes.as<uint64_t>() + n, keys_hi, (size_t)n * 8, hipMemcpyDeviceToDevice,
-                                     st),
-                      "copy codes");
-    }
-    obvhs_status ss = sort_codes(ctx, keys, keys_hi, vals, n);
-    if (ss != OBVHS_OK) return ss;
-    if (ctx->keep_trace) {
         OBVHS_TRY(bvh->sorted_index.ensure((size_t)n * 4), "alloc sorted index");
-        OBVHS_TRY(hipMemcpyAsync(bvh->sorted_index.ptr, vals, (size_t)n * 4, hipMemcpyDeviceToDevice, st),
-                  "copy sorted index");
+        codes = bvh->codes.as<uint64_t>();
+        codes_hi = u128 ? codes + n : nullptr;
+        order_out = bvh->sorted_index.as<uint32_t>();
     }
+    const float4* tris = reinterpret_cast<const float4*>(d_tris);
+    const float4* aabbs = d_tris ? nullptr : reinterpret_cast<const float4*>(d_aabbs);
     Node32* cur = S.clusters_a.as<Node32>();
     Node32* nxt = S.clusters_b.as<Node32>();
-    k_gather<<<nblk, T256, 0, st>>>(leaves, vals, n, cur);
-    OBVHS_TRY(hipGetLastError(), "gather launch");
+    if (n <= SMALL_MAX) {
+        if (u128)
+            k_front_small<true><<<1, SMALL_THREADS, 0, st>>>(tris, aabbs, d_indices, n, misc, hist, iota_out, codes,
+                                                             codes_hi, order_out, cur);
+        else
+            k_front_small<false><<<1, SMALL_THREADS, 0, st>>>(tris, aabbs, d_indices, n, misc, hist, iota_out, codes,
+                                                              codes_hi, order_out, cur);
+        OBVHS_TRY(hipGetLastError(), "small build front launch");
+    } else {
+        k_init_misc<<<1, 64, 0, st>>>(misc, n, hist);
+        if (d_tris)
+            k_leaf_init_tris<<<nblk, T256, 0, st>>>(tris, d_indices, n, leaves, misc, partials, iota_out);
+        else
+            k_leaf_init_aabbs<<<nblk, T256, 0, st>>>(aabbs, d_indices, n, leaves, misc, partials, iota_out);
+        k_reduce_bounds<<<1, 1024, 0, st>>>(partials, nblk, misc);
+        k_morton<<<nblk, T256, 0, st>>>(leaves, n, misc, keys, keys_hi, S.tops.as<uint32_t>());
+        OBVHS_TRY(hipGetLastError(), "leaf/morton launch");
+        if (codes) OBVHS_TRY(hipMemcpyAsync(codes, keys, (size_t)n * 8, hipMemcpyDeviceToDevice, st), "copy codes");
+        if (codes_hi)
+            OBVHS_TRY(hipMemcpyAsync(codes_hi, keys_hi, (size_t)n * 8, hipMemcpyDeviceToDevice, st), "copy codes");
+        const obvhs_status ss = sort_gather(ctx, leaves, keys, keys_hi, n, cur, order_out);
+        if (ss != OBVHS_OK) return ss;
+    }
 
     PlocState fin{};
+    bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, n, search_distance, search_depth_threshold, bvh_nodes, hist, dp,
-                                 fused, nullptr, 0u, 0u, fin);
+                                 fused, nullptr, 0u, 0u, fin, resort);
+    if (ps == OBVHS_OK && resort) {
+        ps = resort_gather(ctx, leaves, keys, keys_hi, n, cur, order_out);
+        if (ps == OBVHS_OK)
+            ps = run_passes(ctx, cur, nxt, n, search_distance, search_depth_threshold, bvh_nodes, hist, dp, fused,
+                            nullptr, 0u, 0u, fin, resort);
+    }
     if (ps != OBVHS_OK) return ps;
     bvh->ploc_iterations = fin.depth;
     bvh->cluster_sum = fin.cluster_sum;
@@ -1209,6 +1565,7 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     OBVHS_TRY(S.keys.ensure((size_t)k * 8), "alloc keys");
     if (u128) OBVHS_TRY(S.keys_hi.ensure((size_t)k * 8), "alloc high key words");
     OBVHS_TRY(S.vals.ensure((size_t)k * 4), "alloc vals");
+    OBVHS_TRY(S.tops.ensure((size_t)k * 4), "alloc top key words");
     OBVHS_TRY(S.merge.ensure((size_t)k + 64), "alloc merge");
     const uint32_t nblk = (k + T256 - 1) / T256;
     OBVHS_TRY(S.blocksums.ensure((size_t)nblk * sizeof(uint2) + 64 + (size_t)nblk * 6 * 4), "alloc blocksums");
@@ -1219,23 +1576,27 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     Node32* bvh_nodes = bvh->nodes.as<Node32>();
     uint64_t* keys = S.keys.as<uint64_t>();
     uint64_t* keys_hi = u128 ? S.keys_hi.as<uint64_t>() : nullptr;
-    uint32_t* vals = S.vals.as<uint32_t>();
     uint32_t* hist = bvh->hist.as<uint32_t>();
     // The clusters are copied out first: merges may overwrite the freed slots they came from.
     k_gather<<<nblk, T256, 0, st>>>(bvh_nodes, d_src_slots, k, leaves);
     k_init_misc<<<1, 64, 0, st>>>(misc, k, hist);
     k_bounds_from_node<<<1, 64, 0, st>>>(misc, bvh_nodes);
-    k_morton<<<nblk, T256, 0, st>>>(leaves, k, misc, keys, keys_hi);
+    k_morton<<<nblk, T256, 0, st>>>(leaves, k, misc, keys, keys_hi, S.tops.as<uint32_t>());
     OBVHS_TRY(hipGetLastError(), "rebuild morton launch");
-    obvhs_status ss = sort_codes(ctx, keys, keys_hi, vals, k);
-    if (ss != OBVHS_OK) return ss;
     Node32* cur = S.clusters_a.as<Node32>();
     Node32* nxt = S.clusters_b.as<Node32>();
-    k_gather<<<nblk, T256, 0, st>>>(leaves, vals, k, cur);
-    OBVHS_TRY(hipGetLastError(), "gather launch");
+    const obvhs_status ss = sort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
+    if (ss != OBVHS_OK) return ss;
     PlocState fin{};
+    bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist,
-                                 DpView{}, 0u, d_slot_map, 2u * k - 3u, k - 1u, fin);
+                                 DpView{}, 0u, d_slot_map, 2u * k - 3u, k - 1u, fin, resort);
+    if (ps == OBVHS_OK && resort) {
+        ps = resort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
+        if (ps == OBVHS_OK)
+            ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist, DpView{}, 0u,
+                            d_slot_map, 2u * k - 3u, k - 1u, fin, resort);
+    }
     if (ps != OBVHS_OK) return ps;
     if (!d_slot_map) bvh->node_count = 2u * k - 1u;  // ploc/mod.rs:283-284 (nodes.resize)
     bvh->pass_ordered = d_slot_map == nullptr;    // ploc/mod.rs:502

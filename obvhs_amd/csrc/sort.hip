@@ -1,4 +1,4 @@
-// Stable LSD radix sort of (u64 Morton code, u32 leaf index) pairs for gfx950.
+// Stable LSD radix sort of (u64 or u32 key, u32 value) pairs for gfx950.
 //
 // Replaces the Morton sort of ploc/mod.rs:811-827.  The reference uses unstable sorts whose tie order is not
 // reproducible; this sort is stable, so ties between equal codes keep ascending leaf index (the project rule the
@@ -14,6 +14,9 @@
 //               LDS (half the LDS of staging both at once, so twice the tiles per CU).
 // Tiles are 256 threads x ITEMS keys (ITEMS = 4, 8 or 16, the sort tile the context's tuning table picks per size
 // class; 8 by default); each wave owns a contiguous 64 x ITEMS key segment.  Every tile size gives the same order.
+//
+// u32 keys: a build sorts only the top 32 bits of its Morton codes and orders the short runs of equal tops where the
+// leaves are gathered (ploc.hip), so a key takes 4 passes of 20 bytes instead of 8 passes of 32.
 #include "common.hpp"
 #include "device_util.hpp"
 #include "internal.hpp"
@@ -26,9 +29,9 @@ constexpr int SORT_THREADS = 256;
 constexpr int SORT_MIN_ITEMS = 4;  // the scratch is sized for the smallest tile (the most tiles)
 constexpr int SORT_WAVES = SORT_THREADS / 64;
 
-template <int ITEMS>
+template <class K, int ITEMS>
 __global__ void __launch_bounds__(SORT_THREADS)
-    k_radix_upsweep(const uint64_t* __restrict__ keys, uint32_t n, uint32_t shift, uint32_t num_tiles,
+    k_radix_upsweep(const K* __restrict__ keys, uint32_t n, uint32_t shift, uint32_t num_tiles,
                     uint32_t* __restrict__ counts) {
     constexpr int SORT_TILE = SORT_THREADS * ITEMS;
     __shared__ uint32_t hist[256];
@@ -97,10 +100,10 @@ __global__ void __launch_bounds__(SORT_THREADS)
     if (tid == 0) totals[d] = carry;
 }
 
-template <int ITEMS>
+template <class K, int ITEMS>
 __global__ void __launch_bounds__(SORT_THREADS)
-    k_radix_downsweep(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                      uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n, uint32_t shift,
+    k_radix_downsweep(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
+                      K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n, uint32_t shift,
                       const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ totals,
                       uint32_t num_tiles) {
     constexpr int SORT_TILE = SORT_THREADS * ITEMS;
@@ -108,7 +111,7 @@ __global__ void __launch_bounds__(SORT_THREADS)
     __shared__ uint32_t digit_start[256];
     __shared__ uint32_t gbase[256];
     __shared__ uint32_t scan_tmp[8];
-    __shared__ uint64_t stage[SORT_TILE];  // the tile's keys, then its values
+    __shared__ K stage[SORT_TILE];  // the tile's keys, then its values
 
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = tid >> 6;
@@ -123,7 +126,7 @@ __global__ void __launch_bounds__(SORT_THREADS)
     __syncthreads();
 
     const uint32_t seg = tile_base + wave * (64 * ITEMS);
-    uint64_t k[ITEMS];
+    K k[ITEMS];
     uint32_t v[ITEMS];
     uint32_t rank[ITEMS];
     const uint64_t lt = lanemask_lt();
@@ -131,7 +134,7 @@ __global__ void __launch_bounds__(SORT_THREADS)
     for (int j = 0; j < ITEMS; ++j) {
         uint32_t idx = seg + j * 64 + lane;
         bool valid = idx < n;
-        k[j] = valid ? kin[idx] : 0ull;
+        k[j] = valid ? kin[idx] : (K)0;
         v[j] = valid ? (vin ? vin[idx] : idx) : 0u;
         uint32_t d = (uint32_t)(k[j] >> shift) & 0xffu;
         uint64_t peers = ballot64(valid);
@@ -176,7 +179,7 @@ __global__ void __launch_bounds__(SORT_THREADS)
     for (int j = 0; j < ITEMS; ++j) {
         const uint32_t s = tid + (uint32_t)j * SORT_THREADS;
         if (s < tile_count) {
-            const uint64_t key = stage[s];
+            const K key = stage[s];
             const uint32_t d = (uint32_t)(key >> shift) & 0xffu;
             dst[j] = gbase[d] + (s - digit_start[d]);
             kout[dst[j]] = key;
@@ -211,8 +214,8 @@ size_t radix_sort_scratch_bytes(uint32_t n) {
 // Sorts keys[0..n) ascending (stable) with values.  On entry values may be null (identity 0..n).  `bits` is the
 // number of low key bits that can be non-zero (63 for Morton64).  Result lands in keys/values (even pass count)
 // or is copied back.  scratch must hold radix_sort_scratch_bytes(n).  items: keys per thread of a tile (4, 8, 16).
-template <int ITEMS>
-static hipError_t radix_sort_impl(uint64_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
+template <class K, int ITEMS>
+static hipError_t radix_sort_impl(K* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                                   void* scratch, hipStream_t stream) {
     constexpr int SORT_TILE = SORT_THREADS * ITEMS;
     uint32_t tiles = (n + SORT_TILE - 1) / SORT_TILE;
@@ -222,43 +225,54 @@ static hipError_t radix_sort_impl(uint64_t* keys, uint32_t* values, bool values_
         p += (bytes + 255) & ~size_t(255);
         return r;
     };
-    uint64_t* kalt = reinterpret_cast<uint64_t*>(take((size_t)n * 8));
+    K* kalt = reinterpret_cast<K*>(take((size_t)n * sizeof(K)));
     uint32_t* valt = reinterpret_cast<uint32_t*>(take((size_t)n * 4));
     uint32_t* counts = reinterpret_cast<uint32_t*>(take((size_t)256 * tiles * 4));
     uint32_t* totals = reinterpret_cast<uint32_t*>(take(256 * 4));
     int passes = (bits + 7) / 8;
-    uint64_t* kin = keys;
+    K* kin = keys;
     uint32_t* vin = values;
-    uint64_t* kout = kalt;
+    K* kout = kalt;
     uint32_t* vout = valt;
     for (int pass = 0; pass < passes; ++pass) {
         uint32_t shift = (uint32_t)(pass * 8);
-        k_radix_upsweep<ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, n, shift, tiles, counts);
+        k_radix_upsweep<K, ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, n, shift, tiles, counts);
         k_radix_scan<<<256, SORT_THREADS, 0, stream>>>(counts, totals, tiles);
         const uint32_t* vsrc = (pass == 0 && values_identity) ? nullptr : vin;
-        k_radix_downsweep<ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, vsrc, kout, vout, n, shift, counts,
-                                                                     totals, tiles);
+        k_radix_downsweep<K, ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, vsrc, kout, vout, n, shift, counts,
+                                                                        totals, tiles);
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (kin != keys) {
-        e = hipMemcpyAsync(keys, kin, (size_t)n * 8, hipMemcpyDeviceToDevice, stream);
+        e = hipMemcpyAsync(keys, kin, (size_t)n * sizeof(K), hipMemcpyDeviceToDevice, stream);
         if (e != hipSuccess) return e;
         e = hipMemcpyAsync(values, vin, (size_t)n * 4, hipMemcpyDeviceToDevice, stream);
     }
     return e;
 }
 
-hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
-                            void* scratch, hipStream_t stream, int items) {
+template <class K>
+static hipError_t radix_sort_items(K* keys, uint32_t* values, bool values_identity, uint32_t n, int bits, void* scratch,
+                                   hipStream_t stream, int items) {
     if (n == 0) return hipSuccess;
     switch (items) {
-        case 4: return radix_sort_impl<4>(keys, values, values_identity, n, bits, scratch, stream);
-        case 16: return radix_sort_impl<16>(keys, values, values_identity, n, bits, scratch, stream);
-        default: return radix_sort_impl<8>(keys, values, values_identity, n, bits, scratch, stream);
+        case 4: return radix_sort_impl<K, 4>(keys, values, values_identity, n, bits, scratch, stream);
+        case 16: return radix_sort_impl<K, 16>(keys, values, values_identity, n, bits, scratch, stream);
+        default: return radix_sort_impl<K, 8>(keys, values, values_identity, n, bits, scratch, stream);
     }
+}
+
+hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
+                            void* scratch, hipStream_t stream, int items) {
+    return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
+}
+
+hipError_t radix_sort_pairs32(uint32_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
+                              void* scratch, hipStream_t stream, int items) {
+    return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
 }
 
 }  // namespace obvhs
