@@ -96,7 +96,8 @@ typedef struct obvhs_build_stats {
 
 /* ---- context, memory, timing (no reference counterpart: the crate is CPU-only) ----
  * A context keeps grow-only working memory until it is destroyed: build scratch for its largest build and 224 bytes
- * of traversal stack spill per ray of its largest traversal launch (at most 16M rays' worth, 3.8 GB). */
+ * of traversal stack spill per ray of its largest traversal launch (at most 16M rays' worth, 3.8 GB) and per resident
+ * lane (117 MB). */
 const char* obvhs_status_string(obvhs_status s);
 obvhs_status obvhs_context_create(int device, void* hip_stream, obvhs_context** out);
 obvhs_status obvhs_context_destroy(obvhs_context* ctx);
@@ -118,9 +119,10 @@ obvhs_status obvhs_context_set_trace(obvhs_context* ctx, int enable);
  *                       that distance).  Default 14.
  *   sort_items[c]     : keys per thread of the radix sort's tiles (4, 8 or 16) for a sort of class c.  Default 8.
  *   trav_lds_depth[c] : traversal stack entries kept in LDS (4, 8 or 16) for a BVH of class c.  Default 8.
- *   trav_chunk[c]     : 1: a single-BVH traversal launch of at least two rays per resident lane gives each wave
- *                       interleaved rows of rays and refills a lane as soon as its ray ends (faster for incoherent
- *                       rays, slower for coherent ones); 0: one lane per ray.  Default 0.
+ *   trav_chunk[c]     : 1: a single-BVH traversal launch of at least 1.25 rows of 64 rays per resident wave gives each
+ *                       wave interleaved rows of rays and refills a lane as soon as its ray ends; 0: only the rows
+ *                       whose ray directions differ are traced that way, the others with one lane per ray (batched
+ *                       launches: every row).  Default 0.
  * The last three never change a result, only the speed.  obvhs_tune_* fill entries by measurement. */
 typedef struct obvhs_tune_table {
     uint32_t ploc_radius[4];

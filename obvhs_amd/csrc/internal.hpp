@@ -171,6 +171,7 @@ struct TravScratch {
     uint32_t lanes = 0;
     uint32_t resident = 0;   // lanes the device keeps resident (compute units x 32 waves x 64)
     uint32_t lds_depth = 8;  // stack entries in LDS for the launch (4, 8 or 16); results do not depend on it
+    bool by_row = false;     // launches that are not chunked may be split by row (k_traverse_chunk)
     bool chunked = false;    // wave-owned ray rows with lanes refilled (k_traverse_chunk); results do not depend on it
 };
 // Spill columns (and the lane count) for a traversal launch of n rays.

@@ -8,9 +8,10 @@
 //     slot 31, a pop of the empty stack ends traversal;
 //   * the node test gives the SSE path's results (cwbvh/simd.rs:17-100: mul then add, SSE min/max, tmin clamped to
 //     1e-4, inclusive compare) and the primitive test is Triangle::intersect (triangle.rs:35-76).
-// A step of a lane's walk tests at most TRI_PER_STEP pending triangles and then, once none is left, the next node;
-// an empty node group is replaced by the stack's top at the end of the step.  Each ray's sequence of tests, pushes
-// and pops is the crate's; only how lanes share a wave's steps changes.
+// A step of a lane's walk tests at most TRI_PER_STEP pending triangles (TESTS_PER_STEP in the chunked kernel, whose
+// lanes share them) and then, once none is left, the next node; an empty node group is replaced by the stack's top at
+// the end of the step.  Each ray's sequence of node visits, pushes and pops is the crate's and its triangle results
+// are taken in the crate's order; only how lanes share a wave's steps changes.
 // Stack storage: the bottom LDS entries of each lane's stack live in LDS (one 64-lane column per wave, entry-major;
 // 4, 8 or 16 entries, the depth the context's tuning table holds for the BVH's size class, 8 by default), deeper
 // entries in a per-lane column of an HBM spill array, so LDS does not limit residency.  A launch has one lane per
@@ -19,6 +20,7 @@
 // primitive_indices order) as three.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "cwdp.hpp"
@@ -42,6 +44,16 @@ constexpr float NODE_EPSILON = 0.0001f;  // cwbvh/node.rs:82
 // Triangle tests a lane makes per step of the walk; a lane with more pending keeps them for the next steps and
 // tests its next node only once they are done, so the order of every ray's tests is the crate's.
 constexpr int TRI_PER_STEP = OBVHS_TRI_PER_STEP;
+// A row of 64 rays is coherent when the directions of 8 sampled rays lie within this cosine of the first one's
+// (squared, with the lengths divided out).
+constexpr float ROW_COS2 = 0.9604f;  // 0.98^2
+constexpr uint32_t ROW_SAMPLES = 8;
+// Triangles of a lane that a step of the chunked kernel tests at most.  A step waits for the wave's pending tests, so
+// too few leave lanes that cannot test their next node, too many grow the step: 2 / 3 / 4 / 6 gave 5.95 / 5.58 / 5.36
+// / 5.22 ms on the large scene's 4.19M incoherent rays and 180 / 184 / 193 / 200 us on 1M shadow rays of the
+// heightfield.
+constexpr uint32_t TESTS_PER_STEP = 4;
+constexpr uint32_t CHUNK_MAX_ROWS_PER_WAVE = 16;
 constexpr uint64_t TRAV_MAX_LANES = 1u << 24;  // spill columns (224 B each) for at most 16M lanes: 3.8 GB
 
 struct RayData {
@@ -59,6 +71,21 @@ __device__ __forceinline__ uint32_t octant_inv4(float dx, float dy, float dz) {
 }
 
 __device__ __forceinline__ float byte_f(uint32_t w, int b) { return (float)((w >> (8 * b)) & 0xffu); }
+
+// (byte b of v) << (byte b of by), both bytes selected by the shift itself; by's bytes are below 32.
+__device__ __forceinline__ uint32_t shift_bytes(int b, uint32_t v, uint32_t by) {
+    uint32_t o;
+#define OBVHS_SHIFT_BYTES(B)                                                                                         \
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #B " src1_sel:BYTE_" #B \
+        : "=v"(o)                                                                                                    \
+        : "v"(by), "v"(v))
+    if (b == 0) OBVHS_SHIFT_BYTES(0);
+    else if (b == 1) OBVHS_SHIFT_BYTES(1);
+    else if (b == 2) OBVHS_SHIFT_BYTES(2);
+    else OBVHS_SHIFT_BYTES(3);
+#undef OBVHS_SHIFT_BYTES
+    return o;
+}
 
 // CwBvhNode::intersect_ray_simd (cwbvh/simd.rs:17-100) with get_child_and_index_bits (cwbvh/node.rs:207-231).
 // Node words: q0 = {p.x, p.y, p.z, e|imask}, q1 = {child_base, prim_base, meta lo, meta hi},
@@ -105,13 +132,10 @@ __device__ __forceinline__ uint32_t intersect_node(const uint4& q0, const uint4&
     const float plz = ROBUST ? (rdz ? 1.0f : -1.0f) : 0.0f;
     const float rt = ray_tmax == ray_tmax ? ray_tmax : -INFINITY;
 
-    uint32_t hit_mask = 0u;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const int h = c >> 2, b = c & 3;
-        float xmin = byte_f(h ? lx1 : lx0, b), xmax = byte_f(h ? hx1 : hx0, b);
-        float ymin = byte_f(h ? ly1 : ly0, b), ymax = byte_f(h ? hy1 : hy0, b);
-        float zmin = byte_f(h ? lz1 : lz0, b), zmax = byte_f(h ? hz1 : hz0, b);
+    const uint32_t cb[2] = {(uint32_t)child_bits8, (uint32_t)(child_bits8 >> 32)};
+    const uint32_t bi[2] = {(uint32_t)bit_index8, (uint32_t)(bit_index8 >> 32)};
+    // Whether the ray meets the child with these planes (nan_z: with the NaN rule).
+    auto child = [&](auto nan_z, float xmin, float xmax, float ymin, float ymax, float zmin, float zmax) {
         if (ROBUST) {
             xmin += plx; xmax -= plx;
             ymin += ply; ymax -= ply;
@@ -127,12 +151,34 @@ __device__ __forceinline__ uint32_t intersect_node(const uint4& q0, const uint4&
             tmin = tmin - fabsf(tmin) * k;
             tmax = tmax + fabsf(tmax) * k;
         }
-        tmin = tminz == tminz ? fmaxf(tmin, NODE_EPSILON) : NODE_EPSILON;
-        tmax = tmaxz == tmaxz ? fminf(tmax, rt) : rt;
-        if (tmin <= tmax) {
-            const uint32_t cb = (uint32_t)(child_bits8 >> (c * 8)) & 0xffu;
-            const uint32_t bi = (uint32_t)(bit_index8 >> (c * 8)) & 0xffu;
-            hit_mask |= cb << bi;
+        tmin = !decltype(nan_z)::value || tminz == tminz ? fmaxf(tmin, NODE_EPSILON) : NODE_EPSILON;
+        tmax = !decltype(nan_z)::value || tmaxz == tmaxz ? fminf(tmax, rt) : rt;
+        return tmin <= tmax;
+    };
+    uint32_t hit_mask = 0u;
+    // No child's z slab value is NaN when the node's z terms are finite (a byte times a finite number is no NaN, and
+    // neither is its sum with another one), so the NaN rule is left out where that holds for the whole wave.
+    const bool z_finite = fabsf(adz) < INFINITY && fabsf(aoz) < INFINITY;
+    if (__builtin_expect(__ballot(!z_finite) == 0ull, 1)) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int h = c >> 2, b = c & 3;
+            const bool hit = child(std::false_type{}, byte_f(h ? lx1 : lx0, b), byte_f(h ? hx1 : hx0, b),
+                                   byte_f(h ? ly1 : ly0, b), byte_f(h ? hy1 : hy0, b), byte_f(h ? lz1 : lz0, b),
+                                   byte_f(h ? hz1 : hz0, b));
+            const uint32_t bits = shift_bytes(b, cb[h], bi[h]);
+            hit_mask |= hit ? bits : 0u;
+        }
+    } else {
+#pragma unroll 1
+        for (uint32_t c = 0; c < 8; ++c) {
+            const bool h = c >= 4u;
+            const uint32_t s = 8u * (c & 3u);
+            auto at = [&](uint32_t w0, uint32_t w1) { return (float)(((h ? w1 : w0) >> s) & 0xffu); };
+            const bool hit = child(std::true_type{}, at(lx0, lx1), at(hx0, hx1), at(ly0, ly1), at(hy0, hy1),
+                                   at(lz0, lz1), at(hz0, hz1));
+            const uint32_t bits = (((h ? cb[1] : cb[0]) >> s) & 0xffu) << (((h ? bi[1] : bi[0]) >> s) & 0xffu);
+            hit_mask |= hit ? bits : 0u;
         }
     }
     return hit_mask;
@@ -411,11 +457,40 @@ __global__ void __launch_bounds__(TRAV_THREADS)
     }  // rays of this lane
 }
 
-// k_traverse for one BVH when a launch holds several rays per resident lane: each 64-lane workgroup (one wave)
-// owns per_wave / 64 rows of 64 rays, rows blockIdx.x, blockIdx.x + W, blockIdx.x + 2W, ... (W workgroups, so the
-// waves sweep the rays together, as a one-ray-per-lane grid does), and a lane whose ray ends takes the wave's next
-// ray at the next step (a wave-uniform count of the rays handed out, no atomics) instead of idling until the wave's
-// longest ray ends.  The steps of every ray are k_traverse's, so the hits are identical.
+// Whether row `row` is coherent, from the directions of ROW_SAMPLES of its rays; lane l looks at sample l % ROW_SAMPLES
+// (one past the launch's rays agrees).  The lanes of a group of ROW_SAMPLES call together with the same row and get
+// the same result, and both kernel roles decide a row with this function.
+__device__ __forceinline__ bool row_coherent(const float4* __restrict__ rays, uint64_t row, uint64_t n) {
+    const uint32_t lane = threadIdx.x, sample = lane % ROW_SAMPLES;
+    const uint64_t k = row * TRAV_THREADS + sample * (TRAV_THREADS / ROW_SAMPLES);
+    float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (k < n) d = rays[4 * k + 1];
+    const int first = (int)(lane - sample);
+    const float fx = __shfl(d.x, first), fy = __shfl(d.y, first), fz = __shfl(d.z, first);
+    const float dot = (d.x * fx + d.y * fy) + d.z * fz;
+    const float dd = (d.x * d.x + d.y * d.y) + d.z * d.z, ff = (fx * fx + fy * fy) + fz * fz;
+    const uint64_t differ = __ballot(k < n && !(dot > 0.0f && dot * dot > ROW_COS2 * dd * ff));
+    return ((differ >> first) & ((1ull << ROW_SAMPLES) - 1ull)) == 0ull;
+}
+
+// k_traverse for larger launches: each 64-lane workgroup (one wave) owns rows of 64 rays, and a lane whose ray ends
+// takes the wave's next ray at the next step (a wave-uniform count of the rays handed out, no atomics) instead of
+// idling until the wave's longest ray ends.  Rows blockIdx.x, blockIdx.x + W, blockIdx.x + 2W, ... of `owners` = W
+// workgroups (so the waves sweep the rays together, as a one-ray-per-lane grid does).
+// The triangle tests of a step are shared: the pending ones of all lanes (TESTS_PER_STEP each) are listed in LDS, a
+// ray's data comes to the lane that tests for it through the LDS crossbar, and each ray then takes its own results in
+// its order, so hits equal k_traverse's.  A lane that tests its own triangles leaves the others of the wave idle (8 to
+// 40% of the lanes had one) and, two a step, kept 41% of the live lanes from their next node: the large scene's 4.19M
+// incoherent rays took 6.02 ms that way against 5.35.  Bound by L2 misses there (31 GB at 5.8 TB/s), by VALU issue on
+// smaller scenes.
+// by_row: refilling lanes pays for incoherent rows (the large scene's rays: 13.5 ms with one lane per ray and its own
+// tests) and costs on coherent ones (1.29M heightfield, 2.07M primary rays: 217 -> 255 us; its lanes fall out of
+// step), so the owners take the incoherent rows (row_coherent) and the workgroups behind them (blockIdx.x >= W) the
+// coherent ones, one row each.  Both roles decide each row by themselves, so the launch needs no other pass and no
+// flags; an owner without rows and a row that is not its workgroup's leave at once.  The line: primary rays whose
+// directions were spread, refilled against one lane per ray in us at a smallest cosine of 0.995 / 0.982 / 0.93 / 0.59
+// within the rows: heightfield 266 / 261 / 268 / 257 against 276 / 310 / 440 / 560, soup 276 / 293 / 316 / 296
+// against 252 / 293 / 515 / 950.
 // SRC_MESHES: as in k_traverse, each ray's mesh (ray_mesh) selects its CWBVH and triangle slices; node_count_in is
 // then the mesh count.
 template <int MODE, int LDS, int SRC = SRC_PLAIN>
@@ -423,70 +498,90 @@ __global__ void __launch_bounds__(TRAV_THREADS)
     k_traverse_chunk(const uint4* __restrict__ nodes_in, uint32_t node_count_in, uint32_t prim_count_in,
                      const float4* __restrict__ tris_in, const float4* __restrict__ rays, uint32_t n,
                      obvhs_ray_hit* __restrict__ hits, uint8_t* __restrict__ miss_out, uint2* __restrict__ spill,
-                     uint32_t per_wave, const MeshDesc* __restrict__ meshes, const uint32_t* __restrict__ ray_mesh) {
+                     uint32_t owners, uint32_t by_row, const MeshDesc* __restrict__ meshes,
+                     const uint32_t* __restrict__ ray_mesh) {
     __shared__ uint2 stack[LDS][TRAV_THREADS];
+    __shared__ uint32_t my_rows[CHUNK_MAX_ROWS_PER_WAVE];  // the wave's rows in turn
     const uint32_t lane = threadIdx.x;
     const uint32_t lanes = gridDim.x * TRAV_THREADS;
     uint2* my_spill = spill + blockIdx.x * TRAV_THREADS + lane;  // entry k >= LDS at my_spill[(k - LDS) * lanes]
+    uint32_t per_wave = 0u;  // rays of the wave (64 per row; the launch's last row may hold fewer)
+    {
+        const bool owner = blockIdx.x < owners;
+        const uint32_t first = owner ? blockIdx.x : blockIdx.x - owners, stride = owner ? owners : gridDim.x - owners;
+        // ROW_SAMPLES lanes look at each row, 64 / ROW_SAMPLES rows at a time
+        for (uint32_t j = 0; j < CHUNK_MAX_ROWS_PER_WAVE; j += TRAV_THREADS / ROW_SAMPLES) {
+            if (((uint64_t)j * stride + first) * TRAV_THREADS >= n) break;  // wave-uniform
+            const uint64_t row = (uint64_t)(j + lane / ROW_SAMPLES) * stride + first;
+            const bool mine = row * TRAV_THREADS < n && (!by_row || row_coherent(rays, row, n) != owner);
+            const uint64_t taken = __ballot(mine && lane % ROW_SAMPLES == 0u);
+            if (mine && lane % ROW_SAMPLES == 0u)
+                my_rows[per_wave / TRAV_THREADS + (uint32_t)__popcll(taken & lanemask_lt())] = (uint32_t)row;
+            per_wave += (uint32_t)__popcll(taken) * TRAV_THREADS;
+        }
+        if (per_wave == 0u) return;  // wave-uniform
+        __syncthreads();
+    }
+    __shared__ uint32_t tests[TESTS_PER_STEP * TRAV_THREADS];  // the step's triangle tests, then their results
     uint32_t handed = 0u;  // rays of the chunk handed out so far (the same in every lane)
     bool live = false;
     uint32_t i = 0u;
     RayData r{};
     WtRay wr{};
     uint32_t oct = 0u, hit_id = INVALID32;
-    float tmax = 0.0f, hit_t = INFINITY;
+    float tmax = 0.0f;
     bool is_miss = true;
     int sp = 0;
     uint2 cur = make_uint2(0u, 0u), prim = make_uint2(0u, 0u);
     const uint4* nodes = nodes_in;
-    const float4* tris = tris_in;
-    uint32_t node_count = node_count_in, prim_count = prim_count_in;
+    uint32_t node_count = node_count_in, prim_begin = 0u, prim_end = prim_count_in;  // the ray's BVH (slices for meshes)
+    auto start = [&](uint32_t ray) {
+        i = ray;
+        const float4 ra = rays[4 * (size_t)i], rb = rays[4 * (size_t)i + 1], rc = rays[4 * (size_t)i + 2],
+                     rd = rays[4 * (size_t)i + 3];
+        r = RayData{ra.x, ra.y, ra.z, rb.x, rb.y, rb.z, rc.x, rc.y, rc.z, rd.x, rd.y};
+        oct = octant_inv4(r.dx, r.dy, r.dz);
+        if (MODE & 2) wr = wt_ray(r);
+        tmax = r.tmax;
+        hit_id = INVALID32;
+        is_miss = true;
+        sp = 0;
+        cur = node_count == 0u ? make_uint2(0u, 0u) : make_uint2(0u, 0x80000000u);
+        prim = make_uint2(0u, 0u);
+        live = true;
+    };
     for (;;) {
-        const uint64_t want = __ballot(!live);
+        const uint64_t want = handed < per_wave ? __ballot(!live) : 0ull;
         if (want != 0ull) {
             if (!live) {
-                // the h-th ray handed out in this wave: row h / 64 of the wave's rows blockIdx.x, blockIdx.x + W, ...
+                // the h-th ray handed out in this wave: ray h % 64 of the (h / 64)-th of its rows
                 const uint32_t h = handed + (uint32_t)__popcll(want & lanemask_lt());
-                const uint64_t k = ((uint64_t)(h / TRAV_THREADS) * gridDim.x + blockIdx.x) * TRAV_THREADS +
-                                   h % TRAV_THREADS;
-                if (h < per_wave && k < n) {
-                    i = (uint32_t)k;
+                const uint64_t k = h < per_wave ? (uint64_t)my_rows[h / TRAV_THREADS] * TRAV_THREADS + h % TRAV_THREADS
+                                                : (uint64_t)n;
+                if (k < n) {
                     if (SRC == SRC_MESHES) {  // the ray's mesh; an out-of-range id sees an empty BVH (a miss)
-                        const uint32_t mi = ray_mesh[i];
+                        const uint32_t mi = ray_mesh[k];
                         nodes = nodes_in;
-                        tris = tris_in;
                         node_count = 0u;
-                        prim_count = 0u;
+                        prim_begin = 0u;
+                        prim_end = 0u;
                         if (mi < node_count_in) {
                             const MeshDesc md = meshes[mi];
                             nodes += (size_t)md.cw_base * 5;
-                            tris += (size_t)md.prim_base * 3;
                             node_count = md.cw_count;
-                            prim_count = md.prim_count;
+                            prim_begin = md.prim_base;
+                            prim_end = md.prim_base + md.prim_count;
                         }
                     }
-                    const float4 ra = rays[4 * (size_t)i], rb = rays[4 * (size_t)i + 1], rc = rays[4 * (size_t)i + 2],
-                                 rd = rays[4 * (size_t)i + 3];
-                    r = RayData{ra.x, ra.y, ra.z, rb.x, rb.y, rb.z, rc.x, rc.y, rc.z, rd.x, rd.y};
-                    oct = octant_inv4(r.dx, r.dy, r.dz);
-                    if (MODE & 2) wr = wt_ray(r);
-                    tmax = r.tmax;
-                    hit_id = INVALID32;
-                    hit_t = INFINITY;
-                    is_miss = true;
-                    sp = 0;
-                    cur = node_count == 0u ? make_uint2(0u, 0u) : make_uint2(0u, 0x80000000u);
-                    prim = make_uint2(0u, 0u);
-                    live = true;
+                    start((uint32_t)k);
                 }
             }
             handed = min(handed + (uint32_t)__popcll(want), per_wave);
         }
         if (__ballot(live) == 0ull) break;  // the chunk is done (wave-uniform)
-        if (!live) continue;
-        // one step of k_traverse's loop
-        bool done = false;
-        const bool node_next = (cur.y & 0xff000000u) != 0u && __popc(prim.y) <= TRI_PER_STEP;
+        // one step of k_traverse's loop (a lane that is not live has no pending triangle and no node)
+        constexpr uint32_t PER_STEP = (MODE & 2) ? (uint32_t)TRI_PER_STEP : TESTS_PER_STEP;
+        const bool node_next = live && (cur.y & 0xff000000u) != 0u && (uint32_t)__popc(prim.y) <= PER_STEP;
         uint32_t child = 0u;
         uint4 q0, q1, q2, q3, q4;
         if (node_next) {
@@ -501,59 +596,106 @@ __global__ void __launch_bounds__(TRAV_THREADS)
                 q4 = np[4];
             }
         }
-        for (int k = 0; k < TRI_PER_STEP && prim.y != 0u; ++k) {
-            const uint32_t local = firstbithigh(prim.y);
-            prim.y &= ~(1u << local);
-            const uint32_t pid = prim.x + local;
-            if (pid >= prim_count) continue;  // malformed input only: never index past the triangle buffer
+        bool done = false;
+        auto result = [&](uint32_t pid, float t) {  // of the lane's tests in order
             if ((MODE & 1) == 0) {
-                const float t = prim_test<MODE>(tris, pid, r, wr, r.tmin, tmax);
                 if (t < tmax) {
                     hit_id = pid;
-                    hit_t = t;
                     tmax = t;
                 }
-            } else {
-                const float t = prim_test<MODE>(tris, pid, r, wr, r.tmin, r.tmax);
-                if (t < r.tmax) {
-                    is_miss = false;
-                    done = true;
-                    break;
+            } else if (t < r.tmax) {
+                is_miss = false;
+                done = true;
+            }
+        };
+        if (MODE & 2) {
+            for (int k = 0; k < TRI_PER_STEP && prim.y != 0u && !done; ++k) {
+                const uint32_t local = firstbithigh(prim.y);
+                prim.y &= ~(1u << local);
+                const uint32_t pid = prim.x + local;
+                if (pid >= prim_end) continue;  // malformed input only: never index past the triangle buffer
+                result(pid, prim_test<MODE>(tris_in, pid, r, wr, r.tmin, (MODE & 1) ? r.tmax : tmax));
+            }
+        } else if (__ballot(prim.y != 0u) != 0ull) {
+            uint32_t rest = prim.y, total = 0u, at[TESTS_PER_STEP];
+#pragma unroll
+            for (uint32_t k = 0; k < TESTS_PER_STEP; ++k) {  // each lane's k-th pending triangle, lanes in order
+                const uint64_t m = __ballot(rest != 0u);
+                at[k] = total + (uint32_t)__popcll(m & lanemask_lt());
+                if (rest != 0u) {
+                    const uint32_t local = firstbithigh(rest);
+                    rest &= ~(1u << local);
+                    // malformed input only (bit 31): never index past the triangle buffer
+                    tests[at[k]] = lane | local << 6 | (prim.x + local < prim_end ? 0u : 0x80000000u);
+                }
+                total += (uint32_t)__popcll(m);
+            }
+            for (uint32_t b = 0; b < total; b += TRAV_THREADS) {
+                const uint32_t e = b + lane < total ? tests[b + lane] : 0x80000000u;
+                const int owner = (int)(e & 63u);
+                RayData o{};
+                o.ox = __shfl(r.ox, owner);
+                o.oy = __shfl(r.oy, owner);
+                o.oz = __shfl(r.oz, owner);
+                o.dx = __shfl(r.dx, owner);
+                o.dy = __shfl(r.dy, owner);
+                o.dz = __shfl(r.dz, owner);
+                const uint32_t pid = (uint32_t)__shfl((int)prim.x, owner) + ((e >> 6) & 31u);
+                if (b + lane < total) {
+                    float t = INFINITY;
+                    if (!(e & 0x80000000u)) t = prim_test<MODE>(tris_in, pid, o, wr, -INFINITY, INFINITY);
+                    tests[b + lane] = __float_as_uint(t);
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < TESTS_PER_STEP; ++k) {
+                if (prim.y != 0u && !done) {
+                    const uint32_t local = firstbithigh(prim.y);
+                    prim.y &= ~(1u << local);
+                    const float t = __uint_as_float(tests[at[k]]);
+                    if (t >= r.tmin) result(prim.x + local, t);
                 }
             }
         }
-        if (!done) {
-            if (node_next) {  // the group's triangles are all tested (at most TRI_PER_STEP were pending)
-                cur.y &= ~(1u << firstbithigh(cur.y));
-                if ((cur.y & 0xff000000u) != 0u) {
-                    if (sp < LDS) stack[sp][lane] = cur;
-                    else my_spill[(size_t)(sp - LDS) * lanes] = cur;
-                    sp = min(sp + 1, STACK_SIZE - 1);
+        if (live) {
+            if (!done) {
+                if (node_next) {  // the group's triangles are all tested (at most PER_STEP were pending)
+                    cur.y &= ~(1u << firstbithigh(cur.y));
+                    if ((cur.y & 0xff000000u) != 0u) {
+                        if (sp < LDS) stack[sp][lane] = cur;
+                        else my_spill[(size_t)(sp - LDS) * lanes] = cur;
+                        sp = min(sp + 1, STACK_SIZE - 1);
+                    }
+                    if (child >= node_count) {
+                        done = true;  // malformed input only: never index past the node buffer
+                    } else {
+                        const uint32_t hm = intersect_node<(MODE & 2) != 0>(q0, q1, q2, q3, q4, r, tmax, oct);
+                        const uint32_t imask = (q0.w >> 24) & 0xffu;
+                        cur = make_uint2(q1.x, (hm & 0xff000000u) | imask);
+                        prim = make_uint2(prim_begin + q1.y, hm & 0x00ffffffu);
+                    }
                 }
-                if (child >= node_count) {
-                    done = true;  // malformed input only: never index past the node buffer
-                } else {
-                    const uint32_t hm = intersect_node<(MODE & 2) != 0>(q0, q1, q2, q3, q4, r, tmax, oct);
-                    const uint32_t imask = (q0.w >> 24) & 0xffu;
-                    cur = make_uint2(q1.x, (hm & 0xff000000u) | imask);
-                    prim = make_uint2(q1.y, hm & 0x00ffffffu);
+                if (!done && (cur.y & 0xff000000u) == 0u) {  // the early pop of k_traverse
+                    if (sp == 0) {
+                        done = prim.y == 0u;
+                    } else {
+                        sp -= 1;
+                        cur = sp < LDS ? stack[sp][lane] : my_spill[(size_t)(sp - LDS) * lanes];
+                    }
                 }
             }
-            if (!done && (cur.y & 0xff000000u) == 0u) {  // the early pop of k_traverse
-                if (sp == 0) {
-                    done = prim.y == 0u;
+            if (done) {
+                if ((MODE & 1) == 0) {
+                    const bool hit = hit_id != INVALID32;
+                    reinterpret_cast<uint4*>(hits)[i] = make_uint4(hit ? hit_id - prim_begin : INVALID32, INVALID32,
+                                                                   INVALID32, __float_as_uint(hit ? tmax : INFINITY));
                 } else {
-                    sp -= 1;
-                    cur = sp < LDS ? stack[sp][lane] : my_spill[(size_t)(sp - LDS) * lanes];
+                    miss_out[i] = is_miss ? 1 : 0;
                 }
+                live = false;
+                prim.y = 0u;
+                cur.y = 0u;
             }
-        }
-        if (done) {
-            if ((MODE & 1) == 0)
-                reinterpret_cast<uint4*>(hits)[i] = make_uint4(hit_id, INVALID32, INVALID32, __float_as_uint(hit_t));
-            else
-                miss_out[i] = is_miss ? 1 : 0;
-            live = false;
         }
     }
 }
@@ -746,10 +888,16 @@ static void launch_depth(uint32_t depth, uint32_t blocks, hipStream_t stream, A.
 // register and LDS use, times the compute units) that the rows of 64 rays are dealt over, rows w, w + W, ... to wave
 // w, so no wave waits for a slot while others run (with a grid of 32 waves per CU and 7 resident, the last 4 per CU
 // started as the first finished and ran alone at the end).  At most CHUNK_MAX_ROWS_PER_WAVE rows per wave; larger
-// launches have more waves than slots.
-constexpr uint32_t CHUNK_MAX_ROWS_PER_WAVE = 16;
+// launches have more waves than slots.  Split by row: as many more workgroups as rows (each looks at its row and
+// traces it when it is coherent), or as the spill columns allow with up to CHUNK_MAX_ROWS_PER_WAVE rows each.
+// Refilling pays from 1.25 rows per resident wave (727K bounce rays, 1.85 rows per wave: 268 -> 222 us); below, and
+// where the table does not ask for it and rows are not looked at (batched launches), each wave has one row, as long
+// as a CU holds CHUNK_MIN_WAVES_PER_CU of them.  With fewer waves a step's latency shows, which is shorter where each
+// lane tests its own triangles (65K rays: 88 us in k_traverse, 106 here; 300K: 258, 247; 500K: 147, 136).
+constexpr uint32_t CHUNK_MIN_WAVES_PER_CU = 16;
 struct ChunkPlan {
-    uint32_t blocks = 0, per_wave = 0;  // per_wave = rays (64 per row) a wave's lanes take in turn
+    uint32_t blocks = 0, owners = 0;
+    bool by_row = false;
 };
 
 template <class K>
@@ -762,37 +910,49 @@ static uint32_t resident_waves_per_cu(K kernel) {
     return (uint32_t)nb;
 }
 
-// The plan for k_traverse_chunk<MODE, LDS, SRC> over n rays; blocks = 0 when the launch should not be chunked (fewer
-// than two rows per resident wave, or more waves than spill columns).
+// The plan for k_traverse_chunk<MODE, LDS, SRC> over n rays; blocks = 0 for k_traverse (few rays, or more waves than
+// spill columns).
 template <int MODE, int LDS, int SRC>
-static ChunkPlan chunk_plan(uint32_t n, const TravScratch& ts) {
+static ChunkPlan chunk_plan(uint32_t n, const TravScratch& ts, bool by_row) {
     static const uint32_t per_cu = resident_waves_per_cu(k_traverse_chunk<MODE, LDS, SRC>);
     ChunkPlan p;
-    if (!ts.chunked || per_cu == 0u || ts.resident == 0u) return p;
+    if (per_cu == 0u || ts.resident == 0u) return p;
     const uint64_t cus = std::max<uint32_t>(1u, ts.resident / (32u * TRAV_THREADS));
     const uint64_t waves = cus * per_cu;
     const uint64_t rows = ((uint64_t)n + TRAV_THREADS - 1) / TRAV_THREADS;
-    if (rows < 2u * waves) return p;
+    const uint64_t columns = ts.lanes / TRAV_THREADS;
+    if ((!ts.chunked && !by_row) || 4u * rows < 5u * waves) {  // one row per wave
+        if (rows < cus * CHUNK_MIN_WAVES_PER_CU || rows > columns) return p;
+        p.blocks = p.owners = (uint32_t)rows;
+        return p;
+    }
     // every resident slot takes a wave (rows dealt one at a time: the waves' row counts differ by at most one)
     const uint64_t per = std::min<uint64_t>((rows + waves - 1) / waves, CHUNK_MAX_ROWS_PER_WAVE);
-    const uint64_t blocks = std::max<uint64_t>(waves, (rows + per - 1) / per);
-    if (blocks * TRAV_THREADS > ts.lanes) return p;
-    p.blocks = (uint32_t)blocks;
-    p.per_wave = (uint32_t)(per * TRAV_THREADS);
+    const uint64_t owners = std::max<uint64_t>(waves, (rows + per - 1) / per);
+    if (owners > columns) return p;
+    uint64_t behind = 0;  // workgroups of the coherent rows
+    if (by_row) {
+        behind = std::min<uint64_t>(rows, columns - owners);
+        if (behind * CHUNK_MAX_ROWS_PER_WAVE < rows) return p;
+    }
+    p.owners = (uint32_t)owners;
+    p.blocks = (uint32_t)(owners + behind);
+    p.by_row = by_row;
     return p;
 }
 
-// k_traverse_chunk<MODE, depth, SRC> with the launch's LDS stack depth, when chunk_plan chunks the launch; false
-// (nothing launched) otherwise.
+// k_traverse_chunk<MODE, depth, SRC> with the launch's LDS stack depth, when chunk_plan has a plan; false (nothing
+// launched) otherwise.  Single-BVH launches whose table entry does not ask for chunking are split by row.
 template <int MODE, int SRC, int LDS>
 static bool launch_chunk_depth(uint32_t n, const TravScratch& ts, hipStream_t stream, const uint4* nd,
                                uint32_t node_count, uint32_t prim_count, const float4* tr, const float4* ry,
                                obvhs_ray_hit* hits, uint8_t* miss, uint2* sp, const MeshDesc* meshes,
                                const uint32_t* ray_mesh) {
-    const ChunkPlan p = chunk_plan<MODE, LDS, SRC>(n, ts);
+    const bool by_row = SRC == SRC_PLAIN && !ts.chunked && ts.by_row;
+    const ChunkPlan p = chunk_plan<MODE, LDS, SRC>(n, ts, by_row);
     if (!p.blocks) return false;
     k_traverse_chunk<MODE, LDS, SRC><<<p.blocks, TRAV_THREADS, 0, stream>>>(
-        nd, node_count, prim_count, tr, ry, n, hits, miss, sp, p.per_wave, meshes, ray_mesh);
+        nd, node_count, prim_count, tr, ry, n, hits, miss, sp, p.owners, p.by_row ? 1u : 0u, meshes, ray_mesh);
     return true;
 }
 
@@ -829,8 +989,6 @@ hipError_t launch_traverse(const CwNode* nodes, uint32_t node_count, uint32_t pr
     const MeshDesc* no_meshes = nullptr;
     const uint32_t* no_map = nullptr;
     const TraceSegment* no_segs = nullptr;
-    // Chunked launches (when the tuning table asks for them: incoherent rays) need at least two rows per resident
-    // wave; each lane then takes that many rays in turn, refilled in the wave.
     if (mode > 5 || (node_visits && mode != 0)) return hipErrorInvalidValue;
     if (!node_visits) {
         bool chunked = false;
@@ -921,7 +1079,8 @@ obvhs_status traverse_scratch(obvhs_context* ctx, TravScratch& ts, uint64_t n) {
         ctx->trav_lanes = (uint32_t)std::max(1, prop.multiProcessorCount) * 32u * TRAV_THREADS;
     }
     const uint64_t want = (std::min<uint64_t>(n, TRAV_MAX_LANES) + TRAV_THREADS - 1) / TRAV_THREADS * TRAV_THREADS;
-    const uint32_t lanes = (uint32_t)std::max<uint64_t>(ctx->trav_lanes, want);
+    uint32_t lanes = (uint32_t)std::max<uint64_t>(ctx->trav_lanes, want);
+    if (n > ctx->trav_lanes) lanes += ctx->trav_lanes;  // the owners of a launch split by row (k_traverse_chunk)
     // columns for the shallowest LDS depth a launch may use (4): every depth's spill fits
     const size_t bytes = (size_t)lanes * (STACK_SIZE - 4) * sizeof(uint2);
     const hipError_t e = ctx->scratch.trav_spill.ensure(bytes);
@@ -929,6 +1088,7 @@ obvhs_status traverse_scratch(obvhs_context* ctx, TravScratch& ts, uint64_t n) {
     ts.spill = ctx->scratch.trav_spill.ptr;
     ts.lanes = lanes;
     ts.resident = ctx->trav_lanes;
+    ts.by_row = true;
     return OBVHS_OK;
 }
 
