@@ -88,79 +88,63 @@ __device__ __forceinline__ uint32_t dleft(uint32_t b) { return (b >> 2) & 7u; }
 __device__ __forceinline__ uint32_t dright(uint32_t b) { return (b >> 5) & 7u; }
 __device__ __forceinline__ uint32_t dpack(uint32_t k, uint32_t l, uint32_t r) { return k | (l << 2) | (r << 5); }
 
-// Decision i of an internal node's entry.
-__device__ __forceinline__ uint32_t node_decision(const DpView& dp, uint32_t first_index, uint32_t i) {
-    return dbyte(dp.rec[dp_key(dp, first_index)].meta, i);
-}
-__device__ __forceinline__ uint32_t node_kind(const DpView& dp, const Node32& nx, uint32_t i) {
-    return nx.prim_count != 0u ? KIND_LEAF : dkind(node_decision(dp, nx.first_index, i));
-}
-
-// Everything the parent's evaluation needs from one child.  (Per-decision values selected by a runtime index are
-// read from memory, not from a register array, so the evaluation stays free of private-memory spills.)
+// Everything the parent's evaluation needs from one child, in registers: the whole record's loads go out together.
 struct ChildDp {
     float cost[7];
-    uint2 meta;       // seven decision bytes
-    size_t key;
-    uint2 subdepth;
+    uint32_t size[7];   // per decision, the CWBVH nodes the child contributes when taken through it
+    uint32_t depth[7];  // per decision, the CWBVH levels below the parent through it
     uint32_t nprims;
-    uint32_t cwsize;
-    uint32_t cwdepth;
+    uint4 plist;        // leaf list (nprims <= 3)
     bool leaf;
 };
 
+// Contributions of a child taken through decision d: its own CWBVH subtree (size and depth) when it becomes a CWBVH
+// child, those of its distributed descendants when it is DISTRIBUTE, nothing when it is a leaf child.  SUB_INVALID
+// marks a subtree that cannot be built.
 __device__ __forceinline__ void load_child_dp(const DpView& dp, const Node32& c, ChildDp& o) {
     o.leaf = c.prim_count != 0u;
     if (o.leaf) {
         const float leaf = half_area(node_box(c)) * (float)c.prim_count * PRIM_COST;
 #pragma unroll
-        for (int k = 0; k < 7; ++k) o.cost[k] = leaf;
-        o.meta = make_uint2(0u, 0u);
-        o.subdepth = make_uint2(0u, 0u);
-        o.key = 0;
+        for (int k = 0; k < 7; ++k) {
+            o.cost[k] = leaf;
+            o.size[k] = 0u;
+            o.depth[k] = 0u;
+        }
         o.nprims = c.prim_count;
-        o.cwsize = 1u;
-        o.cwdepth = 1u;
+        o.plist = make_uint4(c.first_index, 0u, 0u, 1u);
     } else {
-        o.key = dp_key(dp, c.first_index);
-        const DpRec& e = dp.rec[o.key];
-        const float4 c0 = *reinterpret_cast<const float4*>(&e.cost[0]);
-        const float4 c1 = *reinterpret_cast<const float4*>(&e.cost[4]);  // cost[4..6], nprims
-        const uint4 m = *reinterpret_cast<const uint4*>(&e.meta);         // meta, subdepth
-        o.cost[0] = c0.x;
-        o.cost[1] = c0.y;
-        o.cost[2] = c0.z;
-        o.cost[3] = c0.w;
-        o.cost[4] = c1.x;
-        o.cost[5] = c1.y;
-        o.cost[6] = c1.z;
-        o.nprims = __float_as_uint(c1.w);
-        o.meta = make_uint2(m.x, m.y);
-        o.subdepth = make_uint2(m.z, m.w);
-        o.cwsize = e.cwsize;
-        o.cwdepth = e.cwdepth;
+        const uint4* e = reinterpret_cast<const uint4*>(&dp.rec[dp_key(dp, c.first_index)]);
+        const uint4 c0 = e[0], c1 = e[1], s0 = e[2], s1 = e[3], m = e[4], kc = e[5];
+        o.plist = e[6];
+        o.cost[0] = __uint_as_float(c0.x);
+        o.cost[1] = __uint_as_float(c0.y);
+        o.cost[2] = __uint_as_float(c0.z);
+        o.cost[3] = __uint_as_float(c0.w);
+        o.cost[4] = __uint_as_float(c1.x);
+        o.cost[5] = __uint_as_float(c1.y);
+        o.cost[6] = __uint_as_float(c1.z);
+        o.nprims = c1.w;
+        const uint32_t sub[7] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z};
+        const uint32_t cwsize = s1.w, cwdepth = kc.z;
+        const uint2 meta = make_uint2(m.x, m.y), subdepth = make_uint2(m.z, m.w);
+        const bool internal = dkind(dbyte(meta, 0u)) == KIND_INTERNAL;
+        const uint32_t size0 = internal ? (cwsize == 0u ? SUB_INVALID : cwsize) : 0u, depth0 = internal ? cwdepth : 0u;
+#pragma unroll
+        for (uint32_t d = 0; d < 7u; ++d) {
+            const bool dist = dkind(dbyte(meta, d)) == KIND_DISTRIBUTE;
+            o.size[d] = dist ? sub[d] : size0;
+            o.depth[d] = dist ? dbyte(subdepth, d) : depth0;
+        }
     }
-}
-
-// Contribution of child c taken through its decision d: its own CWBVH subtree when it becomes a CWBVH child,
-// the contributions of its distributed descendants when it is DISTRIBUTE, nothing when it is a leaf child.
-__device__ __forceinline__ uint32_t child_contribution(const DpView& dp, const ChildDp& c, uint32_t d) {
-    if (c.leaf) return 0u;
-    if (dkind(dbyte(c.meta, d)) == KIND_DISTRIBUTE) return dp.rec[c.key].sub[d];
-    if (dkind(dbyte(c.meta, 0u)) == KIND_INTERNAL) return c.cwsize == 0u ? SUB_INVALID : c.cwsize;
-    return 0u;
-}
-
-// Depth counterpart of child_contribution.
-__device__ __forceinline__ uint32_t child_depth(const ChildDp& c, uint32_t d) {
-    if (c.leaf) return 0u;
-    if (dkind(dbyte(c.meta, d)) == KIND_DISTRIBUTE) return dbyte(c.subdepth, d);
-    if (dkind(dbyte(c.meta, 0u)) == KIND_INTERNAL) return c.cwdepth;
-    return 0u;
 }
 
 // Evaluates the entry of the internal node with box `box` whose children records are `l` and `r` (slots first,
 // first + 1) and stores it under its key.  Returns a DERR_* bit or 0.
+// The sizes and depths below the chosen pair of decisions are carried along with its cost, so the evaluation is one
+// round of loads, arithmetic and one round of stores.  (Reading the chosen pair's sizes from the records afterwards
+// took up to 14 loads one after the other, each behind its own branch: 9.7K of the 16.8K cycles of a pass of
+// k_ploc_tail, where the entries wait on nothing else.)
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                 const Node32& r) {
     if ((l.prim_count != 0u && l.prim_count != 1u) || (r.prim_count != 0u && r.prim_count != 1u))
@@ -171,19 +155,25 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     const uint32_t num_primitives = L.nprims + R.nprims;
     const float ha = half_area(box);
     float cost[7];
-    uint32_t meta[7];
+    uint32_t meta[7], sub[7], sd[7];
     {
         const float cost_leaf =
             num_primitives <= dp.max_prims ? ((float)num_primitives) * ha * PRIM_COST : INFINITY;
         float cost_distribute = INFINITY;
         uint32_t dl = DIDX_INVALID, dr = DIDX_INVALID;
+        sub[0] = SUB_INVALID;
+        sd[0] = 0u;
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
             const float c = L.cost[k] + R.cost[6 - k];
+            const uint32_t size = __builtin_elementwise_add_sat(L.size[k], R.size[6 - k]);  // SUB_INVALID stays
+            const uint32_t depth = max(L.depth[k], R.depth[6 - k]);
             if (c < cost_distribute) {
                 cost_distribute = c;
                 dl = (uint32_t)k;
                 dr = (uint32_t)(6 - k);
+                sub[0] = size;
+                sd[0] = depth;
             }
         }
         const float cost_internal = cost_distribute + ha;
@@ -199,13 +189,19 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     for (int i = 1; i < 7; ++i) {
         float cost_distribute = cost[i - 1];
         uint32_t dl = DIDX_INVALID, dr = DIDX_INVALID;
+        sub[i] = sub[i - 1];
+        sd[i] = sd[i - 1];
 #pragma unroll
         for (int k = 0; k < i; ++k) {
             const float c = L.cost[k] + R.cost[i - k - 1];
+            const uint32_t size = __builtin_elementwise_add_sat(L.size[k], R.size[i - k - 1]);
+            const uint32_t depth = max(L.depth[k], R.depth[i - k - 1]);
             if (c < cost_distribute) {
                 cost_distribute = c;
                 dl = (uint32_t)k;
                 dr = (uint32_t)(i - k - 1);
+                sub[i] = size;
+                sd[i] = depth;
             }
         }
         if (dl != DIDX_INVALID) {
@@ -216,28 +212,14 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
             meta[i] = meta[i - 1];
         }
     }
-    uint32_t sub[7], sd[7];
 #pragma unroll
-    for (int i = 0; i < 7; ++i) {
-        const uint32_t dl = dleft(meta[i]), dr = dright(meta[i]);
-        if (dl == DIDX_INVALID || dr == DIDX_INVALID) {
-            sub[i] = SUB_INVALID;
-            sd[i] = 0u;
-        } else {
-            const uint32_t a = child_contribution(dp, L, dl), b = child_contribution(dp, R, dr);
-            sub[i] = (a == SUB_INVALID || b == SUB_INVALID) ? SUB_INVALID : a + b;
-            sd[i] = min(255u, max(child_depth(L, dl), child_depth(R, dr)));
-        }
-    }
+    for (int i = 0; i < 7; ++i) sd[i] = min(255u, sd[i]);
+    // The leaves count_primitives (bvh2_to_cwbvh.rs:197-211) visits, left subtree first.  Each child holds at least
+    // one leaf, so the left list has one or two entries.
     uint4 pl = make_uint4(0u, 0u, 0u, 0u);
-    if (num_primitives <= 3u) {
-        // The leaves count_primitives (bvh2_to_cwbvh.rs:197-211) visits, left subtree first.  Each child holds at
-        // least one leaf, so the left list has one or two entries.
-        uint4 a = make_uint4(l.first_index, 0u, 0u, 1u), c = make_uint4(r.first_index, 0u, 0u, 1u);
-        if (!L.leaf) a = dp.rec[L.key].plist;
-        if (!R.leaf) c = dp.rec[R.key].plist;
-        pl = a.w >= 2u ? make_uint4(a.x, a.y, c.x, num_primitives) : make_uint4(a.x, c.x, c.y, num_primitives);
-    }
+    if (num_primitives <= 3u)
+        pl = L.plist.w >= 2u ? make_uint4(L.plist.x, L.plist.y, R.plist.x, num_primitives)
+                             : make_uint4(L.plist.x, R.plist.x, R.plist.y, num_primitives);
     // The whole 128-byte entry in eight 16-byte stores (the padding too, so that no 32-byte sector of the line is
     // left partly written).
     uint4* e = reinterpret_cast<uint4*>(&dp.rec[dp_key(dp, first)]);
@@ -253,63 +235,6 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     e[6] = pl;
     e[7] = make_uint4(0u, 0u, 0u, 0u);
     return 0u;
-}
-
-// get_children(node, 0) from the cost table alone: the node's children are the slots first and first + 1 and their
-// first_index values are in its `kids` entry, so each level of the walk loads one entry (decisions and children
-// together) instead of a node and then its decisions.  Children are appended left-first like the reference's
-// recursion (bvh2_to_cwbvh.rs:346-397).  Outputs per child: its slot, and its decision-0 kind in 2 bits of *kinds.
-// Returns the count, -1 when more than 8 children would be produced, -2 on a malformed decision (distribute index
-// invalid).
-__device__ __forceinline__ int get_children_kids(const DpView& dp, uint32_t first, uint32_t meta0, uint32_t* children,
-                                                 uint32_t* kinds) {
-    uint32_t stk_slot[8], stk_info[8], stk_i[8];
-    int sp = 0;
-    int cc = 0;
-    uint32_t kb = 0u;
-    const uint32_t dl = dleft(meta0), dr = dright(meta0);
-    if (dl == DIDX_INVALID || dr == DIDX_INVALID) return -2;
-    const uint2 k0 = dp.rec[dp_key(dp, first)].kids;
-    stk_slot[0] = first + 1u;
-    stk_info[0] = k0.y;
-    stk_i[0] = dr;
-    stk_slot[1] = first;
-    stk_info[1] = k0.x;
-    stk_i[1] = dl;
-    sp = 2;
-    while (sp > 0) {
-        sp--;
-        const uint32_t x = stk_slot[sp], info = stk_info[sp], i = stk_i[sp];
-        uint32_t kind0 = KIND_LEAF;
-        if (!(info & KID_LEAF)) {  // a leaf is never DISTRIBUTE
-            const uint32_t f = info & ~KID_LEAF;
-            const size_t key = dp_key(dp, f);
-            const uint2 m = dp.rec[key].meta;
-            const uint2 kx = dp.rec[key].kids;  // same line as the decisions; used when the child is distributed
-            const uint32_t b = dbyte(m, i);
-            if (dkind(b) == KIND_DISTRIBUTE) {
-                const uint32_t cl = dleft(b), cr = dright(b);
-                if (cl == DIDX_INVALID || cr == DIDX_INVALID) return -2;
-                if (sp + 2 > 8) return -1;
-                stk_slot[sp] = f + 1u;
-                stk_info[sp] = kx.y;
-                stk_i[sp] = cr;
-                sp++;
-                stk_slot[sp] = f;
-                stk_info[sp] = kx.x;
-                stk_i[sp] = cl;
-                sp++;
-                continue;
-            }
-            kind0 = dkind(dbyte(m, 0u));
-        }
-        if (cc >= 8) return -1;
-        children[cc] = x;
-        kb |= kind0 << (2 * cc);
-        cc++;
-    }
-    *kinds = kb;
-    return cc;
 }
 
 }  // namespace obvhs
