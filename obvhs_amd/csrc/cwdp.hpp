@@ -88,141 +88,118 @@ __device__ __forceinline__ uint32_t dleft(uint32_t b) { return (b >> 2) & 7u; }
 __device__ __forceinline__ uint32_t dright(uint32_t b) { return (b >> 5) & 7u; }
 __device__ __forceinline__ uint32_t dpack(uint32_t k, uint32_t l, uint32_t r) { return k | (l << 2) | (r << 5); }
 
-// Everything the parent's evaluation needs from one child, in registers: the whole record's loads go out together.
+// Everything the parent's evaluation needs from one child, in registers.
 struct ChildDp {
     float cost[7];
     uint32_t size[7];   // per decision, the CWBVH nodes the child contributes when taken through it
     uint32_t depth[7];  // per decision, the CWBVH levels below the parent through it
     uint32_t nprims;
     uint4 plist;        // leaf list (nprims <= 3)
-    bool leaf;
 };
 
-// Contributions of a child taken through decision d: its own CWBVH subtree (size and depth) when it becomes a CWBVH
-// child, those of its distributed descendants when it is DISTRIBUTE, nothing when it is a leaf child.  SUB_INVALID
-// marks a subtree that cannot be built.
-__device__ __forceinline__ void load_child_dp(const DpView& dp, const Node32& c, ChildDp& o) {
-    o.leaf = c.prim_count != 0u;
-    if (o.leaf) {
-        const float leaf = half_area(node_box(c)) * (float)c.prim_count * PRIM_COST;
+// The first 112 bytes of a record, as loaded.
+struct DpRaw {
+    uint4 w[7];
+};
+__device__ __forceinline__ DpRaw load_dp_raw(const DpRec* rec) {
+    const uint4* e = reinterpret_cast<const uint4*>(rec);
+    DpRaw r;
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            o.cost[k] = leaf;
-            o.size[k] = 0u;
-            o.depth[k] = 0u;
-        }
-        o.nprims = c.prim_count;
-        o.plist = make_uint4(c.first_index, 0u, 0u, 1u);
-    } else {
-        const uint4* e = reinterpret_cast<const uint4*>(&dp.rec[dp_key(dp, c.first_index)]);
-        const uint4 c0 = e[0], c1 = e[1], s0 = e[2], s1 = e[3], m = e[4], kc = e[5];
-        o.plist = e[6];
-        o.cost[0] = __uint_as_float(c0.x);
-        o.cost[1] = __uint_as_float(c0.y);
-        o.cost[2] = __uint_as_float(c0.z);
-        o.cost[3] = __uint_as_float(c0.w);
-        o.cost[4] = __uint_as_float(c1.x);
-        o.cost[5] = __uint_as_float(c1.y);
-        o.cost[6] = __uint_as_float(c1.z);
-        o.nprims = c1.w;
-        const uint32_t sub[7] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z};
-        const uint32_t cwsize = s1.w, cwdepth = kc.z;
-        const uint2 meta = make_uint2(m.x, m.y), subdepth = make_uint2(m.z, m.w);
-        const bool internal = dkind(dbyte(meta, 0u)) == KIND_INTERNAL;
-        const uint32_t size0 = internal ? (cwsize == 0u ? SUB_INVALID : cwsize) : 0u, depth0 = internal ? cwdepth : 0u;
+    for (int k = 0; k < 7; ++k) r.w[k] = e[k];
+    return r;
+}
+
+// The child's costs and contributions through each decision d: its own CWBVH subtree (size and depth) when it becomes
+// a CWBVH child, those of its distributed descendants when it is DISTRIBUTE, nothing when it is a leaf child.
+// SUB_INVALID marks a subtree that cannot be built.  raw: the child's record (any record for a leaf).
+__device__ __forceinline__ ChildDp child_dp(const Node32& c, const DpRaw& raw) {
+    ChildDp o;
+    const bool leaf = c.prim_count != 0u;
+    const float leaf_cost = half_area(node_box(c)) * (float)c.prim_count * PRIM_COST;
+    const uint4 c0 = raw.w[0], c1 = raw.w[1], s0 = raw.w[2], s1 = raw.w[3], m = raw.w[4], kc = raw.w[5], pl = raw.w[6];
+    const uint32_t cost[7] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z}, sub[7] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z};
+    const uint32_t cwsize = s1.w, cwdepth = kc.z;
+    const uint2 meta = leaf ? make_uint2(0u, 0u) : make_uint2(m.x, m.y);  // a leaf's decisions are all LEAF
+    const uint2 subdepth = make_uint2(m.z, m.w);
+    const bool internal = dkind(dbyte(meta, 0u)) == KIND_INTERNAL;
+    const uint32_t size0 = internal ? (cwsize == 0u ? SUB_INVALID : cwsize) : 0u, depth0 = internal ? cwdepth : 0u;
 #pragma unroll
-        for (uint32_t d = 0; d < 7u; ++d) {
-            const bool dist = dkind(dbyte(meta, d)) == KIND_DISTRIBUTE;
-            o.size[d] = dist ? sub[d] : size0;
-            o.depth[d] = dist ? dbyte(subdepth, d) : depth0;
-        }
+    for (uint32_t d = 0; d < 7u; ++d) {
+        const bool dist = dkind(dbyte(meta, d)) == KIND_DISTRIBUTE;
+        o.cost[d] = leaf ? leaf_cost : __uint_as_float(cost[d]);
+        o.size[d] = dist ? sub[d] : size0;
+        o.depth[d] = dist ? dbyte(subdepth, d) : depth0;
     }
+    o.nprims = leaf ? c.prim_count : c1.w;
+    o.plist = leaf ? make_uint4(c.first_index, 0u, 0u, 1u) : pl;
+    return o;
 }
 
 // Evaluates the entry of the internal node with box `box` whose children records are `l` and `r` (slots first,
 // first + 1) and stores it under its key.  Returns a DERR_* bit or 0.
-// The sizes and depths below the chosen pair of decisions are carried along with its cost, so the evaluation is one
-// round of loads, arithmetic and one round of stores.  (Reading the chosen pair's sizes from the records afterwards
-// took up to 14 loads one after the other, each behind its own branch: 9.7K of the 16.8K cycles of a pass of
-// k_ploc_tail, where the entries wait on nothing else.)
+// One round of loads (both records at once, whatever the children are), selects without branches that carry the
+// sizes and depths below the best pair of decisions along with its cost, one round of stores.  Where entries wait on
+// each other the evaluation is a latency: in k_ploc_tail it took 9.7K cycles when the chosen pair's sizes were read
+// from the records afterwards (up to 14 loads one after the other), 7.5K with the records loaded one after the other
+// and a branch per candidate pair (1.29M-triangle build: the tail 215 -> 182 us, the grid passes' compactions 376 ->
+// 338 us, the refit's table 792 -> 630 us).
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                 const Node32& r) {
-    if ((l.prim_count != 0u && l.prim_count != 1u) || (r.prim_count != 0u && r.prim_count != 1u))
-        return DERR_CW_NONUNIT_LEAF;  // bvh2_to_cwbvh.rs:243-247
-    ChildDp L, R;
-    load_child_dp(dp, l, L);
-    load_child_dp(dp, r, R);
+    DpRec* const rec = &dp.rec[dp_key(dp, first)];
+    const bool ll = l.prim_count != 0u, rl = r.prim_count != 0u;
+    // a leaf has no record: the table's first is read in its place (a line every lane shares) and not used
+    const DpRaw raw_l = load_dp_raw(&dp.rec[ll ? (size_t)dp.kbase : dp_key(dp, l.first_index)]);
+    const DpRaw raw_r = load_dp_raw(&dp.rec[rl ? (size_t)dp.kbase : dp_key(dp, r.first_index)]);
+    const ChildDp L = child_dp(l, raw_l), R = child_dp(r, raw_r);
     const uint32_t num_primitives = L.nprims + R.nprims;
     const float ha = half_area(box);
+    const float cost_leaf = num_primitives <= dp.max_prims ? ((float)num_primitives) * ha * PRIM_COST : INFINITY;
+    // aux: the pair's decision byte without its kind (dpack's distribute indices) and its depth from bit 8 up
     float cost[7];
     uint32_t meta[7], sub[7], sd[7];
-    {
-        const float cost_leaf =
-            num_primitives <= dp.max_prims ? ((float)num_primitives) * ha * PRIM_COST : INFINITY;
-        float cost_distribute = INFINITY;
-        uint32_t dl = DIDX_INVALID, dr = DIDX_INVALID;
-        sub[0] = SUB_INVALID;
-        sd[0] = 0u;
+    auto pick = [&](int last, float& best, uint32_t& size, uint32_t& aux) {  // pairs (k, last - k), first strict minimum
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            const float c = L.cost[k] + R.cost[6 - k];
-            const uint32_t size = __builtin_elementwise_add_sat(L.size[k], R.size[6 - k]);  // SUB_INVALID stays
-            const uint32_t depth = max(L.depth[k], R.depth[6 - k]);
-            if (c < cost_distribute) {
-                cost_distribute = c;
-                dl = (uint32_t)k;
-                dr = (uint32_t)(6 - k);
-                sub[0] = size;
-                sd[0] = depth;
-            }
+        for (int k = 0; k <= last; ++k) {
+            const float c = L.cost[k] + R.cost[last - k];
+            const uint32_t s = __builtin_elementwise_add_sat(L.size[k], R.size[last - k]);  // SUB_INVALID stays
+            const uint32_t a = dpack(0u, (uint32_t)k, (uint32_t)(last - k)) | max(L.depth[k], R.depth[last - k]) << 8;
+            const bool lower = c < best;
+            best = lower ? c : best;
+            size = lower ? s : size;
+            aux = lower ? a : aux;
         }
-        const float cost_internal = cost_distribute + ha;
-        if (cost_leaf < cost_internal) {
-            cost[0] = cost_leaf;
-            meta[0] = dpack(KIND_LEAF, dl, dr);
-        } else {
-            cost[0] = cost_internal;
-            meta[0] = dpack(KIND_INTERNAL, dl, dr);
-        }
-    }
+    };
+    constexpr uint32_t NONE = (DIDX_INVALID << 2) | (DIDX_INVALID << 5);  // no pair has a finite cost; depth 0
+    float best = INFINITY;
+    uint32_t size = SUB_INVALID, aux = NONE;
+    pick(6, best, size, aux);
+    const float cost_internal = best + ha;
+    cost[0] = cost_leaf < cost_internal ? cost_leaf : cost_internal;
+    meta[0] = (aux & 0xffu) | (cost_leaf < cost_internal ? KIND_LEAF : KIND_INTERNAL);
+    sub[0] = size;
+    sd[0] = aux >> 8;
 #pragma unroll
     for (int i = 1; i < 7; ++i) {
-        float cost_distribute = cost[i - 1];
-        uint32_t dl = DIDX_INVALID, dr = DIDX_INVALID;
-        sub[i] = sub[i - 1];
-        sd[i] = sd[i - 1];
-#pragma unroll
-        for (int k = 0; k < i; ++k) {
-            const float c = L.cost[k] + R.cost[i - k - 1];
-            const uint32_t size = __builtin_elementwise_add_sat(L.size[k], R.size[i - k - 1]);
-            const uint32_t depth = max(L.depth[k], R.depth[i - k - 1]);
-            if (c < cost_distribute) {
-                cost_distribute = c;
-                dl = (uint32_t)k;
-                dr = (uint32_t)(i - k - 1);
-                sub[i] = size;
-                sd[i] = depth;
-            }
-        }
-        if (dl != DIDX_INVALID) {
-            cost[i] = cost_distribute;
-            meta[i] = dpack(KIND_DISTRIBUTE, dl, dr);
-        } else {
-            cost[i] = cost[i - 1];
-            meta[i] = meta[i - 1];
-        }
+        best = cost[i - 1];
+        size = sub[i - 1];
+        aux = NONE;
+        pick(i - 1, best, size, aux);
+        const bool found = (aux & 0xffu) != NONE;  // a pair's indices are below 7
+        cost[i] = best;
+        meta[i] = found ? ((aux & 0xffu) | KIND_DISTRIBUTE) : meta[i - 1];
+        sub[i] = size;
+        sd[i] = found ? aux >> 8 : sd[i - 1];
     }
 #pragma unroll
     for (int i = 0; i < 7; ++i) sd[i] = min(255u, sd[i]);
     // The leaves count_primitives (bvh2_to_cwbvh.rs:197-211) visits, left subtree first.  Each child holds at least
     // one leaf, so the left list has one or two entries.
-    uint4 pl = make_uint4(0u, 0u, 0u, 0u);
-    if (num_primitives <= 3u)
-        pl = L.plist.w >= 2u ? make_uint4(L.plist.x, L.plist.y, R.plist.x, num_primitives)
-                             : make_uint4(L.plist.x, R.plist.x, R.plist.y, num_primitives);
+    const bool two = L.plist.w >= 2u, few = num_primitives <= 3u;
+    const uint4 pl = make_uint4(few ? L.plist.x : 0u, few ? (two ? L.plist.y : R.plist.x) : 0u,
+                                few ? (two ? R.plist.x : R.plist.y) : 0u, few ? num_primitives : 0u);
     // The whole 128-byte entry in eight 16-byte stores (the padding too, so that no 32-byte sector of the line is
     // left partly written).
-    uint4* e = reinterpret_cast<uint4*>(&dp.rec[dp_key(dp, first)]);
+    uint4* e = reinterpret_cast<uint4*>(rec);
     e[0] = make_uint4(__float_as_uint(cost[0]), __float_as_uint(cost[1]), __float_as_uint(cost[2]),
                       __float_as_uint(cost[3]));
     e[1] = make_uint4(__float_as_uint(cost[4]), __float_as_uint(cost[5]), __float_as_uint(cost[6]), num_primitives);
@@ -230,11 +207,11 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     e[3] = make_uint4(sub[4], sub[5], sub[6], sub[0] == SUB_INVALID ? 0u : 1u + sub[0]);
     e[4] = make_uint4(meta[0] | meta[1] << 8 | meta[2] << 16 | meta[3] << 24, meta[4] | meta[5] << 8 | meta[6] << 16,
                       sd[0] | sd[1] << 8 | sd[2] << 16 | sd[3] << 24, sd[4] | sd[5] << 8 | sd[6] << 16);
-    e[5] = make_uint4(l.first_index | (L.leaf ? KID_LEAF : 0u), r.first_index | (R.leaf ? KID_LEAF : 0u), 1u + sd[0],
-                      0u);
+    e[5] = make_uint4(l.first_index | (ll ? KID_LEAF : 0u), r.first_index | (rl ? KID_LEAF : 0u), 1u + sd[0], 0u);
     e[6] = pl;
     e[7] = make_uint4(0u, 0u, 0u, 0u);
-    return 0u;
+    // checked last, so that the records' loads do not wait for the leaf counts (bvh2_to_cwbvh.rs:243-247)
+    return l.prim_count > 1u || r.prim_count > 1u ? DERR_CW_NONUNIT_LEAF : 0u;
 }
 
 }  // namespace obvhs
