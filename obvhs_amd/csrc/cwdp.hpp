@@ -88,6 +88,12 @@ __device__ __forceinline__ uint32_t dleft(uint32_t b) { return (b >> 2) & 7u; }
 __device__ __forceinline__ uint32_t dright(uint32_t b) { return (b >> 5) & 7u; }
 __device__ __forceinline__ uint32_t dpack(uint32_t k, uint32_t l, uint32_t r) { return k | (l << 2) | (r << 5); }
 
+// What the evaluation reads of a child's node.
+struct DpChild {
+    uint32_t first_index, prim_count;
+    float area;  // half area of its box
+};
+
 // Everything the parent's evaluation needs from one child, in registers.
 struct ChildDp {
     float cost[7];
@@ -112,10 +118,10 @@ __device__ __forceinline__ DpRaw load_dp_raw(const DpRec* rec) {
 // The child's costs and contributions through each decision d: its own CWBVH subtree (size and depth) when it becomes
 // a CWBVH child, those of its distributed descendants when it is DISTRIBUTE, nothing when it is a leaf child.
 // SUB_INVALID marks a subtree that cannot be built.  raw: the child's record (any record for a leaf).
-__device__ __forceinline__ ChildDp child_dp(const Node32& c, const DpRaw& raw) {
+__device__ __forceinline__ ChildDp child_dp(const DpChild& c, const DpRaw& raw) {
     ChildDp o;
     const bool leaf = c.prim_count != 0u;
-    const float leaf_cost = half_area(node_box(c)) * (float)c.prim_count * PRIM_COST;
+    const float leaf_cost = c.area * (float)c.prim_count * PRIM_COST;
     const uint4 c0 = raw.w[0], c1 = raw.w[1], s0 = raw.w[2], s1 = raw.w[3], m = raw.w[4], kc = raw.w[5], pl = raw.w[6];
     const uint32_t cost[7] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z}, sub[7] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z};
     const uint32_t cwsize = s1.w, cwdepth = kc.z;
@@ -135,16 +141,16 @@ __device__ __forceinline__ ChildDp child_dp(const Node32& c, const DpRaw& raw) {
     return o;
 }
 
-// Evaluates the entry of the internal node with box `box` whose children records are `l` and `r` (slots first,
-// first + 1) and stores it under its key.  Returns a DERR_* bit or 0.
+// Evaluates the entry of the internal node of half area `ha` whose children are `l` and `r` (slots first, first + 1)
+// and stores it under its key.  Returns a DERR_* bit or 0.
 // One round of loads (both records at once, whatever the children are), selects without branches that carry the
 // sizes and depths below the best pair of decisions along with its cost, one round of stores.  Where entries wait on
 // each other the evaluation is a latency: in k_ploc_tail it took 9.7K cycles when the chosen pair's sizes were read
 // from the records afterwards (up to 14 loads one after the other), 7.5K with the records loaded one after the other
 // and a branch per candidate pair (1.29M-triangle build: the tail 215 -> 182 us, the grid passes' compactions 376 ->
 // 338 us, the refit's table 792 -> 630 us).
-__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
-                                                const Node32& r) {
+__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
+                                                const DpChild& r) {
     DpRec* const rec = &dp.rec[dp_key(dp, first)];
     const bool ll = l.prim_count != 0u, rl = r.prim_count != 0u;
     // a leaf has no record: the table's first is read in its place (a line every lane shares) and not used
@@ -152,7 +158,6 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     const DpRaw raw_r = load_dp_raw(&dp.rec[rl ? (size_t)dp.kbase : dp_key(dp, r.first_index)]);
     const ChildDp L = child_dp(l, raw_l), R = child_dp(r, raw_r);
     const uint32_t num_primitives = L.nprims + R.nprims;
-    const float ha = half_area(box);
     const float cost_leaf = num_primitives <= dp.max_prims ? ((float)num_primitives) * ha * PRIM_COST : INFINITY;
     // aux: the pair's decision byte without its kind (dpack's distribute indices) and its depth from bit 8 up
     float cost[7];
@@ -212,6 +217,13 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
     e[7] = make_uint4(0u, 0u, 0u, 0u);
     // checked last, so that the records' loads do not wait for the leaf counts (bvh2_to_cwbvh.rs:243-247)
     return l.prim_count > 1u || r.prim_count > 1u ? DERR_CW_NONUNIT_LEAF : 0u;
+}
+
+// The same for a node with box `box` and children `l` and `r`.
+__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
+                                                const Node32& r) {
+    return dp_evaluate(dp, half_area(box), first, DpChild{l.first_index, l.prim_count, half_area(node_box(l))},
+                       DpChild{r.first_index, r.prim_count, half_area(node_box(r))});
 }
 
 }  // namespace obvhs
