@@ -113,6 +113,7 @@ obvhs_status obvhs_context_destroy(obvhs_context* ctx) {
     S.tops.release();
     S.vals.release();
     S.merge.release();
+    S.pass_tiles.release();
     S.blocksums.release();
     S.sort_scratch.release();
     S.misc.release();

@@ -142,7 +142,7 @@ __device__ __forceinline__ ChildDp child_dp(const DpChild& c, const DpRaw& raw) 
 }
 
 // Evaluates the entry of the internal node of half area `ha` whose children are `l` and `r` (slots first, first + 1)
-// and stores it under its key.  Returns a DERR_* bit or 0.
+// and stores it under its key; raw_l and raw_r are the children's records (dp_child_record).  Returns a DERR_* bit or 0.
 // One round of loads (both records at once, whatever the children are), selects without branches that carry the
 // sizes and depths below the best pair of decisions along with its cost, one round of stores.  Where entries wait on
 // each other the evaluation is a latency: in k_ploc_tail it took 9.7K cycles when the chosen pair's sizes were read
@@ -150,12 +150,9 @@ __device__ __forceinline__ ChildDp child_dp(const DpChild& c, const DpRaw& raw) 
 // and a branch per candidate pair (1.29M-triangle build: the tail 215 -> 182 us, the grid passes' compactions 376 ->
 // 338 us, the refit's table 792 -> 630 us).
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
-                                                const DpChild& r) {
+                                                const DpChild& r, const DpRaw& raw_l, const DpRaw& raw_r) {
     DpRec* const rec = &dp.rec[dp_key(dp, first)];
     const bool ll = l.prim_count != 0u, rl = r.prim_count != 0u;
-    // a leaf has no record: the table's first is read in its place (a line every lane shares) and not used
-    const DpRaw raw_l = load_dp_raw(&dp.rec[ll ? (size_t)dp.kbase : dp_key(dp, l.first_index)]);
-    const DpRaw raw_r = load_dp_raw(&dp.rec[rl ? (size_t)dp.kbase : dp_key(dp, r.first_index)]);
     const ChildDp L = child_dp(l, raw_l), R = child_dp(r, raw_r);
     const uint32_t num_primitives = L.nprims + R.nprims;
     const float cost_leaf = num_primitives <= dp.max_prims ? ((float)num_primitives) * ha * PRIM_COST : INFINITY;
@@ -219,11 +216,28 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint
     return l.prim_count > 1u || r.prim_count > 1u ? DERR_CW_NONUNIT_LEAF : 0u;
 }
 
+// The record to load for a child.  A leaf has none: the table's first is read in its place (a line every lane shares)
+// and not used.
+__device__ __forceinline__ const DpRec* dp_child_record(const DpView& dp, const DpChild& c) {
+    return &dp.rec[c.prim_count != 0u ? (size_t)dp.kbase : dp_key(dp, c.first_index)];
+}
+__device__ __forceinline__ const DpRec* dp_child_record(const DpView& dp, const Node32& c) {
+    return &dp.rec[c.prim_count != 0u ? (size_t)dp.kbase : dp_key(dp, c.first_index)];
+}
+__device__ __forceinline__ DpChild dp_child(const Node32& c) {
+    return DpChild{c.first_index, c.prim_count, half_area(node_box(c))};
+}
+
+__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
+                                                const DpChild& r) {
+    const DpRaw raw_l = load_dp_raw(dp_child_record(dp, l)), raw_r = load_dp_raw(dp_child_record(dp, r));
+    return dp_evaluate(dp, ha, first, l, r, raw_l, raw_r);
+}
+
 // The same for a node with box `box` and children `l` and `r`.
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                 const Node32& r) {
-    return dp_evaluate(dp, half_area(box), first, DpChild{l.first_index, l.prim_count, half_area(node_box(l))},
-                       DpChild{r.first_index, r.prim_count, half_area(node_box(r))});
+    return dp_evaluate(dp, half_area(box), first, dp_child(l), dp_child(r));
 }
 
 }  // namespace obvhs

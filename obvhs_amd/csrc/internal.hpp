@@ -46,6 +46,7 @@ struct BuildScratch {
     DevBuf vals;        // u32[n]
     DevBuf merge;       // i8[n]
     DevBuf blocksums;   // uint2[n/256+1]
+    DevBuf pass_tiles;  // tile counts and merge lists of the one-launch PLOC passes
     DevBuf sort_scratch;
     DevBuf misc;        // bounds keys, states, error word
     DevBuf cw_scratch;  // conversion working memory: item lists

@@ -541,6 +541,13 @@ __global__ void __launch_bounds__(SMALL_THREADS)
     }
 }
 
+// A workgroup barrier for data in LDS only: global loads and stores in flight are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Classification of cluster i (ploc/mod.rs:423-439): `emit` when it goes to the next pass (kept, or the higher
 // index of a mutual pair, which becomes the parent), `mrg` when it is the higher index of a mutual pair.
 // A self-pair (no finite neighbour, already flagged as an error) is treated as kept so that no slot underflows.
@@ -865,6 +872,10 @@ __global__ void __launch_bounds__(1024) k_ploc_scan_apply(uint2* __restrict__ bl
     }
 }
 
+// Merges of a tile: a merge is counted at its higher cluster; pairs inside the tile use two of its clusters, and at most
+// r of its clusters pair with distinct clusters in [base - r, base): at most 128 + r / 2.
+constexpr uint32_t MAX_TILE_MERGES = (T256 + MAX_RADIUS) / 2;
+
 // Compaction of one 256-cluster tile (ploc/mod.rs:420-493): kept clusters and the parents of mutual pairs go to
 // `next` in order; a merge's two children go to the slots below the pass's insert index in the serial loop's order
 // (`pe0` / `pm0`: the emits and merges of the tiles before this one).  The tile's merges are then
@@ -880,9 +891,6 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
                                              const DpView& dp, uint32_t fused, const uint32_t* __restrict__ slot_map,
                                              uint32_t vtop, uint32_t map_len, uint32_t* __restrict__ err,
                                              uint32_t* we, uint32_t* wm) {
-    // A merge is counted at its higher cluster; pairs inside the tile use two of its clusters, and at most r of its
-    // clusters pair with distinct clusters in [base - r, base): at most 128 + r / 2 merges.
-    constexpr uint32_t MAX_TILE_MERGES = (T256 + MAX_RADIUS) / 2;
     __shared__ Node32 s_left[MAX_TILE_MERGES], s_right[MAX_TILE_MERGES];
     __shared__ uint32_t s_first[MAX_TILE_MERGES];
     const uint64_t be = __ballot(emit), bm = __ballot(mrg);
@@ -949,76 +957,322 @@ __global__ void __launch_bounds__(T256) k_ploc_compact(const Node32* __restrict_
                  &misc->err, we, wm);
 }
 
-// k_ploc_scan and k_ploc_compact in one launch for passes of at most SCAN_FUSED_BLOCKS tiles: each workgroup sums the
-// (emit, merge) counts of the tiles before its own (at most 4 per thread), and workgroup 0 also sums them all and
-// writes the next pass's state, as k_ploc_scan does.
-constexpr uint32_t SCAN_FUSED_BLOCKS = 1024;
-__global__ void __launch_bounds__(T256) k_ploc_scan_compact(const Node32* __restrict__ cur, Node32* __restrict__ next,
-                                                            const int8_t* __restrict__ merge, Misc* misc,
-                                                            uint32_t slot, const uint2* __restrict__ blocksums,
-                                                            uint32_t nblocks, Node32* __restrict__ bvh_nodes, DpView dp,
-                                                            uint32_t fused, const uint32_t* __restrict__ slot_map,
-                                                            uint32_t vtop, uint32_t map_len,
-                                                            uint32_t* __restrict__ hist) {
-    __shared__ uint32_t we[T256 / 64], wm[T256 / 64];
-    __shared__ uint2 pre;
-    const PlocState st = misc->state[slot];
-    const uint32_t i = blockIdx.x * T256 + threadIdx.x;
-    Node32 a{};
-    if (i < st.count) a = load_node(&cur[i]);
-    bool emit, mrg;
-    uint32_t b;
-    classify(merge, i, st.count, emit, mrg, b);
-    const uint32_t upto = blockIdx.x == 0 ? nblocks : blockIdx.x;  // workgroup 0 sums every tile (the totals)
-    uint32_t E = 0, M = 0;
-    for (uint32_t t = threadIdx.x; t < upto; t += T256) {
-        const uint2 v = blocksums[t];
-        E += v.x;
-        M += v.y;
+// ---- passes of at most PASS_TILES tiles: one launch per pass ----
+// A pass's compaction needs the emits and merges of every tile before a cluster's (a scan over the tiles), so it is a
+// launch behind the search.  Here it is left to the next pass's launch: a tile leaves its emitted clusters at the front
+// of its own 256 slots (with its counts) and its merges in a list, and the next launch starts with the scan of the
+// counts (every workgroup scans them all, at most 1,024), finds its own 256 clusters and their window by it, and, with
+// other waves than those that search, gives the listed merges of tile blockIdx.x their slots, writes their children
+// and evaluates their cost-table entries.  A parent emitted by the pass before carries MERGE_RANK and its merge's rank
+// in its tile in the place of its first_index until then.  k_ploc_flush ends a run of such passes: dense clusters, the
+// last merges, the state.  The loads of a merge's entry are issued a barrier ahead of their use, so they run under the
+// search.  Latency bounds these passes (2.5 us of each launch are the launch): 1.29M-triangle build, 675 tiles down
+// to 26: 11.6 -> 9.0 us a pass (65,536 triangles, 256 tiles down to 9: 11.4 -> 7.8).
+constexpr uint32_t PASS_TILES = 1024;
+constexpr int PASS_THREADS = 512;
+constexpr uint32_t MERGE_RANK = 0x80000000u;                       // prim_count of such a parent
+constexpr uint32_t PASS_MERGE_THREAD0 = (uint32_t)SC_THREADS;      // threads from here on take a merge each
+static_assert(PASS_THREADS - (int)PASS_MERGE_THREAD0 >= (int)MAX_TILE_MERGES, "a thread per merge");
+
+struct PassMerge {
+    Node32 left, right;
+};
+
+// The tiles' counts before a pass, scanned: for tile t the clusters and merges of the tiles before it.
+struct PassScan {
+    uint32_t emits[PASS_TILES + 1], merges[PASS_TILES + 1];
+    uint32_t wave_e[PASS_THREADS / 64], wave_m[PASS_THREADS / 64];
+};
+
+// Fills ps for ntiles counts; ends with a barrier.  Every thread calls.
+__device__ __forceinline__ void pass_scan(const uint2* __restrict__ counts, uint32_t ntiles, PassScan& ps) {
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, t = 2u * tid;
+    const uint2 c0 = t < ntiles ? counts[t] : make_uint2(0u, 0u);
+    const uint2 c1 = t + 1u < ntiles ? counts[t + 1u] : make_uint2(0u, 0u);
+    const uint32_t ie = wave_inclusive_scan_dpp(c0.x + c1.x), im = wave_inclusive_scan_dpp(c0.y + c1.y);
+    if ((tid & 63u) == 63u) {
+        ps.wave_e[wave] = ie;
+        ps.wave_m[wave] = im;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        E += (uint32_t)__shfl_xor((int)E, off);
-        M += (uint32_t)__shfl_xor((int)M, off);
+    lds_barrier();
+    uint32_t e = ie - (c0.x + c1.x), m = im - (c0.y + c1.y);
+#pragma unroll
+    for (uint32_t w = 0; w < PASS_THREADS / 64; ++w) {
+        e += w < wave ? ps.wave_e[w] : 0u;
+        m += w < wave ? ps.wave_m[w] : 0u;
     }
-    const uint32_t wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63u) == 0) {
-        we[wave] = E;
-        wm[wave] = M;
+    ps.emits[t] = e;
+    ps.merges[t] = m;
+    ps.emits[t + 1u] = e + c0.x;
+    ps.merges[t + 1u] = m + c0.y;
+    if (tid == (uint32_t)PASS_THREADS - 1u) {
+        ps.emits[t + 2u] = e + c0.x + c1.x;
+        ps.merges[t + 2u] = m + c0.y + c1.y;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t te = 0, tm = 0;
-        for (int w = 0; w < T256 / 64; ++w) {
-            te += we[w];
-            tm += wm[w];
-        }
-        if (blockIdx.x == 0) {
-            PlocState nx = st;
-            if (st.count > 1) {
-                nx.count = te;
-                nx.insert = st.insert - 2u * tm;
-                nx.depth = st.depth + 1u;
-                nx.cluster_sum = st.cluster_sum + st.count;
-                hist[nx.depth] = nx.insert;
-            }
-            misc->state[slot ^ 1u] = nx;
-            pre = make_uint2(0u, 0u);
-        } else {
-            pre = make_uint2(te, tm);
-        }
-    }
-    __syncthreads();
-    const uint2 off = pre;
-    __syncthreads();  // compact_tile reuses we / wm
-    compact_tile(cur, next, a, emit, mrg, b, st, off.x, off.y, bvh_nodes, dp, fused, slot_map, vtop, map_len,
-                 &misc->err, we, wm);
+    lds_barrier();
 }
 
-// A workgroup barrier for data in LDS only: global stores in flight are not waited for.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+// The state after the pass that state `st` was before.
+__device__ __forceinline__ PlocState pass_next(const PlocState& st, const PassScan& ps) {
+    PlocState nx = st;
+    if (st.count > 1u) {
+        nx.count = ps.emits[PASS_TILES];
+        nx.insert = st.insert - 2u * ps.merges[PASS_TILES];
+        nx.depth = st.depth + 1u;
+        nx.cluster_sum = st.cluster_sum + st.count;
+    }
+    return nx;
+}
+
+// A cluster of tile t as the pass before left it: a parent's rank becomes its first child slot.
+__device__ __forceinline__ Node32 pass_cluster(Node32 c, uint32_t merges_before, const PlocState& st,
+                                               const uint32_t* __restrict__ slot_map, uint32_t vtop, uint32_t map_len) {
+    if (c.prim_count == MERGE_RANK) {
+        uint32_t first = 0u;
+        (void)child_slot(st.insert - 2u * (merges_before + c.first_index + 1u), slot_map, vtop, map_len, first);
+        c.prim_count = 0u;
+        c.first_index = first;
+    }
+    return c;
+}
+
+// One pass over the clusters in `cur`: dense (`ntiles` = 0) or as a pass left them in ntiles tiles with `counts`
+// and `merges_in`; the result goes to next, counts_out and merges_out, a tile per workgroup.
+template <int R>
+__global__ void __launch_bounds__(PASS_THREADS)
+    k_ploc_pass(const Node32* __restrict__ cur, Node32* __restrict__ next, const uint2* __restrict__ counts,
+                uint32_t ntiles, uint2* __restrict__ counts_out, const PassMerge* __restrict__ merges_in,
+                PassMerge* __restrict__ merges_out, Misc* misc, uint32_t slot, uint32_t r, uint32_t dist1,
+                Node32* __restrict__ bvh_nodes, DpView dp, uint32_t fused, const uint32_t* __restrict__ slot_map,
+                uint32_t vtop, uint32_t map_len, uint32_t* __restrict__ hist) {
+    __shared__ PassScan ps;
+    __shared__ float s[6][SC_WINDOW];
+    __shared__ uint32_t w_pc[SC_WINDOW], w_fi[SC_WINDOW];  // of clusters from base - r on
+    __shared__ int8_t mm[T256 + 2 * MAX_RADIUS];  // offsets of clusters [base - r, base + 256 + r)
+    __shared__ float pcost[R > 0 ? R : 1][SC_WINDOW];
+    __shared__ uint32_t we[T256 / 64], wm[T256 / 64], w_nan[PASS_THREADS / 64], s_tile0;
+    const uint32_t t = threadIdx.x, base = blockIdx.x * T256;
+    const PlocState st = misc->state[slot];
+    const bool dense = ntiles == 0u;
+    PlocState nx = st;
+    const int wstart = (int)base - 2 * (int)r, wlen = T256 + 4 * (int)r;
+    if (!dense) {
+        pass_scan(counts, ntiles, ps);
+        nx = pass_next(st, ps);
+    }
+    if (blockIdx.x == 0 && t == 0) {
+        misc->state[slot ^ 1u] = nx;
+        if (!dense && st.count > 1u) hist[nx.depth] = nx.insert;
+    }
+    const uint32_t count = nx.count;
+    const bool search = count > 1u && base < count;  // workgroup-uniform
+    // the merges of tile blockIdx.x of the pass before: their nodes are loaded now
+    const uint32_t mj = t - PASS_MERGE_THREAD0;
+    const uint32_t my_merges = !dense && blockIdx.x < ntiles ? ps.merges[blockIdx.x + 1u] - ps.merges[blockIdx.x] : 0u;
+    const bool merging = t >= PASS_MERGE_THREAD0 && mj < my_merges;
+    Node32 ml{}, mr{};
+    if (merging) {
+        const PassMerge* pm = &merges_in[(size_t)blockIdx.x * MAX_TILE_MERGES + mj];
+        ml = load_node(&pm->left);
+        mr = load_node(&pm->right);
+    }
+    if (!search) {  // beyond the clusters, or a lone cluster, which goes through
+        if (t == 0) {
+            const bool lone = count == 1u && blockIdx.x == 0;
+            if (lone) {
+                uint32_t tile = 0u;
+                if (!dense)
+                    while (ps.emits[tile + 1u] == 0u) ++tile;
+                store_node(&next[0], pass_cluster(load_node(&cur[(size_t)tile * T256]), dense ? 0u : ps.merges[tile], st,
+                                                  slot_map, vtop, map_len));
+            }
+            counts_out[blockIdx.x] = make_uint2(lone ? 1u : 0u, 0u);
+        }
+        if (my_merges == 0u) return;
+    }
+    bool nan_here = false;
+    if (search) {
+        auto put = [&](int w, const Node32& nd) {
+            s[0][w] = nd.minx;
+            s[1][w] = nd.miny;
+            s[2][w] = nd.minz;
+            s[3][w] = nd.maxx;
+            s[4][w] = nd.maxy;
+            s[5][w] = nd.maxz;
+            w_pc[w] = nd.prim_count;
+            w_fi[w] = nd.first_index;
+            nan_here |= box_has_nan_any(node_box(nd));
+        };
+        for (int w = (int)t; w < wlen; w += PASS_THREADS) {
+            const int g = wstart + w;
+            if (g >= 0 && (uint32_t)g < count) {
+                if (dense) put(w, load_node(&cur[g]));
+            } else if (R > 0) {
+#pragma unroll
+                for (int a = 0; a < 6; ++a) s[a][w] = __builtin_nanf("");
+            }
+        }
+        if (!dense) {
+            // the tile that holds the window's first cluster, then the tiles up to its last, two at a time
+            const uint32_t w0 = wstart > 0 ? (uint32_t)wstart : 0u, w1 = min(count, (uint32_t)(wstart + wlen));
+#pragma unroll
+            for (uint32_t k = 0; k < 2u; ++k) {
+                const uint32_t tile = 2u * t + k;
+                if (ps.emits[tile] <= w0 && ps.emits[tile + 1u] > w0) s_tile0 = tile;
+            }
+            lds_barrier();
+            for (uint32_t tile = s_tile0 + (t >> 8); tile < ntiles && ps.emits[tile] < w1; tile += PASS_THREADS / T256) {
+                const uint32_t first = ps.emits[tile], g = first + (t & 255u);
+                if (g < ps.emits[tile + 1u] && g >= w0 && g < w1)
+                    put((int)g - wstart, pass_cluster(load_node(&cur[(size_t)tile * T256 + (t & 255u)]),
+                                                      ps.merges[tile], st, slot_map, vtop, map_len));
+            }
+        }
+    }
+    // the merges' slots, children and table records
+    uint32_t mfirst = 0u;
+    DpRaw raw_l, raw_r;
+    if (merging) {
+        if (!child_slot(st.insert - 2u * (ps.merges[blockIdx.x] + mj + 1u), slot_map, vtop, map_len, mfirst)) {
+            atomicOr(&misc->err, DERR_CAPACITY);
+            mfirst = UINT32_MAX;
+        } else {
+            store_node(&bvh_nodes[mfirst], ml);
+            store_node(&bvh_nodes[mfirst + 1u], mr);
+            if (fused) {
+                raw_l = load_dp_raw(dp_child_record(dp, ml));
+                raw_r = load_dp_raw(dp_child_record(dp, mr));
+            }
+        }
+    }
+    if ((t & 63u) == 0u) w_nan[t >> 6] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    if (nan_here) w_nan[t >> 6] = 1u;
+    lds_barrier();
+    uint32_t any_nan = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < PASS_THREADS / 64; ++w) any_nan |= w_nan[w];
+    const bool nonan = any_nan == 0u;  // NaN-free window: costs from union_area_nonan
+    const bool pairs = R > 0 && !dist1 && nonan;  // workgroup-uniform
+    if constexpr (R > 0) {
+        if (search && pairs) {
+            if (t < PASS_MERGE_THREAD0)
+                for (int w = (int)t; w < T256 + 3 * R; w += SC_THREADS) pair_costs<R>(s, pcost, w);
+        }
+    }
+    if (search && pairs) lds_barrier();
+    // thread t < 256: cluster base + t; thread 256 + h, h < 2r: halo cluster base - r + h or base + 256 + h - r
+    int c = -1;
+    if (t < (uint32_t)T256) c = (int)(base + t);
+    else if (t - T256 < 2u * r) c = t - T256 < r ? (int)base - (int)r + (int)(t - T256) : (int)(base + t - r);
+    if (search && c >= 0 && (uint32_t)c < count) {
+        int8_t m = 0;
+        bool unrolled = false;
+        if constexpr (R > 0) {
+            if (!dist1) {
+                const int lc = c - wstart;
+                const int b = pairs ? pick_from_pairs<R>(pcost, lc)
+                                    : cluster_merge_unrolled<R, false>(s[0], s[1], s[2], s[3], s[4], s[5], lc);
+                if (b == 0) atomicOr(&misc->err, DERR_SELF_MERGE);
+                m = (int8_t)b;
+                unrolled = true;
+            }
+        }
+        if (!unrolled) m = cluster_merge(s, wstart, (uint32_t)c, count, r, dist1, nonan, &misc->err);
+        mm[c - ((int)base - (int)r)] = m;
+    }
+    if (fused && merging && mfirst != UINT32_MAX) {
+        const uint32_t e = dp_evaluate(dp, half_area(box_union(node_box(ml), node_box(mr))), mfirst,
+                                       dp_child(ml), dp_child(mr), raw_l, raw_r);
+        if (e) atomicOr(&misc->err, e);
+    }
+    lds_barrier();
+    // classify (ploc/mod.rs:423-439) the tile's clusters from the offsets in LDS
+    bool emit = false, mrg = false;
+    int partner = 0;
+    if (search && t < (uint32_t)T256 && base + t < count) {
+        const int i = (int)(base + t);
+        partner = i + (int)mm[i - ((int)base - (int)r)];
+        const bool mutual = partner + (int)mm[partner - ((int)base - (int)r)] == i;
+        emit = !mutual || partner <= i;
+        mrg = mutual && partner < i;
+    }
+    const uint64_t be = __ballot(emit), bm = __ballot(mrg);
+    const uint32_t wave = t >> 6;
+    if ((t & 63u) == 0 && wave < (uint32_t)(T256 / 64)) {
+        we[wave] = (uint32_t)__popcll(be);
+        wm[wave] = (uint32_t)__popcll(bm);
+    }
+    lds_barrier();
+    if (t == 0 && search) {
+        uint32_t E = 0, M = 0;
+        for (int w = 0; w < T256 / 64; ++w) {
+            E += we[w];
+            M += wm[w];
+        }
+        counts_out[blockIdx.x] = make_uint2(E, M);
+    }
+    if (!emit) return;
+    uint32_t pe = 0u, pm = 0u;
+    for (uint32_t w = 0; w < wave; ++w) {
+        pe += we[w];
+        pm += wm[w];
+    }
+    pe += (uint32_t)__popcll(be & lanemask_lt());
+    auto cluster = [&](int g) {
+        const int w = g - wstart;
+        return Node32{s[0][w], s[1][w], s[2][w], w_pc[w], s[3][w], s[4][w], s[5][w], w_fi[w]};
+    };
+    Node32 out = cluster((int)(base + t));
+    if (mrg) {
+        pm += (uint32_t)__popcll(bm & lanemask_lt());
+        if (pm < MAX_TILE_MERGES) {
+            const Node32 b = cluster(partner);
+            PassMerge* o = &merges_out[(size_t)blockIdx.x * MAX_TILE_MERGES + pm];
+            store_node(&o->left, out);
+            store_node(&o->right, b);
+            out = make_node(box_union(node_box(out), node_box(b)), MERGE_RANK, pm);
+        } else {
+            atomicOr(&misc->err, DERR_CAPACITY);
+        }
+    }
+    store_node(&next[(size_t)base + pe], out);
+}
+
+// The end of a run of k_ploc_pass launches: the clusters of the last one's tiles, dense, and its merges.
+__global__ void __launch_bounds__(PASS_THREADS)
+    k_ploc_flush(const Node32* __restrict__ cur, Node32* __restrict__ next, const uint2* __restrict__ counts,
+                 uint32_t ntiles, const PassMerge* __restrict__ merges_in, Misc* misc, uint32_t slot,
+                 Node32* __restrict__ bvh_nodes, DpView dp, uint32_t fused, const uint32_t* __restrict__ slot_map,
+                 uint32_t vtop, uint32_t map_len, uint32_t* __restrict__ hist) {
+    __shared__ PassScan ps;
+    const uint32_t t = threadIdx.x, tile = blockIdx.x;
+    const PlocState st = misc->state[slot];
+    pass_scan(counts, ntiles, ps);
+    const PlocState nx = pass_next(st, ps);
+    if (tile == 0 && t == 0) {
+        misc->state[slot ^ 1u] = nx;
+        if (st.count > 1u) hist[nx.depth] = nx.insert;
+    }
+    const uint32_t mb = ps.merges[tile], nm = ps.merges[tile + 1u] - mb;
+    if (t < T256 && ps.emits[tile] + t < ps.emits[tile + 1u])
+        store_node(&next[ps.emits[tile] + t],
+                   pass_cluster(load_node(&cur[(size_t)tile * T256 + t]), mb, st, slot_map, vtop, map_len));
+    const uint32_t mj = t - PASS_MERGE_THREAD0;
+    if (t < PASS_MERGE_THREAD0 || mj >= nm) return;
+    const PassMerge* pm = &merges_in[(size_t)tile * MAX_TILE_MERGES + mj];
+    const Node32 l = load_node(&pm->left), r = load_node(&pm->right);
+    uint32_t first;
+    if (!child_slot(st.insert - 2u * (mb + mj + 1u), slot_map, vtop, map_len, first)) {
+        atomicOr(&misc->err, DERR_CAPACITY);
+        return;
+    }
+    store_node(&bvh_nodes[first], l);
+    store_node(&bvh_nodes[first + 1u], r);
+    if (fused) {
+        const uint32_t e = dp_evaluate(dp, box_union(node_box(l), node_box(r)), first, l, r);
+        if (e) atomicOr(&misc->err, e);
+    }
 }
 
 // A cluster in the tail's LDS arrays: lo = box minimum and prim_count, hi = box maximum and first_index.
@@ -1540,6 +1794,32 @@ static void launch_tail(hipStream_t st, const Node32* cur, Misc* misc, uint32_t 
 #undef OBVHS_TAIL
 }
 
+// Working memory of the one-launch passes: two arrays of tile counts, two of merge lists (18.9 MB at most).
+static size_t pass_tile_bytes(uint32_t n) {
+    const size_t tiles = std::min<uint32_t>((n + T256 - 1) / T256, PASS_TILES);
+    return 2 * PASS_TILES * sizeof(uint2) + 2 * tiles * MAX_TILE_MERGES * sizeof(PassMerge);
+}
+
+// The one-launch pass for the search distance (each allowed distance has its unrolled instance).
+static void launch_pass(uint32_t blocks, hipStream_t st, const Node32* cur, Node32* next, const uint2* counts,
+                        uint32_t ntiles, uint2* counts_out, const PassMerge* merges_in, PassMerge* merges_out,
+                        Misc* misc, uint32_t slot, uint32_t r, uint32_t dist1, Node32* bvh_nodes, const DpView& dp,
+                        uint32_t fused, const uint32_t* slot_map, uint32_t vtop, uint32_t map_len, uint32_t* hist) {
+#define OBVHS_PASS(RR)                                                                                              \
+    k_ploc_pass<RR><<<blocks, PASS_THREADS, 0, st>>>(cur, next, counts, ntiles, counts_out, merges_in, merges_out, \
+                                                     misc, slot, r, dist1, bvh_nodes, dp, fused, slot_map, vtop,    \
+                                                     map_len, hist)
+    switch (r) {
+        case 2: OBVHS_PASS(2); break;
+        case 6: OBVHS_PASS(6); break;
+        case 14: OBVHS_PASS(14); break;
+        case 24: OBVHS_PASS(24); break;
+        case 32: OBVHS_PASS(32); break;
+        default: OBVHS_PASS(0); break;
+    }
+#undef OBVHS_PASS
+}
+
 static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uint32_t n, uint32_t r,
                                uint32_t search_depth_threshold, Node32* bvh_nodes, uint32_t* hist, DpView dp,
                                uint32_t fused, const uint32_t* slot_map, uint32_t vtop, uint32_t map_len,
@@ -1550,19 +1830,37 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
     Misc* misc = S.misc.as<Misc>();
     int8_t* merge = S.merge.as<int8_t>();
     uint2* blocksums = S.blocksums.as<uint2>();
+    const uint32_t tiles = std::min<uint32_t>((n + T256 - 1) / T256, PASS_TILES);
+    uint2* pass_counts[2] = {S.pass_tiles.as<uint2>(), S.pass_tiles.as<uint2>() + PASS_TILES};
+    PassMerge* pass_merges[2];
+    pass_merges[0] = reinterpret_cast<PassMerge*>(pass_counts[1] + PASS_TILES);
+    pass_merges[1] = pass_merges[0] + (size_t)tiles * MAX_TILE_MERGES;
     uint32_t known = n;
     uint32_t pass = 0;
     uint32_t slot = 0;
     PlocState hstate{};
     while (known > TAIL_MAX) {
         const uint32_t blocks = (known + T256 - 1) / T256;
-        for (int k = 0; k < PASSES_PER_SYNC; ++k) {
-            const uint32_t dist1 = (r == 1 || pass < search_depth_threshold) ? 1u : 0u;
-            launch_search_count(blocks, st, cur, misc, slot, r, dist1, merge, blocksums);
-            if (blocks <= SCAN_FUSED_BLOCKS) {
-                k_ploc_scan_compact<<<blocks, T256, 0, st>>>(cur, nxt, merge, misc, slot, blocksums, blocks, bvh_nodes,
-                                                            dp, fused, slot_map, vtop, map_len, hist);
-            } else {
+        if (blocks <= PASS_TILES) {
+            // one launch per pass, then the flush; counts and merges double-buffered
+            for (int k = 0; k < PASSES_PER_SYNC; ++k) {
+                const uint32_t dist1 = (r == 1 || pass < search_depth_threshold) ? 1u : 0u;
+                launch_pass(blocks, st, cur, nxt, pass_counts[k & 1], k == 0 ? 0u : blocks, pass_counts[(k & 1) ^ 1],
+                            pass_merges[k & 1], pass_merges[(k & 1) ^ 1], misc, slot, r, dist1, bvh_nodes, dp, fused,
+                            slot_map, vtop, map_len, hist);
+                std::swap(cur, nxt);
+                slot ^= 1u;
+                pass++;
+            }
+            constexpr int last = PASSES_PER_SYNC & 1;
+            k_ploc_flush<<<blocks, PASS_THREADS, 0, st>>>(cur, nxt, pass_counts[last], blocks, pass_merges[last], misc,
+                                                          slot, bvh_nodes, dp, fused, slot_map, vtop, map_len, hist);
+            std::swap(cur, nxt);
+            slot ^= 1u;
+        } else {
+            for (int k = 0; k < PASSES_PER_SYNC; ++k) {
+                const uint32_t dist1 = (r == 1 || pass < search_depth_threshold) ? 1u : 0u;
+                launch_search_count(blocks, st, cur, misc, slot, r, dist1, merge, blocksums);
                 if (blocks <= SCAN_ONE_BLOCK) {
                     k_ploc_scan<<<1, 1024, 0, st>>>(blocksums, blocks, misc, slot, hist);
                 } else {
@@ -1575,10 +1873,10 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
                 }
                 k_ploc_compact<<<blocks, T256, 0, st>>>(cur, nxt, merge, misc, slot, blocksums, bvh_nodes, dp, fused,
                                                        slot_map, vtop, map_len);
+                std::swap(cur, nxt);
+                slot ^= 1u;
+                pass++;
             }
-            std::swap(cur, nxt);
-            slot ^= 1u;
-            pass++;
         }
         OBVHS_TRY(hipGetLastError(), "ploc pass launch");
         uint32_t herr_loop = 0u;
@@ -1635,13 +1933,14 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
     OBVHS_TRY(bvh->nodes.ensure((size_t)bvh->node_count * sizeof(Node32)), "alloc bvh2 nodes");
     BuildScratch& S = ctx->scratch;
     OBVHS_TRY(S.leaves.ensure((size_t)n * sizeof(Node32)), "alloc leaves");
-    OBVHS_TRY(S.clusters_a.ensure((size_t)n * sizeof(Node32)), "alloc clusters");
-    OBVHS_TRY(S.clusters_b.ensure((size_t)n * sizeof(Node32)), "alloc clusters");
+    OBVHS_TRY(S.clusters_a.ensure(((size_t)n + T256) * sizeof(Node32)), "alloc clusters");  // whole tiles
+    OBVHS_TRY(S.clusters_b.ensure(((size_t)n + T256) * sizeof(Node32)), "alloc clusters");
     OBVHS_TRY(S.keys.ensure((size_t)n * 8), "alloc keys");
     if (u128) OBVHS_TRY(S.keys_hi.ensure((size_t)n * 8), "alloc high key words");
     OBVHS_TRY(S.vals.ensure((size_t)n * 4), "alloc vals");
     OBVHS_TRY(S.tops.ensure((size_t)n * 4), "alloc top key words");
     OBVHS_TRY(S.merge.ensure((size_t)n + 64), "alloc merge");
+    OBVHS_TRY(S.pass_tiles.ensure(pass_tile_bytes(n)), "alloc pass tiles");
     const uint32_t nblk = (n + T256 - 1) / T256;
     OBVHS_TRY(S.blocksums.ensure((size_t)nblk * sizeof(uint2) + 64 + (size_t)nblk * 6 * 4), "alloc blocksums");
     OBVHS_TRY(S.sort_scratch.ensure(radix_sort_scratch_bytes(n)), "alloc sort scratch");
@@ -1733,13 +2032,14 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     BuildScratch& S = ctx->scratch;
     OBVHS_TRY(bvh->hist.ensure((size_t)(k + 1) * 4), "alloc pass history");
     OBVHS_TRY(S.leaves.ensure((size_t)k * sizeof(Node32)), "alloc leaves");
-    OBVHS_TRY(S.clusters_a.ensure((size_t)k * sizeof(Node32)), "alloc clusters");
-    OBVHS_TRY(S.clusters_b.ensure((size_t)k * sizeof(Node32)), "alloc clusters");
+    OBVHS_TRY(S.clusters_a.ensure(((size_t)k + T256) * sizeof(Node32)), "alloc clusters");  // whole tiles
+    OBVHS_TRY(S.clusters_b.ensure(((size_t)k + T256) * sizeof(Node32)), "alloc clusters");
     OBVHS_TRY(S.keys.ensure((size_t)k * 8), "alloc keys");
     if (u128) OBVHS_TRY(S.keys_hi.ensure((size_t)k * 8), "alloc high key words");
     OBVHS_TRY(S.vals.ensure((size_t)k * 4), "alloc vals");
     OBVHS_TRY(S.tops.ensure((size_t)k * 4), "alloc top key words");
     OBVHS_TRY(S.merge.ensure((size_t)k + 64), "alloc merge");
+    OBVHS_TRY(S.pass_tiles.ensure(pass_tile_bytes(k)), "alloc pass tiles");
     const uint32_t nblk = (k + T256 - 1) / T256;
     OBVHS_TRY(S.blocksums.ensure((size_t)nblk * sizeof(uint2) + 64 + (size_t)nblk * 6 * 4), "alloc blocksums");
     OBVHS_TRY(S.sort_scratch.ensure(radix_sort_scratch_bytes(k)), "alloc sort scratch");
