@@ -15,7 +15,11 @@
 //                quantises the child in slot s; prefix sums over the slots give the leaf primitive offsets and the
 //                internal children's DFS-derived node index, child base and primitive base, and the 80-byte node
 //                is assembled with lane shuffles (convert_to_cwbvh_impl, bvh2_to_cwbvh.rs:75-193;
-//                count_primitives 197-211).
+//                count_primitives 197-211).  A level of few nodes is one chain of loads and arithmetic (25K cycles
+//                before, 20K now at 2.4 GHz): the walk's 3 to 5 dependent loads 8K, the octant assignment 8.7K -> 5.7K
+//                (costs as order keys, the round's pick by two group minima instead of three-word butterflies), the
+//                primitives' gather 2.1K -> 1.1K (stored last), the level count and the items loaded side by side.
+//                1.29M triangles, 11 levels: 213 -> 191 us.
 // The exponent exp2(ceil(log2(x))) (bvh2_to_cwbvh.rs:85-88) goes through the host libm's log2f in the reference;
 // a 256-entry table of per-exponent mantissa thresholds, generated from that same log2f when the context is
 // created, reproduces it with integer compares.
@@ -168,6 +172,7 @@ constexpr int DPP_ROW_SHL4 = 0x104;
 constexpr int DPP_ROW_SHR1 = 0x111;
 constexpr int DPP_ROW_SHR2 = 0x112;
 constexpr int DPP_ROW_SHR4 = 0x114;
+constexpr int DPP_HALF_MIRROR = 0x141;  // lane i of 8 reads lane 7 - i
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
@@ -178,15 +183,17 @@ __device__ __forceinline__ uint32_t g8_xor4(uint32_t v, uint32_t r) {
     const uint32_t up = dpp<DPP_ROW_SHL4>(v), dn = dpp<DPP_ROW_SHR4>(v);
     return (r & 4u) ? dn : up;
 }
-__device__ __forceinline__ float g8_xor1f(float v) { return __uint_as_float(g8_xor1(__float_as_uint(v))); }
-__device__ __forceinline__ float g8_xor2f(float v) { return __uint_as_float(g8_xor2(__float_as_uint(v))); }
-__device__ __forceinline__ float g8_xor4f(float v, uint32_t r) { return __uint_as_float(g8_xor4(__float_as_uint(v), r)); }
 __device__ __forceinline__ uint32_t g8_or(uint32_t v) {
-    const uint32_t r = threadIdx.x & 7u;
     v |= g8_xor1(v);
     v |= g8_xor2(v);
-    v |= g8_xor4(v, r);
-    return v;
+    return v | dpp<DPP_HALF_MIRROR>(v);  // the other quad's, as in g8_min
+}
+// Smallest value of the group: after the quad steps every lane of a quad holds the quad's, and the mirrored half row
+// (lane i reads lane 7 - i) is the other quad's.
+__device__ __forceinline__ uint32_t g8_min(uint32_t v) {
+    v = min(v, g8_xor1(v));
+    v = min(v, g8_xor2(v));
+    return min(v, dpp<DPP_HALF_MIRROR>(v));
 }
 __device__ __forceinline__ uint32_t g8_inclusive_sum(uint32_t v, uint32_t r) {
     uint32_t t = dpp<DPP_ROW_SHR1>(v);
@@ -222,6 +229,8 @@ struct EmitOut {
     uint32_t rank;
     CwItem item;
     CwPre pre;
+    uint32_t* prims;  // where the slot's num_prims primitives p0, p1, p2 go
+    uint32_t num_prims, p0, p1, p2;
 };
 
 // One CWBVH node by the 8-lane group of lane r (every lane of the group calls with the same item).
@@ -285,34 +294,28 @@ __device__ __forceinline__ void emit_node(const Node32* __restrict__ nodes, cons
         }
         const uint32_t b = internal ? dbyte(rmeta, fdi) : 0u;
         const bool dist = internal && dkind(b) == KIND_DISTRIBUTE;
-        if (dist && (dleft(b) == DIDX_INVALID || dright(b) == DIDX_INVALID)) werr = DERR_CW_DISTRIBUTE;
-        werr = g8_or(werr);
-        if (werr != 0u || g8_or(dist ? 1u : 0u) == 0u) break;
-        const uint32_t w = mine ? (dist ? 2u : 1u) : 0u;
-        // every lane's width (2 bits each) in one word; lane r of the new frontier takes entry part of the entry of
-        // source lane q whose range [acc_q, acc_q + w_q) holds r (acc_q: the widths of the lanes before q)
-        const uint32_t widths = g8_or(w << (2u * r));
-        int src = 0;
-        uint32_t part = 0u, acc = 0u;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const uint32_t wq = (widths >> (2 * q)) & 3u;
-            if (r >= acc && r < acc + wq) {
-                src = q;
-                part = r - acc;
-            }
-            acc += wq;
+        // bit r: entry r is DISTRIBUTE; bit 8: one of them is malformed
+        const bool malformed = dist && (dleft(b) == DIDX_INVALID || dright(b) == DIDX_INVALID);
+        const uint32_t split = g8_or((dist ? 1u << r : 0u) | (malformed ? 0x100u : 0u));
+        if (split & 0x100u) {
+            werr = DERR_CW_DISTRIBUTE;
+            break;
         }
-        const int F2 = (int)acc;
+        if (split == 0u) break;
+        const int F2 = F + (int)__popc(split);
         if (F2 > 8) {  // more than 8 children
             werr = DERR_CAPACITY;
             break;
         }
+        // entry q moves to place q + (splits before it) and, split, takes the next place too: bit p of begins is set
+        // where an entry begins; lane r of the new frontier belongs to the last entry that begins at or before r
+        const uint32_t begins = g8_or(mine ? 1u << (r + (uint32_t)__popc(split & ((1u << r) - 1u))) : 0u);
+        const int src = (int)__popc(begins & ((2u << r) - 1u)) - 1;
+        const uint32_t part = (begins >> r & 1u) ^ 1u;
         const uint32_t sx = (uint32_t)__shfl((int)fx, src, 8), sinfo = (uint32_t)__shfl((int)finfo, src, 8);
         const uint32_t sdi = (uint32_t)__shfl((int)fdi, src, 8), sb = (uint32_t)__shfl((int)b, src, 8);
         const uint32_t skx = (uint32_t)__shfl((int)rkids.x, src, 8), sky = (uint32_t)__shfl((int)rkids.y, src, 8);
-        const uint32_t sw = (widths >> (2 * src)) & 3u;
-        if (sw == 2u) {  // a DISTRIBUTE entry's children: slots first, first + 1
+        if (split >> src & 1u) {  // a DISTRIBUTE entry's children: slots first, first + 1
             fx = (sinfo & ~KID_LEAF) + part;
             finfo = part != 0u ? sky : skx;
             fdi = part != 0u ? dright(sb) : dleft(sb);
@@ -348,43 +351,32 @@ __device__ __forceinline__ void emit_node(const Node32* __restrict__ nodes, cons
         const float px = (nb.hx + nb.lx) * 0.5f, py = (nb.hy + nb.ly) * 0.5f, pz = (nb.hz + nb.lz) * 0.5f;
         const float vx = (cb.hx + cb.lx) * 0.5f - px, vy = (cb.hy + cb.ly) * 0.5f - py,
                     vz = (cb.hz + cb.lz) * 0.5f - pz;
-        const float FMAX = 3.40282347e+38f;
-        uint32_t filled = 0u;
-        bool assigned = false;
+        // The cost of each slot as a key that orders like it (adding 0 makes -0 and 0 equal); a cost that is not below
+        // f32::MAX is never picked.  A round: the group's smallest key, then the smallest (child, slot) that has it.
+        constexpr uint32_t NEVER = 0xffffffffu;
+        uint32_t key[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const float dx = (s & 4) ? -1.0f : 1.0f, dy = (s & 2) ? -1.0f : 1.0f, dz = (s & 1) ? -1.0f : 1.0f;
+            const float v = (dx * vx + dy * vy) + dz * vz;  // exact for d in {+-1}^3
+            key[s] = has && v < 3.40282347e+38f ? f32_order_key(v + 0.0f) : NEVER;
+        }
         my_slot = -1;
+#pragma unroll 1
         for (int round = 0; round < 8; ++round) {
-            float bc = FMAX;
-            int bs = -1;
-            if (has && !assigned) {
+            const uint32_t own = min(min(min(key[0], key[1]), min(key[2], key[3])),
+                                     min(min(key[4], key[5]), min(key[6], key[7])));
+            const uint32_t low = g8_min(own);
+            if (low == NEVER) break;  // nothing left to place (the same in all 8 lanes)
+            uint32_t pick = NEVER;
 #pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    const float dx = (s & 4) ? -1.0f : 1.0f, dy = (s & 2) ? -1.0f : 1.0f,
-                                dz = (s & 1) ? -1.0f : 1.0f;
-                    const float v = (dx * vx + dy * vy) + dz * vz;  // exact for d in {+-1}^3
-                    if (!((filled >> s) & 1u) && v < bc) {
-                        bc = v;
-                        bs = s;
-                    }
-                }
-            }
-            int bl = (int)r;
+            for (int s = 7; s >= 0; --s) pick = key[s] == low ? r << 3 | (uint32_t)s : pick;
+            pick = g8_min(pick);
+            const uint32_t slot = pick & 7u;
+            const bool won = pick >> 3 == r;
+            my_slot = won ? (int)slot : my_slot;
 #pragma unroll
-            for (int m = 1; m < 8; m <<= 1) {
-                const float oc = m == 1 ? g8_xor1f(bc) : (m == 2 ? g8_xor2f(bc) : g8_xor4f(bc, r));
-                const int os = (int)(m == 1 ? g8_xor1((uint32_t)bs) : (m == 2 ? g8_xor2((uint32_t)bs) : g8_xor4((uint32_t)bs, r)));
-                const int ol = (int)(m == 1 ? g8_xor1((uint32_t)bl) : (m == 2 ? g8_xor2((uint32_t)bl) : g8_xor4((uint32_t)bl, r)));
-                if (os >= 0 && (bs < 0 || oc < bc || (oc == bc && ol < bl))) {
-                    bc = oc;
-                    bs = os;
-                    bl = ol;
-                }
-            }
-            if (bs < 0) break;  // the same (bs, bl) in all 8 lanes
-            filled |= 1u << bs;
-            if ((uint32_t)bl == r) {
-                assigned = true;
-                my_slot = bs;
-            }
+            for (int s = 0; s < 8; ++s) key[s] = won || slot == (uint32_t)s ? NEVER : key[s];
         }
         if (g8_or(has && my_slot < 0 ? 1u : 0u)) {
             if (r == 0u) atomicOr(&misc->err, DERR_CW_ORDER);
@@ -436,12 +428,13 @@ __device__ __forceinline__ void emit_node(const Node32* __restrict__ nodes, cons
         if (r == 0u) atomicOr(&misc->err, bad);
         return;
     }
-    if (lpc != 0u) {
-        const uint32_t dst = it.b + prim_off;
-        if (dst < pcap) oprims[dst] = bprims[pl.x];
-        if (lpc >= 2u && dst + 1u < pcap) oprims[dst + 1u] = bprims[pl.y];
-        if (lpc >= 3u && dst + 2u < pcap) oprims[dst + 2u] = bprims[pl.z];
-    }
+    // the leaf's primitives are loaded here and stored last
+    const uint32_t dst = it.b + prim_off;
+    const uint32_t np = dst < pcap ? min(lpc, pcap - dst) : 0u;
+    uint32_t p0 = 0u, p1 = 0u, p2 = 0u;
+    if (np >= 1u) p0 = bprims[pl.x];
+    if (np >= 2u) p1 = bprims[pl.y];
+    if (np >= 3u) p2 = bprims[pl.z];
 
     // The 80-byte node (bvh2_to_cwbvh.rs:85-170): exponents, quantised child boxes, meta bytes.
     const uint32_t ex = cw_exponent(nb.hx - nb.lx), ey = cw_exponent(nb.hy - nb.ly), ez = cw_exponent(nb.hz - nb.lz);
@@ -475,7 +468,12 @@ __device__ __forceinline__ void emit_node(const Node32* __restrict__ nodes, cons
     if (r < 5u) reinterpret_cast<uint4*>(&onodes[it.cw_index])[r] = chunk;
 
     // Children's DFS numbering (pre-order, child blocks appended at visit time, bvh2_to_cwbvh.rs:172-191); the
-    // caller places the items.
+    // caller places the items and stores the primitives.
+    eo.prims = oprims + dst;
+    eo.num_prims = np;
+    eo.p0 = p0;
+    eo.p1 = p1;
+    eo.p2 = p2;
     if (num_internal == 0u) return;
     const uint32_t s_cw = (uint32_t)__shfl((int)rcw, sl, 8), s_np = (uint32_t)__shfl((int)rnp, sl, 8);
     const uint32_t s_meta0 = (uint32_t)__shfl((int)(rmeta.x & 0xffu), sl, 8);
@@ -498,22 +496,36 @@ __global__ void __launch_bounds__(T256) k_cw_emit(const Node32* __restrict__ nod
                                                   DpView dp,
                                                   const CwItem* __restrict__ in_items, CwItem* __restrict__ out_items,
                                                   const CwPre* __restrict__ in_pre, CwPre* __restrict__ out_pre,
-                                                  uint32_t level, uint32_t order_children, CwNode* __restrict__ out,
-                                                  uint32_t* __restrict__ out_prims, uint32_t cw_cap, uint32_t prim_cap,
-                                                  CwMisc* misc, const MeshDesc* __restrict__ meshes) {
+                                                  uint32_t item_cap, uint32_t level, uint32_t order_children,
+                                                  CwNode* __restrict__ out, uint32_t* __restrict__ out_prims,
+                                                  uint32_t cw_cap, uint32_t prim_cap, CwMisc* misc,
+                                                  const MeshDesc* __restrict__ meshes) {
     constexpr uint32_t GROUPS = T256 / 8;
     __shared__ uint32_t s_count, s_base;
     const uint32_t r = threadIdx.x & 7u;
+    // the first items are loaded beside the count (item_cap: what the lists hold)
+    uint32_t t = blockIdx.x * GROUPS + (threadIdx.x >> 3);
+    CwItem item{};
+    CwPre pre{};
+    if (t < item_cap) {
+        item = in_items[t];
+        pre = in_pre[t];
+    }
     const uint32_t count = misc->level_count[level];
     for (uint32_t first = blockIdx.x * GROUPS; first < count; first += gridDim.x * GROUPS) {
-        const uint32_t t = first + (threadIdx.x >> 3);
         EmitOut eo;
         eo.num_internal = 0u;
         eo.isint = 0u;
         eo.rank = 0u;
+        eo.num_prims = 0u;
         if (t < count)
-            emit_node(nodes, bvh2_prims, dp, in_items[t], in_pre[t], r, level, order_children, out, out_prims,
-                      cw_cap, prim_cap, misc, meshes, eo);
+            emit_node(nodes, bvh2_prims, dp, item, pre, r, level, order_children, out, out_prims, cw_cap, prim_cap,
+                      misc, meshes, eo);
+        t += gridDim.x * GROUPS;
+        if (t < count) {
+            item = in_items[t];
+            pre = in_pre[t];
+        }
         if (threadIdx.x == 0) s_count = 0u;
         __syncthreads();
         uint32_t off = 0u;
@@ -526,6 +538,9 @@ __global__ void __launch_bounds__(T256) k_cw_emit(const Node32* __restrict__ nod
             out_items[s_base + off + eo.rank] = eo.item;
             out_pre[s_base + off + eo.rank] = eo.pre;
         }
+        if (eo.num_prims >= 1u) eo.prims[0] = eo.p0;
+        if (eo.num_prims >= 2u) eo.prims[1] = eo.p1;
+        if (eo.num_prims >= 3u) eo.prims[2] = eo.p2;
         __syncthreads();  // s_count and s_base are reused by the next iteration
     }
 }
@@ -737,7 +752,7 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
         const CwItem* in_items = level == 0 ? &misc->root_item : items[level & 1];
         const CwPre* in_pre = level == 0 ? &misc->root_pre : pres[level & 1];
         k_cw_emit<<<g, T256, 0, st>>>(nodes, bvh2->prim_indices.as<uint32_t>(), dp, in_items,
-                                      items[(level + 1) & 1], in_pre, pres[(level + 1) & 1], level,
+                                      items[(level + 1) & 1], in_pre, pres[(level + 1) & 1], (uint32_t)cap, level,
                                       order_children ? 1u : 0u, out->nodes.as<CwNode>(),
                                       out->prim_indices.as<uint32_t>(), ncw, n, misc, nullptr);
         bound = cap * 8;  // never past 8 * ncw, however deep the tree
@@ -810,7 +825,8 @@ obvhs_status cwbvh_convert_batch(obvhs_context* ctx, const Node32* nodes, const 
         if (capl == 0) continue;
         const uint32_t g = (uint32_t)std::min<uint64_t>((capl * 8 + T256 - 1) / T256, EMIT_MAX_BLOCKS);
         k_cw_emit<<<g, T256, 0, st>>>(nodes, bvh2_prims, dp, items[level & 1], items[(level + 1) & 1],
-                                      pres[level & 1], pres[(level + 1) & 1], level, order_children ? 1u : 0u,
+                                      pres[level & 1], pres[(level + 1) & 1], (uint32_t)capl, level,
+                                      order_children ? 1u : 0u,
                                       out_nodes.as<CwNode>(), out_prims.as<uint32_t>(), 0u, 0u, misc,
                                       d_meshes);
         bound = capl * 8;
