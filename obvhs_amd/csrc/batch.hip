@@ -299,27 +299,17 @@ __global__ void __launch_bounds__(T256) k_b_search(const Node32* __restrict__ cu
 }
 
 // ploc/mod.rs:423-439 within the cluster's segment (indices are global, offsets stay inside the segment).
-__device__ __forceinline__ void b_classify(const int8_t* __restrict__ merge, const uint32_t* __restrict__ cmesh,
-                                           const SegState* __restrict__ seg, uint32_t i, uint32_t total, bool& emit,
-                                           bool& mrg, uint32_t& b) {
-    emit = false;
-    mrg = false;
-    b = i;
-    if (i >= total) return;
-    const SegState sg = seg[cmesh[i]];
-    if (sg.count <= 1u) {
-        emit = true;
-        return;
-    }
-    const int bi = (int)i + (int)merge[i];
-    b = (uint32_t)bi;
-    const bool mutual = bi + (int)merge[bi] == (int)i;
-    if (!mutual || bi == (int)i) {
-        emit = true;
-    } else if (bi < (int)i) {
-        emit = true;
-        mrg = true;
-    }
+struct BCls {
+    bool emit, mrg;
+    uint32_t b;  // the neighbour
+};
+__device__ __forceinline__ BCls b_classify(const int8_t* __restrict__ merge, const uint32_t* __restrict__ cmesh,
+                                           const SegState* __restrict__ seg, uint32_t i, uint32_t total) {
+    const bool valid = i < total;
+    const bool pair = valid && seg[cmesh[valid ? i : 0u]].count > 1u;
+    const int bi = pair ? (int)i + (int)merge[i] : (int)i;
+    const bool mutual = pair && bi + (int)merge[bi] == (int)i;
+    return BCls{valid && (!mutual || bi <= (int)i), mutual && bi < (int)i, (uint32_t)bi};
 }
 
 __global__ void __launch_bounds__(T256) k_b_count(const int8_t* __restrict__ merge, const uint32_t* __restrict__ cmesh,
@@ -327,10 +317,8 @@ __global__ void __launch_bounds__(T256) k_b_count(const int8_t* __restrict__ mer
                                                   uint2* __restrict__ blocksums, uint32_t q) {
     __shared__ uint32_t we[T256 / 64], wm[T256 / 64];
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
-    bool emit, mrg;
-    uint32_t b;
-    b_classify(merge, cmesh, seg, i, misc->total[q], emit, mrg, b);
-    const uint32_t e = (uint32_t)__popcll(__ballot(emit)), m = (uint32_t)__popcll(__ballot(mrg));
+    const BCls k = b_classify(merge, cmesh, seg, i, misc->total[q]);
+    const uint32_t e = (uint32_t)__popcll(__ballot(k.emit)), m = (uint32_t)__popcll(__ballot(k.mrg));
     const uint32_t wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63u) == 0) {
         we[wave] = e;
@@ -519,9 +507,9 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     Node32 a{};
     if (i < total) a = load_node(&cur[i]);  // before the classification's dependent loads and the barrier
-    bool emit, mrg;
-    uint32_t b;
-    b_classify(merge, cmesh, seg, i, total, emit, mrg, b);
+    const BCls k = b_classify(merge, cmesh, seg, i, total);
+    const bool emit = k.emit, mrg = k.mrg;
+    const uint32_t b = k.b;
     const uint64_t be = __ballot(emit), bm = __ballot(mrg);
     const uint64_t lt = lanemask_lt();
     const uint32_t wave = threadIdx.x >> 6;
@@ -529,7 +517,7 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
         we[wave] = (uint32_t)__popcll(be);
         wm[wave] = (uint32_t)__popcll(bm);
     }
-    __syncthreads();
+    lds_barrier();
     if (emit) {
         uint32_t pe = offsets[blockIdx.x].x, pm = 0u;
         for (uint32_t w = 0; w < wave; ++w) {
@@ -562,7 +550,7 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
             store_node(&next[pos], a);
         }
     }
-    __syncthreads();
+    lds_barrier();  // the stores are not waited for
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
     if (threadIdx.x < nm) {
         const Node32 l = s_left[threadIdx.x], r = s_right[threadIdx.x];

@@ -231,6 +231,8 @@ __device__ __forceinline__ DpChild dp_child(const Node32& c) {
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
                                                 const DpChild& r) {
     const DpRaw raw_l = load_dp_raw(dp_child_record(dp, l)), raw_r = load_dp_raw(dp_child_record(dp, r));
+    // every load stays above this line: spread over the evaluation to save registers, each part waits on its own
+    __builtin_amdgcn_sched_barrier(0);
     return dp_evaluate(dp, ha, first, l, r, raw_l, raw_r);
 }
 

@@ -41,6 +41,13 @@ __device__ __forceinline__ bool box_has_nan(const Box& b) {
     return isnan(b.lx) || isnan(b.ly) || isnan(b.lz) || isnan(b.hx) || isnan(b.hy) || isnan(b.hz);
 }
 
+// A workgroup barrier for data in LDS only: global loads and stores in flight are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // morton.rs:35-43
 __device__ __forceinline__ uint64_t split_by_3_u64(uint32_t a) {
     uint64_t x = (uint64_t)a & 0x1fffffull;

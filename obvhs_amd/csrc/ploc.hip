@@ -541,36 +541,18 @@ __global__ void __launch_bounds__(SMALL_THREADS)
     }
 }
 
-// A workgroup barrier for data in LDS only: global loads and stores in flight are not waited for.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Classification of cluster i (ploc/mod.rs:423-439): `emit` when it goes to the next pass (kept, or the higher
 // index of a mutual pair, which becomes the parent), `mrg` when it is the higher index of a mutual pair.
 // A self-pair (no finite neighbour, already flagged as an error) is treated as kept so that no slot underflows.
-__device__ __forceinline__ void classify(const int8_t* merge, uint32_t i, uint32_t count, bool& emit, bool& mrg,
-                                         uint32_t& b) {
-    emit = false;
-    mrg = false;
-    b = i;
-    if (i >= count) return;
-    if (count == 1) {
-        emit = true;
-        return;
-    }
-    int m = merge[i];
-    int bi = (int)i + m;
-    b = (uint32_t)bi;
-    bool mutual = bi + (int)merge[bi] == (int)i;
-    if (!mutual || bi == (int)i) {
-        emit = true;
-    } else if (bi < (int)i) {
-        emit = true;
-        mrg = true;
-    }
+struct Cls {
+    bool emit, mrg;
+    uint32_t b;  // the neighbour
+};
+__device__ __forceinline__ Cls classify(const int8_t* merge, uint32_t i, uint32_t count) {
+    const bool valid = i < count, pair = valid && count > 1u;
+    const int bi = pair ? (int)i + (int)merge[i] : (int)i;
+    const bool mutual = pair && bi + (int)merge[bi] == (int)i;
+    return Cls{valid && (!mutual || bi <= (int)i), mutual && bi < (int)i, (uint32_t)bi};
 }
 
 // The neighbour search of one pass (ploc/mod.rs:329-419) and the per-tile counts of emitted clusters and merges in
@@ -744,7 +726,7 @@ __global__ void __launch_bounds__(SC_THREADS) k_ploc_search_count(const Node32* 
     if (t < (uint32_t)T256) c = (int)(base + t);
     else if (t - T256 < 2u * r) c = t - T256 < r ? (int)base - (int)r + (int)(t - T256) : (int)(base + t - r);
     if (c >= 0 && (uint32_t)c < count) {
-        int8_t m;
+        int8_t m = 0;
         bool unrolled = false;
         if constexpr (R > 0) {
             if (!dist1) {
@@ -883,7 +865,7 @@ constexpr uint32_t MAX_TILE_MERGES = (T256 + MAX_RADIUS) / 2;
 // clusters merge runs the evaluation in about one wave per tile instead of in every wave with a few lanes active.
 // The caller classifies its cluster and loads its node (`a`, for i < count) at the start of the kernel, so that
 // those loads overlap the tile offsets' loads.  Called by every thread of the workgroup (it holds workgroup
-// barriers).
+// barriers, for LDS only: the clusters' stores are not waited for).
 __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Node32* __restrict__ next,
                                              const Node32& a, bool emit, bool mrg, uint32_t b,
                                              const PlocState& st, uint32_t pe0, uint32_t pm0,
@@ -900,7 +882,7 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
         we[wave] = (uint32_t)__popcll(be);
         wm[wave] = (uint32_t)__popcll(bm);
     }
-    __syncthreads();
+    lds_barrier();
     if (emit) {
         uint32_t pe = pe0, pm = pm0;
         for (uint32_t w = 0; w < wave; ++w) {
@@ -929,7 +911,7 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
         }
     }
     if (!fused) return;  // uniform
-    __syncthreads();
+    lds_barrier();
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
     if (threadIdx.x < nm && s_first[threadIdx.x] != UINT32_MAX) {
         const Node32 l = s_left[threadIdx.x], r = s_right[threadIdx.x];
@@ -949,11 +931,9 @@ __global__ void __launch_bounds__(T256) k_ploc_compact(const Node32* __restrict_
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     Node32 a{};
     if (i < st.count) a = load_node(&cur[i]);
-    bool emit, mrg;
-    uint32_t b;
-    classify(merge, i, st.count, emit, mrg, b);
+    const Cls k = classify(merge, i, st.count);
     const uint2 off = offsets[blockIdx.x];
-    compact_tile(cur, next, a, emit, mrg, b, st, off.x, off.y, bvh_nodes, dp, fused, slot_map, vtop, map_len,
+    compact_tile(cur, next, a, k.emit, k.mrg, k.b, st, off.x, off.y, bvh_nodes, dp, fused, slot_map, vtop, map_len,
                  &misc->err, we, wm);
 }
 
@@ -1502,8 +1482,10 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_ploc_tail(const Node32* __rest
             be[q] = bm[q] = 0ull;
             if (q > 0 && !two) continue;  // uniform
             const uint32_t i = two ? tid * TAIL_ITEMS + q : tid;
-            uint32_t b;
-            classify(mg, i, count, emit[q], mrg[q], b);
+            const Cls k = classify(mg, i, count);
+            const uint32_t b = k.b;
+            emit[q] = k.emit;
+            mrg[q] = k.mrg;
             be[q] = __ballot(emit[q]);
             bm[q] = __ballot(mrg[q]);
             // everything this thread writes is read before anyone overwrites the LDS arrays
