@@ -12,6 +12,7 @@
 //     (ploc/mod.rs:508-528), prefix sums run over the whole array, and a per-mesh pass computes each segment's
 //     new start, count, insert index and merge base so that child slots are insert_m - 2(s_m + 1) with s_m the
 //     merge's rank inside its mesh (ploc/mod.rs:420-487).  Finished meshes keep one cluster that is copied along.
+//     Once no mesh has more than 1,024 clusters, one workgroup per mesh makes its remaining passes (tail.hpp).
 //     The cost table is evaluated by the merges (cwdp.hpp) with the mesh's key base.
 //   * CWBVH emit: one launch per level over all meshes (cwbvh.hip).
 //   * traversal: one lane per ray, the ray's mesh selects the CWBVH and triangle slices.
@@ -26,6 +27,7 @@
 #include "cwdp.hpp"
 #include "device_util.hpp"
 #include "internal.hpp"
+#include "tail.hpp"
 
 struct obvhs_batch {
     obvhs::DevBuf tri_offsets;    // u32[m+1]
@@ -46,9 +48,10 @@ namespace obvhs {
 namespace {
 
 constexpr int T256 = 256;
-constexpr uint32_t MAX_RADIUS = 32;
 // Passes between host reads; 8 and 16 measured slower here (16.1 -> 16.8 and 18.3 ms): grids sized at the last read.
 constexpr int PASSES_PER_SYNC = 4;
+// Clusters of a mesh that one workgroup takes over (k_b_tail).
+constexpr int B_TAIL_MAX = 1024;
 
 struct SegState {
     uint32_t start;   // first cluster of the mesh in the current cluster array
@@ -62,8 +65,9 @@ struct SegState {
 struct BatchMisc {
     uint32_t err;
     uint32_t total[2];   // clusters in the current array (by pass parity)
-    uint32_t active;     // 1 if a mesh has more than one cluster after the last pass, else 0
+    uint32_t large;      // 1 if a mesh has more than B_TAIL_MAX clusters after the last pass, else 0
     uint32_t totals[2];  // emits, merges of the pass
+    uint32_t passes;     // of the mesh that took most
 };
 
 __device__ __forceinline__ uint32_t mesh_in(const uint32_t* __restrict__ offsets, uint32_t lo, uint32_t hi,
@@ -89,7 +93,8 @@ __global__ void __launch_bounds__(T256) k_b_init(uint32_t* __restrict__ bounds, 
         misc->err = 0u;
         misc->total[0] = n_total;
         misc->total[1] = 0u;
-        misc->active = 0u;
+        misc->large = 0u;
+        misc->passes = 0u;
     }
     if (i >= m) return;
     for (int a = 0; a < 3; ++a) {
@@ -390,7 +395,7 @@ __global__ void __launch_bounds__(T256) k_b_count(const int8_t* __restrict__ mer
     }
 }
 
-// Also writes the next pass's cluster count (total[q ^ 1]) and clears the active-mesh flag k_b_segments sets.
+// Also writes the next pass's cluster count (total[q ^ 1]) and clears the flag k_b_segments sets.
 __global__ void __launch_bounds__(1024) k_b_scan(uint2* __restrict__ blocksums, uint32_t nblocks, BatchMisc* misc,
                                                  uint32_t q) {
     __shared__ uint32_t se[16], sm[16];
@@ -424,7 +429,7 @@ __global__ void __launch_bounds__(1024) k_b_scan(uint2* __restrict__ blocksums, 
         misc->totals[0] = re;
         misc->totals[1] = rm;
         misc->total[q ^ 1u] = re;
-        misc->active = 0u;
+        misc->large = 0u;
     }
     __syncthreads();
     uint32_t ee = se[wave] + ie - E, em = sm[wave] + im - M;
@@ -454,7 +459,7 @@ __global__ void __launch_bounds__(1024) k_b_scan_apply(uint2* __restrict__ block
         misc->totals[0] = all.x;
         misc->totals[1] = all.y;
         misc->total[q ^ 1u] = all.x;
-        misc->active = 0u;
+        misc->large = 0u;
     }
 }
 
@@ -522,7 +527,7 @@ __global__ void __launch_bounds__(T256) k_b_segments(const int8_t* __restrict__ 
                                                      uint32_t m, BatchMisc* misc, uint32_t q) {
     const uint32_t k = (blockIdx.x * T256 + threadIdx.x) >> 6;
     const uint32_t lane = threadIdx.x & 63u;
-    bool active = false;
+    bool large = false;
     if (k < m) {  // wave-uniform
         const SegState sg = seg[k];
         if (sg.count == 0u) {
@@ -536,13 +541,13 @@ __global__ void __launch_bounds__(T256) k_b_segments(const int8_t* __restrict__ 
                 seg[k].mbase = head.y;
                 const SegState nx{head.x, end.x - head.x, sg.insert - 2u * merges, 0u};
                 seg_next[k] = nx;
-                active = nx.count > 1u;
+                large = nx.count > (uint32_t)B_TAIL_MAX;
             }
         }
     }
-    // One flag write per block: the host only asks whether any mesh is still active, and 4,096 waves adding to
-    // one counter serialise on it.
-    if (__syncthreads_or(active) && threadIdx.x == 0) misc->active = 1u;
+    // One flag write per block: the host only asks whether any mesh is still large, and 4,096 waves adding to one
+    // counter serialise on it.
+    if (__syncthreads_or(large) && threadIdx.x == 0) misc->large = 1u;
 }
 
 __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ cur, Node32* __restrict__ next,
@@ -616,21 +621,32 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     }
 }
 
-// Roots (ploc/mod.rs:499): the mesh's last cluster goes to its node 0.
-__global__ void __launch_bounds__(T256) k_b_roots(const Node32* __restrict__ cur, const SegState* __restrict__ seg,
-                                                  const MeshDesc* __restrict__ meshes, uint32_t m,
-                                                  Node32* __restrict__ nodes, uint32_t* __restrict__ prims,
-                                                  BatchMisc* misc) {
-    const uint32_t k = blockIdx.x * T256 + threadIdx.x;
-    if (k >= m) return;
-    const SegState sg = seg[k];
-    const MeshDesc md = meshes[k];
-    if (md.prim_count == 0u) return;
-    if (sg.count != 1u || sg.insert != 1u) {
-        atomicOr(&misc->err, DERR_SELF_MERGE);  // ploc/mod.rs:496
+// The remaining passes of every mesh of search distance r, one workgroup per mesh (tail.hpp), once no mesh has more
+// than B_TAIL_MAX clusters; its last cluster goes to the mesh's node 0 (ploc/mod.rs:495-499).  R: r if that distance
+// has an unrolled search, else 0.
+// A mesh's chain of passes bounds a workgroup, not any throughput; two of them fit a CU's LDS.  4,096 icospheres of up
+// to 20,480 triangles: passes 16 to 48 in 321 us, about 0.8 ms as launches over all meshes (build 10.17 -> 9.69 ms).
+template <int R>
+__global__ void __launch_bounds__(B_TAIL_MAX / 2, 4) k_b_tail(const Node32* __restrict__ cur,
+                                                           const SegState* __restrict__ seg, BatchMisc* misc,
+                                                           const MeshDesc* __restrict__ meshes, uint32_t r,
+                                                           uint32_t first_pass, uint32_t depth_threshold,
+                                                           Node32* __restrict__ nodes, DpView dp, uint32_t q) {
+    const MeshDesc md = meshes[blockIdx.x];
+    const SegState sg = seg[blockIdx.x];
+    if (md.prim_count == 0u || md.radius != r || misc->total[q] == 0u) return;  // total 0: DERR_RESORT
+    if (sg.count == 0u || sg.count > (uint32_t)B_TAIL_MAX) {
+        if (threadIdx.x == 0) atomicOr(&misc->err, DERR_CAPACITY);
         return;
     }
-    store_node(&nodes[md.node_base], load_node(&cur[sg.start]));
+    dp.kbase = md.prim_base;
+    PlocState st{sg.count, sg.insert, first_pass, 0u, 0ull};
+    ploc_tail<R, B_TAIL_MAX>(cur + sg.start, st, first_pass, r, r == 1u ? 1u : 0u, depth_threshold,
+                             nodes + md.node_base, nullptr, dp, 1u, nullptr, 0u, 0u, &misc->err);
+    if (threadIdx.x == 0) {
+        if (st.count != 1u || st.insert != 1u) atomicOr(&misc->err, DERR_SELF_MERGE);
+        atomicMax(&misc->passes, st.depth);
+    }
 }
 
 // Root box of every mesh's BVH2 (the BLAS bounds a TLAS is built over), as Aabb records.
@@ -651,6 +667,23 @@ __global__ void __launch_bounds__(T256) k_b_root_boxes(const Node32* __restrict_
         hipError_t _e = (expr);                                     \
         if (_e != hipSuccess) return set_hip_error(ctx, _e, where); \
     } while (0)
+
+// The tail for the search distance (each allowed distance has its unrolled instance).
+static void launch_tail(hipStream_t st, const Node32* cur, const SegState* seg, BatchMisc* misc,
+                        const MeshDesc* meshes, uint32_t m, uint32_t r, uint32_t pass, uint32_t threshold,
+                        Node32* nodes, const DpView& dp, uint32_t q) {
+#define OBVHS_TAIL(RR) \
+    k_b_tail<RR><<<m, B_TAIL_MAX / 2, 0, st>>>(cur, seg, misc, meshes, r, pass, threshold, nodes, dp, q)
+    switch (r) {
+        case 2: OBVHS_TAIL(2); break;
+        case 6: OBVHS_TAIL(6); break;
+        case 14: OBVHS_TAIL(14); break;
+        case 24: OBVHS_TAIL(24); break;
+        case 32: OBVHS_TAIL(32); break;
+        default: OBVHS_TAIL(0); break;
+    }
+#undef OBVHS_TAIL
+}
 
 static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const uint32_t* h_offsets,
                                 uint32_t m, uint32_t r, uint32_t sdt, uint32_t max_prims, obvhs_batch* B) {
@@ -757,64 +790,75 @@ static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris
         if (ss != OBVHS_OK) return ss;
     }
 
-    uint32_t known = n;
-    uint32_t pass = 0;
-    int cm = 0;    // which cluster-mesh buffer is current
-    int cs = 0;    // which segment table is current
+    // The search distances of the meshes, for the tail's launches.
+    bool has_radius[MAX_RADIUS + 1] = {};
+    for (const MeshDesc& md : B->meshes)
+        if (md.prim_count) has_radius[md.radius] = true;
     uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
     for (;;) {
-        const uint32_t blocks = (known + T256 - 1) / T256;
-        for (int rep = 0; rep < PASSES_PER_SYNC; ++rep) {
-            const uint32_t q = pass & 1u;
-            k_b_search<<<blocks, T256, 0, st>>>(cur, cmesh[cm], seg[cs], misc, d_meshes, rmax,
-                                                pass < sdt ? 1u : 0u, merge, q);
-            k_b_count<<<blocks, T256, 0, st>>>(merge, cmesh[cm], seg[cs], misc, blocksums, q);
-            if (blocks <= B_SCAN_ONE_BLOCK) {
-                k_b_scan<<<1, 1024, 0, st>>>(blocksums, blocks, misc, q);
-            } else {
-                uint2* chunk_tot = blocksums + blocks + 16;
-                const uint32_t nchunks = (blocks + SCAN_CHUNK - 1) / SCAN_CHUNK;
-                k_b_scan_chunks<<<nchunks, 1024, 0, st>>>(blocksums, blocks, chunk_tot);
-                k_b_scan_apply<<<nchunks, 1024, 0, st>>>(blocksums, blocks, chunk_tot, nchunks, misc, q);
+        uint32_t known = n;
+        uint32_t pass = 0;
+        int cm = 0;  // which cluster-mesh buffer is current
+        int cs = 0;  // which segment table is current
+        bool large = biggest > (uint32_t)B_TAIL_MAX;
+        uint32_t err = 0;
+        while (large && err == 0u) {
+            const uint32_t blocks = (known + T256 - 1) / T256;
+            for (int rep = 0; rep < PASSES_PER_SYNC; ++rep) {
+                const uint32_t q = pass & 1u;
+                k_b_search<<<blocks, T256, 0, st>>>(cur, cmesh[cm], seg[cs], misc, d_meshes, rmax,
+                                                    pass < sdt ? 1u : 0u, merge, q);
+                k_b_count<<<blocks, T256, 0, st>>>(merge, cmesh[cm], seg[cs], misc, blocksums, q);
+                if (blocks <= B_SCAN_ONE_BLOCK) {
+                    k_b_scan<<<1, 1024, 0, st>>>(blocksums, blocks, misc, q);
+                } else {
+                    uint2* chunk_tot = blocksums + blocks + 16;
+                    const uint32_t nchunks = (blocks + SCAN_CHUNK - 1) / SCAN_CHUNK;
+                    k_b_scan_chunks<<<nchunks, 1024, 0, st>>>(blocksums, blocks, chunk_tot);
+                    k_b_scan_apply<<<nchunks, 1024, 0, st>>>(blocksums, blocks, chunk_tot, nchunks, misc, q);
+                }
+                k_b_segments<<<(m + 3u) / 4u, T256, 0, st>>>(merge, cmesh[cm], seg[cs], seg[cs ^ 1], blocksums, m,
+                                                              misc, q);
+                k_b_compact<<<blocks, T256, 0, st>>>(cur, nxt, cmesh[cm], cmesh[cm ^ 1], merge, seg[cs], misc,
+                                                     blocksums, d_meshes, nodes, dp, q);
+                std::swap(cur, nxt);
+                cm ^= 1;
+                cs ^= 1;
+                pass++;
             }
-            k_b_segments<<<(m + 3u) / 4u, T256, 0, st>>>(merge, cmesh[cm], seg[cs], seg[cs ^ 1], blocksums, m,
-                                                          misc, q);
-            k_b_compact<<<blocks, T256, 0, st>>>(cur, nxt, cmesh[cm], cmesh[cm ^ 1], merge, seg[cs], misc, blocksums,
-                                                 d_meshes, nodes, dp, q);
-            std::swap(cur, nxt);
-            cm ^= 1;
-            cs ^= 1;
-            pass++;
+            OBVHS_TRY(hipGetLastError(), "batch pass launch");
+            OBVHS_TRY(hipMemcpyAsync(h, misc, 16, hipMemcpyDeviceToHost, st), "read batch state");
+            OBVHS_TRY(hipStreamSynchronize(st), "batch pass sync");
+            err = h[0];
+            large = h[3] != 0u;
+            // Every mesh of several clusters merges at least one pair per pass unless costs are NaN.
+            const uint32_t now = h[1 + (pass & 1u)];
+            if (err == 0u && large && now >= known) return OBVHS_ERR_PLOC_SELF_MERGE;
+            known = now;
         }
-        OBVHS_TRY(hipGetLastError(), "batch pass launch");
-        OBVHS_TRY(hipMemcpyAsync(h, misc, 16, hipMemcpyDeviceToHost, st), "read batch state");
-        OBVHS_TRY(hipStreamSynchronize(st), "batch pass sync");
-        if (h[0] & ~DERR_RESORT) return device_error_to_status(h[0] & ~DERR_RESORT);
-        if (h[0]) {
-            // A long run of equal keys: the passes found no clusters and wrote none, so the codes and the leaves'
-            // meshes are as they were.  The segments, the counts and the error word start over (so do the bounds,
-            // which the codes no longer need).
-            k_b_init<<<mblk, T256, 0, st>>>(bounds, offsets, m, seg[0], misc, n);
-            cur = S.clusters_a.as<Node32>();
-            nxt = S.clusters_b.as<Node32>();
-            pass = 0;
-            cm = cs = 0;
-            const obvhs_status ss = sort_codes_then_meshes();
-            if (ss != OBVHS_OK) return ss;
-            continue;
+        if (err == 0u) {
+            for (uint32_t rr = 1; rr <= MAX_RADIUS; ++rr)
+                if (has_radius[rr])
+                    launch_tail(st, cur, seg[cs], misc, d_meshes, m, rr, pass, sdt, nodes, dp, pass & 1u);
+            OBVHS_TRY(hipGetLastError(), "batch tail launch");
+            OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(BatchMisc), hipMemcpyDeviceToHost, st), "read batch state");
+            OBVHS_TRY(hipStreamSynchronize(st), "batch tail sync");
+            err = h[0];
         }
-        if (h[3] == 0u) break;  // every mesh is down to its root
-        // Every active mesh merges at least one pair per pass unless costs are NaN.
-        const uint32_t now = h[1 + (pass & 1u)];
-        if (now >= known) return OBVHS_ERR_PLOC_SELF_MERGE;
-        known = now;
+        if (err & ~DERR_RESORT) return device_error_to_status(err & ~DERR_RESORT);
+        if (err == 0u) break;
+        // A long run of equal keys: the passes found no clusters and wrote none, so the codes and the leaves' meshes
+        // are as they were.  The segments, the counts and the error word start over (so do the bounds, which the
+        // codes no longer need).
+        k_b_init<<<mblk, T256, 0, st>>>(bounds, offsets, m, seg[0], misc, n);
+        cur = S.clusters_a.as<Node32>();
+        nxt = S.clusters_b.as<Node32>();
+        const obvhs_status ss = sort_codes_then_meshes();
+        if (ss != OBVHS_OK) return ss;
     }
-    B->passes = pass;
-    k_b_roots<<<mblk, T256, 0, st>>>(cur, seg[cs], d_meshes, m, nodes, B->bvh2_prims.as<uint32_t>(), misc);
-    OBVHS_TRY(hipGetLastError(), "batch roots launch");
-    OBVHS_TRY(hipMemcpyAsync(h, misc, 4, hipMemcpyDeviceToHost, st), "read batch err");
-    OBVHS_TRY(hipStreamSynchronize(st), "batch roots sync");
-    if (h[0]) return device_error_to_status(h[0]);
+    // reported in whole rounds of launches
+    const uint32_t deepest = std::max(reinterpret_cast<const BatchMisc*>(h)->passes, 1u);
+    B->passes = (deepest + PASSES_PER_SYNC - 1) / PASSES_PER_SYNC * PASSES_PER_SYNC;
     return cwbvh_convert_batch(ctx, nodes, B->bvh2_prims.as<uint32_t>(), dp, d_meshes, B->meshes, n, true,
                                B->cw_nodes, B->cw_prims, B->cw_total);
 }

@@ -1,5 +1,7 @@
-"""Batched builds where the sort changes form: runs of equal sort keys around the limit of the ranking (64) and a mesh
-too large for the 32-bit keys.  Every mesh's CWBVH equals the oracle's build of that mesh alone."""
+"""Batched builds where the sort and the last passes change form: runs of equal sort keys around the limit of the
+ranking (64), a mesh too large for the 32-bit keys, and meshes of cluster counts around the steps of the one-workgroup
+passes (1,024 clusters at most, several lanes per cluster below 256 and 128, one wave below 64).  Every mesh's CWBVH
+equals the oracle's build of that mesh alone."""
 import numpy as np
 import pytest
 
@@ -34,3 +36,12 @@ def test_many_meshes_one_large(ctx, size):
         _, rcw, rprims = O.build_cwbvh(m, 14, 0, 3)
         assert_same_bytes(n_i, rcw, f"mesh {i} nodes")
         np.testing.assert_array_equal(p_i, rprims)
+
+
+EDGES = [1, 2, 3, 16, 17, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1023, 1024]
+
+
+@pytest.mark.parametrize("more", [[], [1025, 2500]])
+@pytest.mark.parametrize("sd,sdt", [(1, 0), (2, 0), (6, 0), (14, 0), (14, 3), (24, 2), (32, 0)])
+def test_tail_edges(ctx, sd, sdt, more):
+    check_batch_build(ctx, [scenes.soup(n, seed=n) for n in EDGES + more], sd, sdt, 3)
