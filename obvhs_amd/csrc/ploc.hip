@@ -288,7 +288,8 @@ __global__ void __launch_bounds__(T256) k_gather_runs(const Node32* __restrict__
     __shared__ uint32_t tk[WIN];
     __shared__ uint32_t rest[WIN];                  // the bits below the top: 31, or 30 of the high word
     __shared__ uint64_t low[WIDE ? WIN : 1];        // the low word of a 126-bit code
-    const uint32_t base = blockIdx.x * T256;
+    const uint32_t base = xcd_tile() * T256;
+    if (base >= n) return;
     // window slot w holds sorted position base - RUN_MAX + w
     const uint32_t w0 = base < RUN_MAX ? RUN_MAX - base : 0u;             // first slot inside the array
     const uint32_t w1 = min(WIN, n - base + RUN_MAX);                     // end of the slots inside it
@@ -1306,9 +1307,9 @@ static obvhs_status sort_gather(obvhs_context* ctx, const Node32* leaves, const 
               "radix sort (top words)");
     const uint32_t nblk = (n + T256 - 1) / T256;
     if (keys_hi)
-        k_gather_runs<true><<<nblk, T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+        k_gather_runs<true><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
     else
-        k_gather_runs<false><<<nblk, T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+        k_gather_runs<false><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
     OBVHS_TRY(hipGetLastError(), "gather launch");
     return OBVHS_OK;
 }
