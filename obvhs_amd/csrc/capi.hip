@@ -84,7 +84,7 @@ obvhs_status obvhs_context_create(int device, void* hip_stream, obvhs_context** 
     }
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev_start);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev_stop);
-    if (e == hipSuccess) e = hipHostMalloc(&ctx->pinned, 4096, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc(&ctx->pinned, PINNED_BYTES, hipHostMallocDefault);
     if (e == hipSuccess) e = upload_log2_table();
     if (e != hipSuccess) {
         obvhs_status s = set_hip_error(ctx, e, "context create");

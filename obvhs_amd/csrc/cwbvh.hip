@@ -33,6 +33,7 @@
 #include "cwdp.hpp"
 #include "device_util.hpp"
 #include "internal.hpp"
+#include "tail.hpp"
 
 namespace obvhs {
 
@@ -40,7 +41,6 @@ namespace {
 
 constexpr int T256 = 256;
 constexpr uint32_t MAX_CW_LEVELS = 64;
-constexpr uint32_t DP_SMALL_RANGE = 4096;  // ranges at most this large are finished by one workgroup
 
 __constant__ uint32_t c_log2_thresh[256];
 
@@ -137,17 +137,66 @@ __global__ void __launch_bounds__(T256) k_dp_range(const Node32* __restrict__ no
     dp_node(nodes, dp, x, &misc->err);
 }
 
-// Cost table of every node in slots [1, hi) -- the small late passes, processed pass by pass inside one
-// workgroup -- and of the root.  hist[p] for p in [p0, passes] bounds the ranges.
-__global__ void __launch_bounds__(1024) k_dp_small(const Node32* __restrict__ nodes, DpView dp,
-                                                   const uint32_t* __restrict__ hist, uint32_t p0,
-                                                   uint32_t passes, CwMisc* misc) {
-    for (uint32_t p = p0; p < passes; ++p) {
-        const uint32_t lo = hist[p + 1], hi = hist[p];
-        for (uint32_t x = lo + threadIdx.x; x < hi; x += 1024) dp_node(nodes, dp, x, &misc->err);
-        __syncthreads();
+// Cost table of the nodes in slots [0, hist[p0]), at most TOP_NODES of them: what is left after the large passes.  One
+// workgroup lists their internal nodes in LDS with their heights above the finished slots (found pass by pass, LDS
+// only) and evaluates the entries by height (tail.hpp).  A chain of entries bounds it: pass by pass, each waiting for
+// the nodes' and then the records' loads, the last 36 passes of 1.29M triangles (from 4,096 slots a pass on) took 404
+// us; now 7 of them are launches of 4 us and the rest take 57 us.  hist[p] for p in [p0, passes] bounds the passes' slots; hist[passes] is 1.
+constexpr uint32_t TOP_NODES = 2048;
+__global__ void __launch_bounds__(1024) k_dp_top(const Node32* __restrict__ nodes, DpView dp,
+                                                 const uint32_t* __restrict__ hist, uint32_t p0, uint32_t passes,
+                                                 CwMisc* misc) {
+    constexpr uint32_t LEAF = 0xffffffffu;
+    __shared__ TailMerges<(int)TOP_NODES> tm;
+    __shared__ uint32_t first[TOP_NODES];
+    __shared__ uint16_t height[TOP_NODES];
+    __shared__ uint32_t bound[TOP_NODES / 2 + 1], wsum[16], s_count;
+    const uint32_t tid = threadIdx.x, top = hist[p0];  // a pass takes two slots at least: fewer than 1,024 passes
+    const uint32_t np = min(passes - p0, TOP_NODES / 2u);
+    for (uint32_t k = tid; k <= np; k += 1024) bound[k] = hist[p0 + k];
+    float ha[2];
+#pragma unroll
+    for (uint32_t k = 0; k < 2u; ++k) {
+        const uint32_t x = tid + k * 1024u;
+        tm.at[x] = 0u;
+        height[x] = 0;
+        if (x < top) {
+            const Node32 nd = load_node(&nodes[x]);
+            first[x] = nd.prim_count == 0u ? nd.first_index : LEAF;
+            ha[k] = half_area(node_box(nd));
+        }
     }
-    if (threadIdx.x == 0) dp_node(nodes, dp, 0u, &misc->err);
+    if (tid == 0) s_count = 0u;
+    lds_barrier();
+    auto raise = [&](uint32_t x) {
+        const uint32_t f = first[x];
+        if (f != LEAF) height[x] = (uint16_t)(1u + (f + 1u < top ? max(height[f], height[f + 1u]) : 0u));
+    };
+    for (uint32_t p = 0; p < np; ++p) {
+        for (uint32_t x = bound[p + 1] + tid; x < bound[p]; x += 1024) raise(x);
+        lds_barrier();
+    }
+    if (tid == 0) raise(0u);
+    lds_barrier();
+#pragma unroll
+    for (uint32_t k = 0; k < 2u; ++k) {
+        const uint32_t x = tid + k * 1024u;
+        const uint32_t f = x < top ? first[x] : LEAF;
+        if (f == LEAF) continue;
+        const Node32 l = load_node(&nodes[f]), r = load_node(&nodes[f + 1]);
+        const uint32_t m = atomicAdd(&s_count, 1u), h = height[x];
+        tm.first[m] = f;
+        tm.lf[m] = l.first_index;
+        tm.rf[m] = r.first_index;
+        tm.ha[m] = ha[k];
+        tm.la[m] = half_area(node_box(l));
+        tm.ra[m] = half_area(node_box(r));
+        tm.h[m] = (uint16_t)(h | min(l.prim_count, 2u) << 12 | min(r.prim_count, 2u) << 14);
+        atomicAdd(&tm.at[h], 1u);
+    }
+    lds_barrier();
+    const uint32_t err = entries_by_height(tm, wsum, s_count, dp);
+    if (err) atomicOr(&misc->err, err);
 }
 
 // exp2(ceil(log2(x))) for x = max(extent, 1e-20) * (1/255) as the reference computes it with libm; returns the
@@ -695,6 +744,27 @@ DpView bvh_dp_view(const obvhs_bvh2* bvh, uint32_t max_prims) {
     return dp_view_at(bvh->dp.as<char>(), k, max_prims);
 }
 
+// The insert indices after each pass of a tree in PLOC pass order (hist[0] = node count ... hist[passes] = 1), read
+// with one synchronisation of the stream; empty if the tree has no such order.
+hipError_t pass_history(obvhs_context* ctx, const obvhs_bvh2* bvh, std::vector<uint32_t>& hist) {
+    hist.clear();
+    hipStream_t st = ctx->stream;
+    const uint32_t passes = bvh->ploc_iterations;
+    if (!bvh->pass_ordered || passes == 0u) return hipStreamSynchronize(st);
+    hist.resize((size_t)passes + 1u);
+    // through the pinned staging area (its first 64 words are the caller's) when they fit
+    const bool small = hist.size() <= PINNED_BYTES / 4 - 64;
+    uint32_t* to = small ? static_cast<uint32_t*>(ctx->pinned) + 64 : hist.data();
+    hipError_t e = hipMemcpyAsync(to, bvh->hist.ptr, hist.size() * 4, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return e;
+    if (small) memcpy(hist.data(), to, hist.size() * 4);
+    bool ordered = hist[0] == bvh->node_count && hist[passes] == 1u;
+    for (uint32_t p = 0; p < passes; ++p) ordered = ordered && hist[p + 1] < hist[p];
+    if (!ordered) hist.clear();
+    return hipSuccess;
+}
+
 obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_prims_per_leaf,
                            bool order_children, obvhs_cwbvh* out) {
     hipStream_t st = ctx->stream;
@@ -709,28 +779,23 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
     const Node32* nodes = bvh2->nodes.as<Node32>();
     k_cw_init<<<1, 64, 0, st>>>(misc);
     uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
-    if (bvh2->dp_max_prims != max_prims_per_leaf && n > 1 && !bvh2->pass_ordered) {
-        // children moved by reinsertion: evaluate the table over the level lists, deepest level first
-        OBVHS_TRY(bvh_dp_alloc(bvh2), "alloc cost table");
-        const obvhs_status ls = cost_table_levels(ctx, bvh2, bvh_dp_view(bvh2, max_prims_per_leaf), &misc->err);
-        if (ls != OBVHS_OK) return ls;
-        bvh2->dp_max_prims = max_prims_per_leaf;
-    }
     if (bvh2->dp_max_prims != max_prims_per_leaf && n > 1) {
         OBVHS_TRY(bvh_dp_alloc(bvh2), "alloc cost table");
         const DpView dpv = bvh_dp_view(bvh2, max_prims_per_leaf);
-        const uint32_t passes = bvh2->ploc_iterations;
-        std::vector<uint32_t> hist(passes + 1);
-        OBVHS_TRY(hipMemcpyAsync(hist.data(), bvh2->hist.ptr, hist.size() * 4, hipMemcpyDeviceToHost, st),
-                  "read pass history");
-        OBVHS_TRY(hipStreamSynchronize(st), "pass history sync");
-        uint32_t p = 0;
-        for (; p < passes; ++p) {
-            const uint32_t lo = hist[p + 1], hi = hist[p];
-            if (hi - lo <= DP_SMALL_RANGE) break;
-            k_dp_range<<<(hi - lo + T256 - 1) / T256, T256, 0, st>>>(nodes, dpv, lo, hi, misc);
+        std::vector<uint32_t> hist;
+        OBVHS_TRY(pass_history(ctx, bvh2, hist), "read pass history");
+        if (hist.empty()) {
+            // children moved by reinsertion: evaluate the table over the level lists, deepest level first
+            const obvhs_status ls = cost_table_levels(ctx, bvh2, dpv, &misc->err);
+            if (ls != OBVHS_OK) return ls;
+        } else {
+            // the first pass emitted leaves only
+            uint32_t p = 1;
+            for (; hist[p] > TOP_NODES; ++p)
+                k_dp_range<<<(hist[p] - hist[p + 1] + T256 - 1) / T256, T256, 0, st>>>(nodes, dpv, hist[p + 1], hist[p],
+                                                                                      misc);
+            k_dp_top<<<1, 1024, 0, st>>>(nodes, dpv, bvh2->hist.as<uint32_t>(), p, (uint32_t)hist.size() - 1u, misc);
         }
-        k_dp_small<<<1, 1024, 0, st>>>(nodes, dpv, bvh2->hist.as<uint32_t>(), p, passes, misc);
         OBVHS_TRY(hipGetLastError(), "cost table launch");
         bvh2->dp_max_prims = max_prims_per_leaf;
     }

@@ -28,6 +28,8 @@ struct DevBuf {
 };
 
 // PLOC per-pass state, double buffered on the device (pass k reads slot k&1, writes slot (k+1)&1).
+constexpr size_t PINNED_BYTES = 4096;
+
 struct PlocState {
     uint32_t count;
     uint32_t insert;
@@ -81,7 +83,7 @@ struct obvhs_context {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     obvhs::BuildScratch scratch;
     obvhs::QualityScratch quality;
-    void* pinned = nullptr;  // small pinned host staging area
+    void* pinned = nullptr;  // pinned host staging area of PINNED_BYTES
     bool keep_trace = false; // keep Morton codes and the sort permutation of each build (parity tests)
     uint32_t trav_lanes = 0;  // persistent traversal grid size (0 = not yet queried)
     void* noalloc_spill = nullptr;  // this device's address of the static traversal scratch (traverse.hip)
@@ -150,6 +152,7 @@ hipError_t bvh_dp_alloc(obvhs_bvh2* bvh);
 DpView bvh_dp_view(const obvhs_bvh2* bvh, uint32_t max_prims);
 
 // cwbvh.hip
+hipError_t pass_history(obvhs_context* ctx, const obvhs_bvh2* bvh, std::vector<uint32_t>& hist);
 obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_prims_per_leaf,
                            bool order_children, obvhs_cwbvh* out);
 struct MeshDesc;

@@ -149,6 +149,38 @@ struct TailMerges {
     uint32_t at[MAX];  // merges per height, then where each height's merges begin
 };
 
+// The cost-table entries of the listed merges, by height: an entry needs only entries of lower height.  tm.at holds the
+// merges per height on entry (after a barrier); MAX / 2 threads, wsum one word per wave.
+template <int MAX>
+__device__ __forceinline__ uint32_t entries_by_height(TailMerges<MAX>& tm, uint32_t* wsum, uint32_t merges,
+                                                      const DpView& dp) {
+    constexpr int THREADS = MAX / 2;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    // The merges in the order of their heights (1 .. top): where each height begins, then the list.
+    const uint32_t c0 = tm.at[2 * tid], c1 = tm.at[2 * tid + 1];
+    const uint32_t incl = wave_inclusive_scan(c0 + c1);
+    if ((tid & 63u) == 63u) wsum[wave] = incl;
+    lds_barrier();
+    uint32_t base = incl - (c0 + c1);
+    for (uint32_t w = 0; w < wave; ++w) base += wsum[w];
+    tm.at[2 * tid] = base;
+    tm.at[2 * tid + 1] = base + c0;
+    lds_barrier();
+    for (uint32_t m = tid; m < merges; m += THREADS)
+        tm.order[atomicAdd(&tm.at[tm.h[m] & 0xfffu], 1u)] = (uint16_t)m;
+    lds_barrier();  // tm.at[h] is now where height h ends
+    uint32_t err = 0u;
+    for (uint32_t h = 1u; tm.at[h - 1] < merges; ++h) {
+        for (uint32_t j = tm.at[h - 1] + tid; j < tm.at[h]; j += THREADS) {
+            const uint32_t m = tm.order[j], c = tm.h[m];
+            err |= dp_evaluate(dp, tm.ha[m], tm.first[m], DpChild{tm.lf[m], c >> 12 & 3u, tm.la[m]},
+                               DpChild{tm.rf[m], c >> 14, tm.ra[m]});
+        }
+        __syncthreads();  // the next height reads this one's entries
+    }
+    return err;
+}
+
 // One merge of the tail: the children a (higher index) and b go to their slots, the merge to the list; returns the
 // parent (and its height in h).  False slots are reported by the result.
 template <int MAX>
@@ -389,27 +421,7 @@ __device__ __forceinline__ void ploc_tail(const Node32* __restrict__ cur, PlocSt
     }
     uint32_t dp_err = 0u;
     if (fused && merges != 0u) {
-        // The merges in the order of their heights (1 .. top): where each height begins, then the list.
-        const uint32_t c0 = tm.at[2 * tid], c1 = tm.at[2 * tid + 1];
-        const uint32_t incl = wave_inclusive_scan(c0 + c1);
-        if ((tid & 63u) == 63u) wsum[wave] = incl;
-        lds_barrier();
-        uint32_t base = incl - (c0 + c1);
-        for (uint32_t w = 0; w < wave; ++w) base += wsum[w];
-        tm.at[2 * tid] = base;
-        tm.at[2 * tid + 1] = base + c0;
-        lds_barrier();
-        for (uint32_t m = tid; m < merges; m += THREADS)
-            tm.order[atomicAdd(&tm.at[tm.h[m] & 0xfffu], 1u)] = (uint16_t)m;
-        lds_barrier();  // tm.at[h] is now where height h ends
-        for (uint32_t h = 1u; tm.at[h - 1] < merges; ++h) {
-            for (uint32_t j = tm.at[h - 1] + tid; j < tm.at[h]; j += THREADS) {
-                const uint32_t m = tm.order[j], c = tm.h[m];
-                dp_err |= dp_evaluate(dp, tm.ha[m], tm.first[m], DpChild{tm.lf[m], c >> 12 & 3u, tm.la[m]},
-                                      DpChild{tm.rf[m], c >> 14, tm.ra[m]});
-            }
-            __syncthreads();  // the next height reads this one's entries
-        }
+        dp_err = entries_by_height(tm, wsum, merges, dp);
     }
     if (self_merge) atomicOr(err, DERR_SELF_MERGE);
     if (bad_slot) atomicOr(err, DERR_CAPACITY);
