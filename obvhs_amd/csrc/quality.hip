@@ -38,8 +38,12 @@ namespace {
 constexpr int T256 = 256;
 constexpr uint32_t LEVELS_PER_SYNC = 16;
 constexpr uint32_t MIS_ROUNDS_PER_SYNC = 8;
-constexpr uint32_t FIND_THREADS = 1u << 19;  // concurrent find_reinsertion lanes (each owns a stack column)
-constexpr uint32_t FIND_REFILL = 32;  // idle lanes of a wave that take new candidates together (16: 0.4 ms slower)
+// Concurrent find_reinsertion lanes (each owns a stack column); 2^19 lanes spread over more of the tree (9.4 ms, not
+// 9.1).
+constexpr uint32_t FIND_THREADS = 1u << 18;
+// Trees of at least this many nodes (32 MB, what the eight L2s hold) have their candidates walked in node order: the
+// sort costs 0.2 ms and spares 1.4 ms of the walks' 10.8 at 34.5M nodes; at 131K nodes it would cost 50 us a step for 2.
+constexpr uint32_t FIND_BY_NODE = 1u << 20;
 constexpr uint32_t FIND_LDS = 8;  // top stack entries in LDS: 16 KB per block, 32 waves per CU (16 entries: 16% slower)
 
 __device__ __forceinline__ uint32_t sibling_of(uint32_t id) { return (id & 1u) ? id + 1u : id - 1u; }
@@ -306,12 +310,17 @@ struct ReinsMisc {
     uint32_t undecided[MIS_ROUNDS_PER_SYNC];
 };
 
-// reinsertion.rs:247-340, one lane per candidate walk, stack column `tid` of an [sd][nthreads] array; a walk's
-// steps are the crate's in the crate's order, one per loop iteration (start, search step, or climb to the next
-// pivot), so lanes of a wave refill with new candidates independently.
+// reinsertion.rs:247-340, one lane per candidate walk, stack column `tid` of an [sd][nthreads] array; the crate's
+// visits in the crate's order.  cand: the candidates, rank (NULL: their order) their places in the results.
+// Random reads of the tree bound it (34.5M nodes: 2 to 3 TB/s, most L2 lines used by few lanes; 24 of 64 lanes active),
+// so a loop iteration makes one round of loads for as much as it can: both children of an expanded node, of which the
+// first is kept as its own children or dropped when its visit can no longer matter by itself, and a climb together with
+// the visit of the new sibling.  34.5M nodes, two steps of 1.7M and 575K candidates: 11.9 ms with a node per iteration
+// and candidates by area, 10.8 with the pairs, 8.8 in node order.  131K nodes, 16 steps: 2.14 -> 1.71 ms.
 __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restrict__ nodes, uint32_t n_nodes,
                                                            const uint32_t* __restrict__ parents,
-                                                           const uint32_t* __restrict__ cand, uint32_t count,
+                                                           const uint32_t* __restrict__ cand,
+                                                           const uint32_t* __restrict__ rank, uint32_t count,
                                                            uint2* __restrict__ stack, uint32_t sd,
                                                            uint32_t* __restrict__ r_from, uint32_t* __restrict__ r_to,
                                                            uint64_t* __restrict__ keys, ReinsMisc* misc) {
@@ -340,22 +349,25 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
         return ring[sp % FIND_LDS][threadIdx.x];
     };
     // Each lane walks one candidate at a time: the grid first takes candidates [0, nthreads) (lane tid the
-    // candidate tid); a lane that finishes waits until FIND_REFILL lanes of its wave are idle (or none is walking),
-    // and the wave then takes that many further candidates from the counter with one atomic.  Lanes walk
-    // independently, so a long walk no longer holds the other 63 lanes idle until it ends.
+    // candidate tid), then every wave whose lanes are all done the next 64 from the counter, with one atomic.  On large
+    // trees cand is in node order, so that a wave's walks read the same parts of the tree; refilling lanes one by one
+    // (from 8, 16, 32 idle lanes on: 11.6, 10.2, 9.1 ms where whole waves take 8.8) mixes distant walks.
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t step_budget = 2u * n_nodes + 64u;  // walks of a valid tree end long before these budgets
     uint32_t t = tid;
     bool done = t >= count, live = !done, fresh = live;
-    uint32_t node_id = 0u, parent_id = 0u, sib = 0u, pivot_id = 0u, best_to = 0u, climb = 0u, steps = 0u;
+    uint32_t node_id = 0u, parent_id = 0u, pivot_id = 0u, best_to = 0u, climb = 0u, steps = 0u;
     float node_area = 0.0f, area_diff = 0.0f, best_area = 0.0f;
     Box aabb{}, pivot_bbox{};
     bool overflow = false, held = false;
     uint2 top = make_uint2(0u, 0u);
+    // `both`: the entry in `top` stands for both children of a node, by the first.  Stack entries mark it in the id's
+    // top bit; with ids that need all 32 bits they stand for one node each.
+    bool both = false;
+    const uint32_t pair_flag = n_nodes <= 1u << 31 ? 1u << 31 : 0u;
     for (;;) {
         const uint64_t want = __ballot(!live && !done);
-        const uint64_t walking = __ballot(live);
-        if (want != 0ull && ((uint32_t)__popcll(want) >= FIND_REFILL || walking == 0ull)) {
+        if (want != 0ull && __ballot(live) == 0ull) {
             const uint32_t leader = (uint32_t)__ffsll((unsigned long long)want) - 1u;
             uint32_t base = 0u;
             if (lane == leader) base = nthreads + atomicAdd(&misc->next, (uint32_t)__popcll(want));
@@ -382,7 +394,7 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
                 node_area = half_area(aabb);
                 parent_id = parents[node_id];
                 area_diff = half_area(node_box(load_node(&nodes[parent_id])));
-                sib = sibling_of(node_id);
+                const uint32_t sib = sibling_of(node_id);
                 pivot_bbox = node_box(load_node(&nodes[sib]));
                 pivot_id = parent_id;
                 overflow = false;
@@ -390,61 +402,87 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
                 steps = 0u;
                 sp = 0;
                 lo = 0;
-                // The second child of an expanded node is the next entry popped, so it is kept in registers
-                // (`held`) instead of pushed and popped: the same visit order without an LDS round trip.
                 top = make_uint2(__float_as_uint(area_diff), sib);
                 held = true;
+                both = false;
             }
-            if (!held && sp == 0) {
-                // this level's search is over: climb to the next pivot (or end the walk)
-                fin = overflow;
-                if (!fin) {
-                    if (pivot_id != parent_id) {
-                        pivot_bbox = box_union(pivot_bbox, node_box(load_node(&nodes[sib])));
-                        area_diff += half_area(node_box(load_node(&nodes[pivot_id]))) - half_area(pivot_bbox);
-                    }
-                    if (pivot_id == 0u) {
-                        fin = true;
-                    } else if (++climb > sd) {
-                        overflow = true;
-                        fin = true;
-                    } else {
-                        sib = sibling_of(pivot_id);
-                        pivot_id = parents[pivot_id];
-                        sp = 0;
-                        lo = 0;
-                        top = make_uint2(__float_as_uint(area_diff), sib);
-                        held = true;
-                    }
-                }
+            // The next entry that can still matter (best_area only grows), or a climb once this level's search is over.
+            while (!held && sp != 0) {
+                top = pop();
+                both = (top.y & pair_flag) != 0u;
+                top.y &= ~pair_flag;
+                held = !(__uint_as_float(top.x) - node_area <= best_area);
+            }
+            bool climbing = false;
+            if (!held) {
+                fin = overflow || pivot_id == 0u;
+                if (!fin && ++climb > sd) overflow = fin = true;
+                climbing = !fin;
             } else if (++steps > step_budget) {
                 overflow = true;  // ends the walk at the next iteration
                 held = false;
-                sp = 0;
-            } else {
-                if (!held) top = pop();
-                held = false;
-                const float top_area = __uint_as_float(top.x);
-                if (!(top_area - node_area <= best_area)) {
-                    const Node32 dst = load_node(&nodes[top.y]);
-                    const Box db = node_box(dst);
-                    const float merged_area = half_area(box_union(db, aabb));
-                    const float reinsert_area = top_area - merged_area;
-                    if (reinsert_area > best_area) {
-                        best_to = top.y;
-                        best_area = reinsert_area;
+                sp = lo = 0;
+            }
+            if (climbing || held) {
+                // One round of loads: the entry's node, or both children of an expanded one; for a climb the pivot's
+                // sibling, its box and its parent.
+                const bool pair = held && both;
+                const uint32_t id = climbing ? sibling_of(pivot_id) : top.y + (pair ? 1u : 0u);
+                uint32_t up = 0u;
+                if (climbing) up = parents[pivot_id];
+                const Node32 p = load_node(&nodes[id]);
+                Node32 s{};  // the first child, or the pivot the climb leaves
+                if (pair || climbing) s = load_node(&nodes[climbing ? pivot_id : id - 1u]);
+                float area = __uint_as_float(top.x);
+                if (climbing) {
+                    if (pivot_id != parent_id) area_diff += half_area(node_box(s)) - half_area(pivot_bbox);
+                    pivot_bbox = box_union(pivot_bbox, node_box(p));  // for the next climb
+                    pivot_id = up;
+                    area = area_diff;
+                }
+                both = true;  // what this visit opens
+                // A node's visit: the move beside it, and the bound its children get.
+                auto visit = [&](const Node32& n, uint32_t n_id, float& reinsert, float& child) {
+                    const Box b = node_box(n);
+                    reinsert = area - half_area(box_union(b, aabb));
+                    if (reinsert > best_area) {
+                        best_to = n_id;
+                        best_area = reinsert;
                     }
-                    const float child_area = reinsert_area + half_area(db);
-                    // children whose bound already fails would fail it when popped (best_area only grows)
-                    if (dst.prim_count == 0u && !(child_area - node_area <= best_area)) {
-                        if (sp + 2 > sd) {
-                            overflow = true;
-                            held = false;
-                            sp = 0;
-                        } else {
-                            push(make_uint2(__float_as_uint(child_area), dst.first_index));
-                            top = make_uint2(__float_as_uint(child_area), dst.first_index + 1u);
-                            held = true;
+                    child = reinsert + half_area(b);
+                };
+                float reinsert, child;
+                bool open = false;
+                if (!(area - node_area <= best_area)) {
+                    visit(p, id, reinsert, child);
+                    // children whose bound already fails would fail it when popped
+                    open = p.prim_count == 0u && !(child - node_area <= best_area);
+                    if (open) top = make_uint2(__float_as_uint(child), p.first_index);
+                }
+                held = open;
+                if (pair && !(area - node_area <= best_area)) {
+                    if (!open) {
+                        visit(s, id - 1u, reinsert, child);
+                        held = s.prim_count == 0u && !(child - node_area <= best_area);
+                        if (held) top = make_uint2(__float_as_uint(child), s.first_index);
+                    } else {
+                        // The first child's turn comes after the second one's subtree: kept as its own children (when
+                        // the move beside it is no better than the best already), as itself, or not at all.
+                        const Box b = node_box(s);
+                        reinsert = area - half_area(box_union(b, aabb));
+                        child = reinsert + half_area(b);
+                        const bool better = reinsert > best_area;
+                        const bool inner = s.prim_count == 0u && !(child - node_area <= best_area);
+                        if (better || inner) {
+                            if (sp + 2 > sd) {
+                                overflow = true;
+                                held = false;
+                                sp = lo = 0;
+                            } else {
+                                push(!better && child <= area && pair_flag != 0u
+                                         ? make_uint2(__float_as_uint(child), s.first_index | pair_flag)
+                                         : make_uint2(__float_as_uint(area), id - 1u));
+                            }
                         }
                     }
                 }
@@ -459,10 +497,11 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
                 best_to = 0u;
                 best_area = 0.0f;
             }
-            r_from[t] = from;
-            r_to[t] = best_to;
+            const uint32_t at = rank ? rank[t] : t;
+            r_from[at] = from;
+            r_to[at] = best_to;
             pos = best_area > 0.0f;
-            keys[t] = pos ? (uint64_t)(~f32_order_key(best_area)) : 0xffffffffull;
+            keys[at] = pos ? (uint64_t)(~f32_order_key(best_area)) : 0xffffffffull;
             live = false;
         }
         const uint64_t m = __ballot(pos);
@@ -1758,7 +1797,20 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
         OBVHS_TRY(radix_sort_pairs(Q.keys.as<uint64_t>(), Q.vals.as<uint32_t>(), true, ncand, 32,
                                    Q.sort_scratch.ptr, st, sort_items_for(ctx, ncand)),
                   "candidate sort");
-        k_find_reinsertion<<<fthreads / T256, T256, 0, st>>>(nodes, N, parents, Q.vals.as<uint32_t>(), count,
+        const uint32_t* cand = Q.vals.as<uint32_t>();
+        const uint32_t* rank = nullptr;
+        if (N >= FIND_BY_NODE) {
+            uint32_t* by_node = Q.keys.as<uint32_t>();  // the candidate keys are done with
+            OBVHS_TRY(hipMemcpyAsync(by_node, cand, (size_t)count * 4, hipMemcpyDeviceToDevice, st), "copy candidates");
+            int bits = 1;
+            while (bits < 32 && (N >> bits) != 0u) ++bits;
+            OBVHS_TRY(radix_sort_pairs32(by_node, by_node + count, true, count, bits, Q.sort_scratch.ptr, st,
+                                         sort_items_for(ctx, count)),
+                      "candidate order");
+            cand = by_node;
+            rank = by_node + count;
+        }
+        k_find_reinsertion<<<fthreads / T256, T256, 0, st>>>(nodes, N, parents, cand, rank, count,
                                                               Q.stack.as<uint2>(), sd, Q.rfrom.as<uint32_t>(),
                                                               Q.rto.as<uint32_t>(), Q.rkeys.as<uint64_t>(), misc);
         OBVHS_TRY(hipGetLastError(), "find reinsertion launch");
