@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(T256) k_parents(const Node32* __restrict__ nod
 
 // reinsertion.rs:128-147 + 210-218: key of node i (1 <= i < take) is the crate's radix key of -half_area.
 __global__ void __launch_bounds__(T256) k_cand_keys(const Node32* __restrict__ nodes, uint32_t take,
-                                                    uint64_t* __restrict__ keys) {
+                                                    uint32_t* __restrict__ keys) {
     const uint32_t i = blockIdx.x * T256 + threadIdx.x + 1u;
     if (i >= take) return;
     keys[i - 1] = f32_order_key(-half_area(node_box(load_node(&nodes[i]))));
@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
                                                            const uint32_t* __restrict__ rank, uint32_t count,
                                                            uint2* __restrict__ stack, uint32_t sd,
                                                            uint32_t* __restrict__ r_from, uint32_t* __restrict__ r_to,
-                                                           uint64_t* __restrict__ keys, ReinsMisc* misc) {
+                                                           uint32_t* __restrict__ keys, ReinsMisc* misc) {
     // The DFS stack of each lane: its top FIND_LDS entries in an LDS ring, older entries in the lane's HBM column
     // (entry k at stack[k * nthreads + tid]).  Entries [lo, sp) are in the ring, [0, lo) in HBM: a push into a full
     // ring first writes the ring's oldest entry out (off the walk's critical path), a pop of an empty ring reads
@@ -501,7 +501,7 @@ __global__ void __launch_bounds__(T256) k_find_reinsertion(const Node32* __restr
             r_from[at] = from;
             r_to[at] = best_to;
             pos = best_area > 0.0f;
-            keys[at] = pos ? (uint64_t)(~f32_order_key(best_area)) : 0xffffffffull;
+            keys[at] = pos ? ~f32_order_key(best_area) : 0xffffffffu;
             live = false;
         }
         const uint64_t m = __ballot(pos);
@@ -1777,7 +1777,7 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
         if (count == 0) continue;
         OBVHS_TRY(Q.keys.ensure((size_t)ncand * 8), "alloc candidate keys");
         OBVHS_TRY(Q.vals.ensure((size_t)ncand * 4), "alloc candidate values");
-        OBVHS_TRY(Q.rkeys.ensure((size_t)count * 8), "alloc reinsertion keys");
+        OBVHS_TRY(Q.rkeys.ensure((size_t)count * 4), "alloc reinsertion keys");
         OBVHS_TRY(Q.rvals.ensure((size_t)count * 4), "alloc reinsertion order");
         OBVHS_TRY(Q.rfrom.ensure((size_t)count * 4), "alloc reinsertion from");
         OBVHS_TRY(Q.rto.ensure((size_t)count * 4), "alloc reinsertion to");
@@ -1792,10 +1792,10 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
 
         k_fill_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(misc), 0u, sizeof(ReinsMisc) / 4);
         k_parents<<<nblk, T256, 0, st>>>(nodes, N, parents, &misc->negzero);
-        k_cand_keys<<<(ncand + T256 - 1) / T256, T256, 0, st>>>(nodes, take, Q.keys.as<uint64_t>());
+        k_cand_keys<<<(ncand + T256 - 1) / T256, T256, 0, st>>>(nodes, take, Q.keys.as<uint32_t>());
         OBVHS_TRY(hipGetLastError(), "candidate launch");
-        OBVHS_TRY(radix_sort_pairs(Q.keys.as<uint64_t>(), Q.vals.as<uint32_t>(), true, ncand, 32,
-                                   Q.sort_scratch.ptr, st, sort_items_for(ctx, ncand)),
+        OBVHS_TRY(radix_sort_pairs32(Q.keys.as<uint32_t>(), Q.vals.as<uint32_t>(), true, ncand, 32,
+                                     Q.sort_scratch.ptr, st, sort_items_for(ctx, ncand)),
                   "candidate sort");
         const uint32_t* cand = Q.vals.as<uint32_t>();
         const uint32_t* rank = nullptr;
@@ -1812,10 +1812,10 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
         }
         k_find_reinsertion<<<fthreads / T256, T256, 0, st>>>(nodes, N, parents, cand, rank, count,
                                                               Q.stack.as<uint2>(), sd, Q.rfrom.as<uint32_t>(),
-                                                              Q.rto.as<uint32_t>(), Q.rkeys.as<uint64_t>(), misc);
+                                                              Q.rto.as<uint32_t>(), Q.rkeys.as<uint32_t>(), misc);
         OBVHS_TRY(hipGetLastError(), "find reinsertion launch");
-        OBVHS_TRY(radix_sort_pairs(Q.rkeys.as<uint64_t>(), Q.rvals.as<uint32_t>(), true, count, 32,
-                                   Q.sort_scratch.ptr, st, sort_items_for(ctx, count)),
+        OBVHS_TRY(radix_sort_pairs32(Q.rkeys.as<uint32_t>(), Q.rvals.as<uint32_t>(), true, count, 32,
+                                     Q.sort_scratch.ptr, st, sort_items_for(ctx, count)),
                   "reinsertion sort");
         OBVHS_TRY(hipMemcpyAsync(h, misc, 12, hipMemcpyDeviceToHost, st), "read reinsertion count");
         OBVHS_TRY(hipStreamSynchronize(st), "reinsertion count sync");

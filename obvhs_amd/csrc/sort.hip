@@ -12,6 +12,9 @@
 //               ranking (eight 64-lane ballots per item) gives each key its stable rank inside the tile; the tile's
 //               keys are reordered in LDS and written out coalesced per digit run, then its values through the same
 //               LDS (half the LDS of staging both at once, so twice the tiles per CU).
+// Up to FEW_TILES tiles the scan has no launch: the upsweep writes counts[tile][digit] and every tile of the downsweep
+// sums the digits' counts itself.  A sort of 26K keys (13 tiles) was 12 launches of 5 to 8 us, bound by latency; 32 such
+// sorts of a reinsertion: 2.0 -> 1.5 ms.  At 49 tiles both forms take 55 us a sort.
 // Tiles are 256 threads x ITEMS keys (ITEMS = 4, 8 or 16, the sort tile the context's tuning table picks per size
 // class; 8 by default); each wave owns a contiguous 64 x ITEMS key segment.  Every tile size gives the same order.
 //
@@ -29,7 +32,9 @@ constexpr int SORT_THREADS = 256;
 constexpr int SORT_MIN_ITEMS = 4;  // the scratch is sized for the smallest tile (the most tiles)
 constexpr int SORT_WAVES = SORT_THREADS / 64;
 
-template <class K, int ITEMS>
+constexpr uint32_t FEW_TILES = 64;
+
+template <class K, int ITEMS, bool FEW>
 __global__ void __launch_bounds__(SORT_THREADS)
     k_radix_upsweep(const K* __restrict__ keys, uint32_t n, uint32_t shift, uint32_t num_tiles,
                     uint32_t* __restrict__ counts) {
@@ -48,7 +53,8 @@ __global__ void __launch_bounds__(SORT_THREADS)
         }
     }
     __syncthreads();
-    counts[tid * num_tiles + blockIdx.x] = hist[tid];
+    if (FEW) counts[blockIdx.x * 256u + tid] = hist[tid];
+    else counts[tid * num_tiles + blockIdx.x] = hist[tid];
 }
 
 // Exclusive scans over the 256 threads of two u32 values at once (wave scans, then the four wave totals through
@@ -100,7 +106,8 @@ __global__ void __launch_bounds__(SORT_THREADS)
     if (tid == 0) totals[d] = carry;
 }
 
-template <class K, int ITEMS>
+// offsets: the digits' scanned counts, with their totals; FEW: the counts themselves.
+template <class K, int ITEMS, bool FEW>
 __global__ void __launch_bounds__(SORT_THREADS)
     k_radix_downsweep(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
                       K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n, uint32_t shift,
@@ -122,7 +129,18 @@ __global__ void __launch_bounds__(SORT_THREADS)
 
 #pragma unroll
     for (int w = 0; w < SORT_WAVES; ++w) whist[w][tid] = 0u;
-    const uint32_t dtotal = totals[tid], toff = offsets[(size_t)tid * num_tiles + tile];
+    uint32_t dtotal = 0u, toff = 0u;
+    if (FEW) {
+#pragma unroll 8
+        for (uint32_t t = 0; t < num_tiles; ++t) {
+            const uint32_t c = offsets[t * 256u + tid];
+            dtotal += c;
+            toff += t < tile ? c : 0u;
+        }
+    } else {
+        dtotal = totals[tid];
+        toff = offsets[(size_t)tid * num_tiles + tile];
+    }
     __syncthreads();
 
     const uint32_t seg = tile_base + wave * (64 * ITEMS);
@@ -236,11 +254,17 @@ static hipError_t radix_sort_impl(K* keys, uint32_t* values, bool values_identit
     uint32_t* vout = valt;
     for (int pass = 0; pass < passes; ++pass) {
         uint32_t shift = (uint32_t)(pass * 8);
-        k_radix_upsweep<K, ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, n, shift, tiles, counts);
-        k_radix_scan<<<256, SORT_THREADS, 0, stream>>>(counts, totals, tiles);
         const uint32_t* vsrc = (pass == 0 && values_identity) ? nullptr : vin;
-        k_radix_downsweep<K, ITEMS><<<tiles, SORT_THREADS, 0, stream>>>(kin, vsrc, kout, vout, n, shift, counts,
-                                                                        totals, tiles);
+        if (tiles <= FEW_TILES) {
+            k_radix_upsweep<K, ITEMS, true><<<tiles, SORT_THREADS, 0, stream>>>(kin, n, shift, tiles, counts);
+            k_radix_downsweep<K, ITEMS, true><<<tiles, SORT_THREADS, 0, stream>>>(kin, vsrc, kout, vout, n, shift,
+                                                                                  counts, totals, tiles);
+        } else {
+            k_radix_upsweep<K, ITEMS, false><<<tiles, SORT_THREADS, 0, stream>>>(kin, n, shift, tiles, counts);
+            k_radix_scan<<<256, SORT_THREADS, 0, stream>>>(counts, totals, tiles);
+            k_radix_downsweep<K, ITEMS, false><<<tiles, SORT_THREADS, 0, stream>>>(kin, vsrc, kout, vout, n, shift,
+                                                                                   counts, totals, tiles);
+        }
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
