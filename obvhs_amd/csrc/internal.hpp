@@ -60,14 +60,14 @@ constexpr uint32_t MAX_TREE_LEVELS = 8192;
 
 // Working memory of the tree utilities and quality passes (quality.hip).
 struct QualityScratch {
-    DevBuf level_list, level_meta;                                   // levels
+    DevBuf level_list, level_meta, depth_meta;                       // levels
     DevBuf parents, owner, touched, misc;                            // reinsertion state
     DevBuf keys, vals, rkeys, rvals, rfrom, rto, conf, state, stack;  // candidates / reinsertions
     DevBuf sort_scratch;
     DevBuf split_aabbs, split_indices, ha, cand_a, cand_b, halves, flags, sums;  // pre-splits
     DevBuf marks, kept, freed;                                                   // rebuilds
     void release_all() {
-        for (DevBuf* d : {&level_list, &level_meta, &parents, &owner, &touched, &misc, &keys, &vals, &rkeys, &rvals,
+        for (DevBuf* d : {&level_list, &level_meta, &depth_meta, &parents, &owner, &touched, &misc, &keys, &vals, &rkeys, &rvals,
                           &rfrom, &rto, &conf, &state, &stack, &sort_scratch, &split_aabbs, &split_indices, &ha,
                           &cand_a, &cand_b, &halves, &flags, &sums, &marks, &kept, &freed})
             d->release();

@@ -21,6 +21,7 @@
 //                  triangle order by one wave, as the crate sums it); per iteration every candidate's best of 11
 //                  split planes in parallel, appended right halves numbered by an order-preserving scan, the
 //                  candidate list extended and filtered in order.
+#include <stddef.h>
 #include <string.h>
 
 #include <algorithm>
@@ -44,6 +45,11 @@ constexpr uint32_t FIND_THREADS = 1u << 18;
 // Trees of at least this many nodes (32 MB, what the eight L2s hold) have their candidates walked in node order: the
 // sort costs 0.2 ms and spares 1.4 ms of the walks' 10.8 at 34.5M nodes; at 131K nodes it would cost 50 us a step for 2.
 constexpr uint32_t FIND_BY_NODE = 1u << 20;
+// Levels of a reinsertion's tree: trees of fewer nodes than DEPTH_WALK_NODES (what the L2s hold: a walk reads a parent
+// per level and node) find them by k_depths while no node is MAX_WALK deep.  From the root down a level costs 5 us, and
+// reading the counts 20 us for 16 levels, at any size.
+constexpr uint32_t DEPTH_WALK_NODES = 1u << 20;
+constexpr uint32_t MAX_WALK = 512;
 constexpr uint32_t FIND_LDS = 8;  // top stack entries in LDS: 16 KB per block, 32 waves per CU (16 entries: 16% slower)
 
 __device__ __forceinline__ uint32_t sibling_of(uint32_t id) { return (id & 1u) ? id + 1u : id - 1u; }
@@ -155,6 +161,38 @@ __global__ void __launch_bounds__(T256) k_refit_level(Node32* __restrict__ nodes
     const Box u =
         box_union(node_box(load_node(&nodes[nd.first_index])), node_box(load_node(&nodes[nd.first_index + 1])));
     store_node(&nodes[x], make_node(u, 0u, nd.first_index));
+}
+
+// Consecutive levels [lo, hi] of at most REFIT_RUN nodes each by one workgroup, deepest first; the next level's nodes are
+// loaded beside this one's children.  A launch of such a level waits 3 us for its three dependent loads and as long for
+// the next launch; a level here takes 1.3 us.
+constexpr uint32_t REFIT_RUN = 1024;
+__global__ void __launch_bounds__(REFIT_RUN) k_refit_run(Node32* __restrict__ nodes, const uint32_t* __restrict__ list,
+                                                         const uint32_t* __restrict__ meta, uint32_t lo, uint32_t hi) {
+    constexpr uint32_t NONE = 0xffffffffu;
+    uint32_t x, first;
+    auto fetch = [&](uint32_t level) {  // the thread's node; its first child, NONE for a leaf
+        const uint32_t s = meta[2 * level], c = meta[2 * level + 1];
+        x = threadIdx.x < c ? list[s + threadIdx.x] : NONE;
+        first = NONE;
+        if (x != NONE) {
+            const Node32 nd = load_node(&nodes[x]);
+            if (nd.prim_count == 0u) first = nd.first_index;
+        }
+    };
+    fetch(hi);
+    for (uint32_t level = hi;; --level) {
+        const uint32_t node = x, child = first;
+        Node32 l{}, r{};
+        if (child != NONE) {
+            l = load_node(&nodes[child]);
+            r = load_node(&nodes[child + 1]);
+        }
+        if (level > lo) fetch(level - 1);
+        if (child != NONE) store_node(&nodes[node], make_node(box_union(node_box(l), node_box(r)), 0u, child));
+        if (level == lo) break;
+        __syncthreads();  // the boxes just written are the next level's children
+    }
 }
 
 // The same for the slots [lo, hi) a PLOC pass emitted: their children were emitted by earlier passes.
@@ -292,6 +330,73 @@ __global__ void __launch_bounds__(T256) k_parents(const Node32* __restrict__ nod
             __float_as_uint(nd.maxx) == nz || __float_as_uint(nd.maxy) == nz || __float_as_uint(nd.maxz) == nz)
             atomicOr(negzero, 1u);
     }
+}
+
+// Level lists of a small tree from its parents: every node walks up to the root (in parallel, so the tree's depth in
+// loads), then the inner nodes are placed by their depth.  131K nodes of 48 levels: 24 us, against 230 us for 48
+// launches from the root down (k_levels_expand) and the reads between them.
+struct DepthMeta {
+    uint32_t count[MAX_WALK];   // inner nodes per depth
+    uint32_t deepest;           // greatest depth of a node; MAX_WALK: some node is deeper than the walk goes
+    uint32_t pad;
+    uint32_t placed[MAX_WALK];
+};
+
+__global__ void __launch_bounds__(T256) k_depths(const Node32* __restrict__ nodes, uint32_t n,
+                                                 const uint32_t* __restrict__ parents, uint16_t* __restrict__ depths,
+                                                 DepthMeta* __restrict__ dm) {
+    __shared__ uint32_t count[MAX_WALK];
+    __shared__ uint32_t deepest;
+    for (uint32_t k = threadIdx.x; k < MAX_WALK; k += T256) count[k] = 0u;
+    if (threadIdx.x == 0) deepest = 0u;
+    __syncthreads();
+    const uint32_t i = blockIdx.x * T256 + threadIdx.x;
+    if (i < n) {
+        const bool inner = load_node(&nodes[i]).prim_count == 0u;
+        uint32_t d = 0u;
+        for (uint32_t x = i; x != 0u && d < MAX_WALK; ++d) x = parents[x];
+        if (inner && d < MAX_WALK) atomicAdd(&count[d], 1u);
+        atomicMax(&deepest, d);
+        depths[i] = (uint16_t)(inner ? d : MAX_WALK);
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < MAX_WALK; k += T256)
+        if (count[k] != 0u) atomicAdd(&dm->count[k], count[k]);
+    if (threadIdx.x == 0) atomicMax(&dm->deepest, deepest);
+}
+
+// meta: start and count of each depth's list, as k_levels_expand leaves them.
+__global__ void __launch_bounds__(T256) k_place_by_depth(const uint16_t* __restrict__ depths, uint32_t n,
+                                                         DepthMeta* __restrict__ dm, uint32_t* __restrict__ list,
+                                                         uint32_t* __restrict__ meta) {
+    static_assert(MAX_WALK == 2 * T256, "two depths per thread");
+    __shared__ uint32_t start[MAX_WALK], mine[MAX_WALK], wsum[T256 / 64];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    if (dm->deepest >= MAX_WALK) return;  // uniform: depths beyond the walk have no place
+    const uint32_t c0 = dm->count[2 * tid], c1 = dm->count[2 * tid + 1];
+    const uint32_t incl = wave_inclusive_scan(c0 + c1);
+    if ((tid & 63u) == 63u) wsum[wave] = incl;
+    mine[2 * tid] = mine[2 * tid + 1] = 0u;
+    __syncthreads();
+    uint32_t before = incl - (c0 + c1);
+    for (uint32_t w = 0; w < wave; ++w) before += wsum[w];
+    start[2 * tid] = before;
+    start[2 * tid + 1] = before + c0;
+    if (blockIdx.x == 0) {
+        meta[4 * tid] = before;
+        meta[4 * tid + 1] = c0;
+        meta[4 * tid + 2] = before + c0;
+        meta[4 * tid + 3] = c1;
+    }
+    const uint32_t i = blockIdx.x * T256 + tid;
+    const uint32_t d = i < n ? depths[i] : MAX_WALK;
+    uint32_t rank = 0u;
+    if (d < MAX_WALK) rank = atomicAdd(&mine[d], 1u);
+    __syncthreads();
+    for (uint32_t k = tid; k < MAX_WALK; k += T256)
+        if (mine[k] != 0u) start[k] += atomicAdd(&dm->placed[k], mine[k]);
+    __syncthreads();
+    if (d < MAX_WALK && start[d] + rank < (n - 1u) / 2u) list[start[d] + rank] = i;  // the depths begin there
 }
 
 // reinsertion.rs:128-147 + 210-218: key of node i (1 <= i < take) is the crate's radix key of -half_area.
@@ -1490,6 +1595,45 @@ obvhs_status tree_levels(obvhs_context* ctx, obvhs_bvh2* bvh, std::vector<uint32
     return OBVHS_OK;
 }
 
+// The level lists of a reinsertion's tree, inner nodes only, from its parents (k_depths); by tree_levels if it is large
+// or deep.
+static obvhs_status walked_levels(obvhs_context* ctx, obvhs_bvh2* bvh, std::vector<uint32_t>& meta_host,
+                                  uint32_t& levels) {
+    const uint32_t N = bvh->node_count;
+    if (N >= DEPTH_WALK_NODES || N < 3u) return tree_levels(ctx, bvh, meta_host, levels, nullptr);
+    hipStream_t st = ctx->stream;
+    QualityScratch& Q = ctx->quality;
+    OBVHS_TRY(Q.level_list.ensure((size_t)N * 4), "alloc level list");
+    OBVHS_TRY(Q.level_meta.ensure((size_t)(2 * (MAX_TREE_LEVELS + 2) + 1) * 4), "alloc level meta");
+    OBVHS_TRY(Q.depth_meta.ensure(sizeof(DepthMeta)), "alloc depth meta");
+    uint32_t* list = Q.level_list.as<uint32_t>();  // (N - 1) / 2 inner nodes, then the depths
+    uint16_t* depths = reinterpret_cast<uint16_t*>(list + (N - 1) / 2);
+    DepthMeta* dm = Q.depth_meta.as<DepthMeta>();
+    const Node32* nodes = bvh->nodes.as<Node32>();
+    const uint32_t nblk = (N + T256 - 1) / T256;
+    k_fill_u32<<<4, T256, 0, st>>>(reinterpret_cast<uint32_t*>(dm), 0u, sizeof(DepthMeta) / 4);
+    k_parents<<<nblk, T256, 0, st>>>(nodes, N, Q.parents.as<uint32_t>(), nullptr);
+    k_depths<<<nblk, T256, 0, st>>>(nodes, N, Q.parents.as<uint32_t>(), depths, dm);
+    k_place_by_depth<<<nblk, T256, 0, st>>>(depths, N, dm, list, Q.level_meta.as<uint32_t>());
+    OBVHS_TRY(hipGetLastError(), "levels launch");
+    uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
+    static_assert(offsetof(DepthMeta, placed) <= PINNED_BYTES, "the counts fit the staging area");
+    OBVHS_TRY(hipMemcpyAsync(h, dm, offsetof(DepthMeta, placed), hipMemcpyDeviceToHost, st), "read levels");
+    OBVHS_TRY(hipStreamSynchronize(st), "levels sync");
+    const uint32_t deepest = h[MAX_WALK];
+    if (deepest >= MAX_WALK) return tree_levels(ctx, bvh, meta_host, levels, nullptr);
+    levels = deepest + 1u;
+    meta_host.resize(2 * (size_t)levels);
+    uint32_t at = 0;
+    for (uint32_t l = 0; l < levels; ++l) {
+        meta_host[2 * l] = at;
+        meta_host[2 * l + 1] = h[l];
+        at += h[l];
+    }
+    if (2u * at + 1u != N) return OBVHS_ERR_CAPACITY;  // not a tree
+    return OBVHS_OK;
+}
+
 static obvhs_status refit_levels(obvhs_context* ctx, obvhs_bvh2* bvh, const std::vector<uint32_t>& meta,
                                  uint32_t levels) {
     hipStream_t st = ctx->stream;
@@ -1497,6 +1641,13 @@ static obvhs_status refit_levels(obvhs_context* ctx, obvhs_bvh2* bvh, const std:
     Node32* nodes = bvh->nodes.as<Node32>();
     for (uint32_t l = levels; l-- > 0;) {
         const uint32_t s = meta[2 * l], c = meta[2 * l + 1];
+        if (c == 0u) continue;
+        if (c <= REFIT_RUN) {
+            const uint32_t hi = l;
+            while (l > 0 && meta[2 * (l - 1) + 1] <= REFIT_RUN) --l;
+            k_refit_run<<<1, REFIT_RUN, 0, st>>>(nodes, list, ctx->quality.level_meta.as<uint32_t>(), l, hi);
+            continue;
+        }
         k_refit_level<<<(c + T256 - 1) / T256, T256, 0, st>>>(nodes, list, s, c);
     }
     OBVHS_TRY(hipGetLastError(), "refit launch");
@@ -1854,7 +2005,7 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
             k_reins_apply<<<pblk, T256, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, nodes);
         }
         OBVHS_TRY(hipGetLastError(), "apply launch");
-        s = tree_levels(ctx, bvh, meta, levels, nullptr);
+        s = walked_levels(ctx, bvh, meta, levels);
         if (s != OBVHS_OK) return s;
         have_levels = true;
         refit_pending = !replay;
@@ -1869,6 +2020,7 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
         k_fill_u32<<<1, 64, 0, st>>>(&misc->err, 0u, 1);
         for (uint32_t l = levels; l-- > 0;) {
             const uint32_t b = meta[2 * l], c = meta[2 * l + 1];
+            if (c == 0u) continue;
             if (refit_pending)
                 k_refit_dp_level<true><<<(c + T256 - 1) / T256, T256, 0, st>>>(nodes, dp, Q.level_list.as<uint32_t>(),
                                                                               b, c, &misc->err);
