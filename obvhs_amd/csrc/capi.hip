@@ -207,7 +207,7 @@ obvhs_status obvhs_timer_stop(obvhs_context* ctx, float* ms) {
 static obvhs_status ploc_entry(obvhs_context* ctx, const obvhs_triangle* d_tris, const obvhs_aabb* d_aabbs,
                                const uint32_t* d_indices, uint32_t n, uint32_t search_distance,
                                uint32_t sort_precision, uint32_t search_depth_threshold, uint32_t fused_max_prims,
-                               obvhs_bvh2* reuse, obvhs_bvh2** out) {
+                               obvhs_bvh2* reuse, obvhs_bvh2** out, CwRootInfo* info = nullptr) {
     if (!ctx || !out) return OBVHS_ERR_INVALID_ARG;
     if (n > 0 && !d_tris && !d_aabbs) return OBVHS_ERR_INVALID_ARG;
     if (n >= (1u << 31)) return OBVHS_ERR_INVALID_ARG;
@@ -217,7 +217,7 @@ static obvhs_status ploc_entry(obvhs_context* ctx, const obvhs_triangle* d_tris,
     obvhs_bvh2* bvh = reuse ? reuse : new (std::nothrow) obvhs_bvh2();
     if (!bvh) return OBVHS_ERR_OOM;
     obvhs_status s = ploc_build(ctx, d_tris, d_aabbs, d_indices, n, search_distance, sort_precision == 128u,
-                                search_depth_threshold, fused_max_prims, bvh);
+                                search_depth_threshold, fused_max_prims, bvh, info);
     if (s != OBVHS_OK) {
         if (!reuse) obvhs_bvh2_destroy(bvh);
         *out = nullptr;
@@ -358,6 +358,8 @@ obvhs_status obvhs_build_cwbvh_from_tris_ex(obvhs_context* ctx, const obvhs_tria
     const bool reinsert = params->reinsertion_batch_ratio > 0.0f;
     // Without reinsertion the cost table of the conversion is evaluated by the PLOC merges themselves.
     const uint32_t fused = reinsert ? 0u : mp;
+    CwRootInfo info{};  // then the build's last read brings what the conversion would read
+    CwRootInfo* const root = fused && n > 0 ? &info : nullptr;
     obvhs_status s;
     if (params->pre_split && n > 0) {  // cwbvh/builder.rs:26-55
         uint32_t n_split = 0;
@@ -365,16 +367,16 @@ obvhs_status obvhs_build_cwbvh_from_tris_ex(obvhs_context* ctx, const obvhs_tria
         if (s == OBVHS_OK)
             s = ploc_entry(ctx, nullptr, ctx->quality.split_aabbs.as<obvhs_aabb>(),
                            ctx->quality.split_indices.as<uint32_t>(), n_split, params->ploc_search_distance,
-                           params->sort_precision, params->search_depth_threshold, fused, b2, &b2);
+                           params->sort_precision, params->search_depth_threshold, fused, b2, &b2, root);
     } else {
         s = ploc_entry(ctx, d_tris, nullptr, nullptr, n, params->ploc_search_distance, params->sort_precision,
-                       params->search_depth_threshold, fused, b2, &b2);
+                       params->search_depth_threshold, fused, b2, &b2, root);
     }
     if (s == OBVHS_OK) cw->owned_bvh2 = b2;
     if (s == OBVHS_OK && reinsert)  // cwbvh/builder.rs:73
         s = bvh2_reinsertion(ctx, b2, params->reinsertion_batch_ratio, ext ? ext->ratio_sequence : nullptr,
                              ext ? ext->ratio_sequence_len : 0u, mp);
-    if (s == OBVHS_OK) s = cwbvh_convert(ctx, b2, mp, true, cw);
+    if (s == OBVHS_OK) s = cwbvh_convert(ctx, b2, mp, true, cw, root);
     if (s != OBVHS_OK) {
         if (!reuse) obvhs_cwbvh_destroy(cw);
         *out = nullptr;

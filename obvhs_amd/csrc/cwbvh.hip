@@ -24,6 +24,7 @@
 // a 256-entry table of per-exponent mantissa thresholds, generated from that same log2f when the context is
 // created, reproduces it with integer compares.
 #include <math.h>
+#include <stddef.h>
 #include <string.h>
 
 #include <algorithm>
@@ -66,7 +67,7 @@ struct CwPre {
 struct CwMisc {
     uint32_t err;
     uint32_t level_count[MAX_CW_LEVELS + 1];
-    uint32_t info[10];  // k_cw_info: the BVH2 root (8 words), the CWBVH node count and depth
+    CwRootInfo info;    // k_cw_info
     CwItem root_item;   // level 0 of a single conversion
     CwPre root_pre;
 };
@@ -92,29 +93,15 @@ __device__ __forceinline__ CwPre pre_of(const Node32* __restrict__ nds, const Dp
     return p;
 }
 
-// What the host needs before the emit, gathered so that one copy brings it with the error word: the BVH2 root, and
-// the size and depth of the CWBVH subtree it roots (1 and 1 for a single-leaf BVH2).
-__global__ void k_cw_info(const Node32* __restrict__ nodes, DpView dp, CwMisc* misc) {
-    if (threadIdx.x != 0) return;
-    const Node32 root = load_node(&nodes[0]);
-    const uint4* w = reinterpret_cast<const uint4*>(&root);
-    const uint4 a = w[0], b = w[1];
-    misc->info[0] = a.x;
-    misc->info[1] = a.y;
-    misc->info[2] = a.z;
-    misc->info[3] = a.w;
-    misc->info[4] = b.x;
-    misc->info[5] = b.y;
-    misc->info[6] = b.z;
-    misc->info[7] = b.w;
-    uint32_t size = 1u, depth = 1u;
-    if (root.prim_count == 0u) {
-        const DpRec& e = dp.rec[dkey(root.first_index)];
-        size = e.cwsize;
-        depth = e.cwdepth;
+// What the host needs before the emit, gathered so that one copy brings it with the error word, and level 0 of the
+// emit.  init: the error word and the level counts start here (nothing ran before the emit).
+__global__ void k_cw_info(const Node32* __restrict__ nodes, DpView dp, CwMisc* misc, uint32_t init) {
+    if (init) {
+        if (threadIdx.x == 0) misc->err = 0u;
+        for (uint32_t l = threadIdx.x; l <= MAX_CW_LEVELS; l += 64) misc->level_count[l] = l == 0u ? 1u : 0u;
     }
-    misc->info[8] = size;
-    misc->info[9] = depth;
+    if (threadIdx.x != 0) return;
+    misc->info = root_info(nodes, dp);
     misc->root_item = CwItem{0u, 0u, 0u, 0u, 0u};
     misc->root_pre = pre_of(nodes, dp, 0u);
 }
@@ -766,7 +753,7 @@ hipError_t pass_history(obvhs_context* ctx, const obvhs_bvh2* bvh, std::vector<u
 }
 
 obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_prims_per_leaf,
-                           bool order_children, obvhs_cwbvh* out) {
+                           bool order_children, obvhs_cwbvh* out, const CwRootInfo* known) {
     hipStream_t st = ctx->stream;
     const uint32_t N = bvh2->node_count;
     out->node_count = 0;
@@ -777,9 +764,11 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
     OBVHS_TRY(ctx->scratch.cw_misc.ensure(sizeof(CwMisc)), "alloc cwbvh misc");
     CwMisc* misc = ctx->scratch.cw_misc.as<CwMisc>();
     const Node32* nodes = bvh2->nodes.as<Node32>();
-    k_cw_init<<<1, 64, 0, st>>>(misc);
     uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
-    if (bvh2->dp_max_prims != max_prims_per_leaf && n > 1) {
+    const bool table = bvh2->dp_max_prims != max_prims_per_leaf && n > 1;  // to be evaluated
+    if (table) known = nullptr;
+    if (table) k_cw_init<<<1, 64, 0, st>>>(misc);
+    if (table) {
         OBVHS_TRY(bvh_dp_alloc(bvh2), "alloc cost table");
         const DpView dpv = bvh_dp_view(bvh2, max_prims_per_leaf);
         std::vector<uint32_t> hist;
@@ -800,17 +789,20 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
         bvh2->dp_max_prims = max_prims_per_leaf;
     }
     const DpView dp = bvh_dp_view(bvh2, max_prims_per_leaf);
-    // Root, CWBVH node count and depth (the root's subtree size and levels) and device errors: one copy.
-    k_cw_info<<<1, 64, 0, st>>>(nodes, dp, misc);
+    // Root, CWBVH node count and depth (the root's subtree size and levels) and device errors: one copy, unless the
+    // build that has just ended brought them along.
+    k_cw_info<<<1, 64, 0, st>>>(nodes, dp, misc, table ? 0u : 1u);
     OBVHS_TRY(hipGetLastError(), "cwbvh info launch");
-    OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(CwMisc), hipMemcpyDeviceToHost, st), "read cw info");
-    OBVHS_TRY(hipStreamSynchronize(st), "cwbvh dp sync");
-    CwMisc hm;
-    memcpy(&hm, h, sizeof(CwMisc));
-    if (hm.err) return device_error_to_status(hm.err);
-    Node32 root;
-    memcpy(&root, hm.info, sizeof(Node32));
-    const uint32_t ncw = hm.info[8], levels = hm.info[9];
+    CwRootInfo info;
+    if (known) {
+        info = *known;
+    } else {
+        OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(CwMisc), hipMemcpyDeviceToHost, st), "read cw info");
+        OBVHS_TRY(hipStreamSynchronize(st), "cwbvh dp sync");
+        if (h[0]) return device_error_to_status(h[0]);
+        memcpy(&info, reinterpret_cast<const char*>(h) + offsetof(CwMisc, info), sizeof(info));
+    }
+    const uint32_t ncw = info.size, levels = info.depth;
     if (ncw == 0u) return OBVHS_ERR_CW_DISTRIBUTE;  // some CWBVH node's children cannot be distributed
     if (ncw > N) return OBVHS_ERR_CAPACITY;
     if (levels > MAX_CW_LEVELS) return OBVHS_ERR_DEPTH;
@@ -850,8 +842,8 @@ obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_pr
     if (h[0]) return device_error_to_status(h[0]);
     if (h[1 + levels] != 0u) return OBVHS_ERR_DEPTH;  // deeper than the depth table said (cannot happen)
     // total_aabb = bvh2.nodes[0].aabb (bvh2_to_cwbvh.rs:506)
-    out->total_aabb.min = obvhs_vec3a{root.minx, root.miny, root.minz, 0.0f};
-    out->total_aabb.max = obvhs_vec3a{root.maxx, root.maxy, root.maxz, 0.0f};
+    out->total_aabb.min = obvhs_vec3a{info.min[0], info.min[1], info.min[2], 0.0f};
+    out->total_aabb.max = obvhs_vec3a{info.max[0], info.max[1], info.max[2], 0.0f};
     out->node_count = ncw;
     out->prim_count = n;
     return OBVHS_OK;

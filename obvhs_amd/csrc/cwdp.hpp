@@ -20,6 +20,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "internal.hpp"
 
 namespace obvhs {
 
@@ -240,6 +241,18 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                 const Node32& r) {
     return dp_evaluate(dp, half_area(box), first, dp_child(l), dp_child(r));
+}
+
+// The root's part of the evaluated table (1 and 1 for a single-leaf BVH2).
+__device__ __forceinline__ CwRootInfo root_info(const Node32* nodes, const DpView& dp) {
+    const Node32 n = load_node(&nodes[0]);
+    CwRootInfo r{{n.minx, n.miny, n.minz}, {n.maxx, n.maxy, n.maxz}, 1u, 1u};
+    if (n.prim_count == 0u) {
+        const DpRec& e = dp.rec[dkey(n.first_index)];
+        r.size = e.cwsize;
+        r.depth = e.cwdepth;
+    }
+    return r;
 }
 
 }  // namespace obvhs

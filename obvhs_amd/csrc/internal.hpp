@@ -30,6 +30,12 @@ struct DevBuf {
 // PLOC per-pass state, double buffered on the device (pass k reads slot k&1, writes slot (k+1)&1).
 constexpr size_t PINNED_BYTES = 4096;
 
+// What a conversion's launches depend on: the BVH2 root's box, and the size and depth of the CWBVH subtree it roots.
+struct CwRootInfo {
+    float min[3], max[3];
+    uint32_t size, depth;
+};
+
 struct PlocState {
     uint32_t count;
     uint32_t insert;
@@ -146,7 +152,8 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
                           uint32_t search_depth_threshold);
 obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const obvhs_aabb* d_aabbs,
                         const uint32_t* d_indices, uint32_t n, uint32_t search_distance, bool u128,
-                        uint32_t search_depth_threshold, uint32_t fused_max_prims, obvhs_bvh2* bvh);
+                        uint32_t search_depth_threshold, uint32_t fused_max_prims, obvhs_bvh2* bvh,
+                        CwRootInfo* info = nullptr);
 struct DpView;
 hipError_t bvh_dp_alloc(obvhs_bvh2* bvh);
 DpView bvh_dp_view(const obvhs_bvh2* bvh, uint32_t max_prims);
@@ -154,7 +161,8 @@ DpView bvh_dp_view(const obvhs_bvh2* bvh, uint32_t max_prims);
 // cwbvh.hip
 hipError_t pass_history(obvhs_context* ctx, const obvhs_bvh2* bvh, std::vector<uint32_t>& hist);
 obvhs_status cwbvh_convert(obvhs_context* ctx, obvhs_bvh2* bvh2, uint32_t max_prims_per_leaf,
-                           bool order_children, obvhs_cwbvh* out);
+                           bool order_children, obvhs_cwbvh* out,
+                           const CwRootInfo* known = nullptr);
 struct MeshDesc;
 obvhs_status cwbvh_convert_batch(obvhs_context* ctx, const Node32* nodes, const uint32_t* bvh2_prims,
                                  const DpView& dp, MeshDesc* d_meshes, std::vector<MeshDesc>& meshes,

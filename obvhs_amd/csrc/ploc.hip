@@ -51,6 +51,7 @@ struct Misc {
     uint32_t err;
     uint32_t pad;
     PlocState state[2];
+    CwRootInfo info;  // written by the tail of a build that evaluates the cost table
 };
 
 __global__ void k_init_misc(Misc* misc, uint32_t n, uint32_t* hist) {
@@ -1243,7 +1244,10 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_ploc_tail(const Node32* __rest
     }
     ploc_tail<R, TAIL_MAX>(cur, st, first_pass, r, sd_is_one, depth_threshold, bvh_nodes, hist, dp, fused, slot_map,
                            vtop, map_len, &misc->err);
-    if (threadIdx.x == 0) misc->state[slot] = st;
+    if (threadIdx.x == 0) {
+        misc->state[slot] = st;
+        if (fused) misc->info = root_info(bvh_nodes, dp);
+    }
 }
 
 }  // namespace
@@ -1336,8 +1340,9 @@ static obvhs_status resort_gather(obvhs_context* ctx, const Node32* leaves, uint
 // The error word and the pass state of `slot` with one copy (err, pad, state[0], state[1] are adjacent) into the
 // pinned staging area, then a stream synchronisation.
 static hipError_t read_state(const Misc* misc, uint32_t slot, void* pinned, hipStream_t st, PlocState& state,
-                             uint32_t& err) {
-    const size_t lo = offsetof(Misc, err), hi = offsetof(Misc, state) + (slot + 1u) * sizeof(PlocState);
+                             uint32_t& err, CwRootInfo* info = nullptr) {
+    const size_t lo = offsetof(Misc, err),
+                 hi = info ? sizeof(Misc) : offsetof(Misc, state) + (slot + 1u) * sizeof(PlocState);
     hipError_t e = hipMemcpyAsync(pinned, reinterpret_cast<const char*>(misc) + lo, hi - lo, hipMemcpyDeviceToHost,
                                   st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1345,6 +1350,7 @@ static hipError_t read_state(const Misc* misc, uint32_t slot, void* pinned, hipS
     const char* h = static_cast<const char*>(pinned);
     memcpy(&err, h, 4);
     memcpy(&state, h + (offsetof(Misc, state) + slot * sizeof(PlocState) - lo), sizeof(PlocState));
+    if (info) memcpy(info, h + (offsetof(Misc, info) - lo), sizeof(CwRootInfo));
     return hipSuccess;
 }
 
@@ -1409,7 +1415,7 @@ static void launch_pass(uint32_t blocks, hipStream_t st, const Node32* cur, Node
 static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uint32_t n, uint32_t r,
                                uint32_t search_depth_threshold, Node32* bvh_nodes, uint32_t* hist, DpView dp,
                                uint32_t fused, const uint32_t* slot_map, uint32_t vtop, uint32_t map_len,
-                               PlocState& fin, bool& resort) {
+                               PlocState& fin, bool& resort, CwRootInfo* info) {
     resort = false;
     hipStream_t st = ctx->stream;
     BuildScratch& S = ctx->scratch;
@@ -1482,7 +1488,7 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
                 map_len);
     OBVHS_TRY(hipGetLastError(), "ploc tail launch");
     uint32_t herr = 0u;
-    OBVHS_TRY(read_state(misc, slot, ctx->pinned, st, hstate, herr), "read final ploc state");
+    OBVHS_TRY(read_state(misc, slot, ctx->pinned, st, hstate, herr, info), "read final ploc state");
     if (herr & ~DERR_RESORT) return device_error_to_status(herr);
     if (herr) {
         resort = true;
@@ -1495,7 +1501,8 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
 
 obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const obvhs_aabb* d_aabbs,
                         const uint32_t* d_indices, uint32_t n, uint32_t search_distance, bool u128,
-                        uint32_t search_depth_threshold, uint32_t fused_max_prims, obvhs_bvh2* bvh) {
+                        uint32_t search_depth_threshold, uint32_t fused_max_prims, obvhs_bvh2* bvh,
+                        CwRootInfo* info) {
     if (!(search_distance == 1 || search_distance == 2 || search_distance == 6 || search_distance == 14 ||
           search_distance == 24 || search_distance == 32))
         return OBVHS_ERR_INVALID_ARG;  // ploc/mod.rs:550-561
@@ -1587,12 +1594,12 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
     PlocState fin{};
     bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, n, search_distance, search_depth_threshold, bvh_nodes, hist, dp,
-                                 fused, nullptr, 0u, 0u, fin, resort);
+                                 fused, nullptr, 0u, 0u, fin, resort, info);
     if (ps == OBVHS_OK && resort) {
         ps = resort_gather(ctx, leaves, keys, keys_hi, n, cur, order_out);
         if (ps == OBVHS_OK)
             ps = run_passes(ctx, cur, nxt, n, search_distance, search_depth_threshold, bvh_nodes, hist, dp, fused,
-                            nullptr, 0u, 0u, fin, resort);
+                            nullptr, 0u, 0u, fin, resort, info);
     }
     if (ps != OBVHS_OK) return ps;
     bvh->ploc_iterations = fin.depth;
@@ -1649,12 +1656,12 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     PlocState fin{};
     bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist,
-                                 DpView{}, 0u, d_slot_map, 2u * k - 3u, k - 1u, fin, resort);
+                                 DpView{}, 0u, d_slot_map, 2u * k - 3u, k - 1u, fin, resort, nullptr);
     if (ps == OBVHS_OK && resort) {
         ps = resort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
         if (ps == OBVHS_OK)
             ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist, DpView{}, 0u,
-                            d_slot_map, 2u * k - 3u, k - 1u, fin, resort);
+                            d_slot_map, 2u * k - 3u, k - 1u, fin, resort, nullptr);
     }
     if (ps != OBVHS_OK) return ps;
     if (!d_slot_map) bvh->node_count = 2u * k - 1u;  // ploc/mod.rs:283-284 (nodes.resize)

@@ -1968,21 +1968,18 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
         OBVHS_TRY(radix_sort_pairs32(Q.rkeys.as<uint32_t>(), Q.rvals.as<uint32_t>(), true, count, 32,
                                      Q.sort_scratch.ptr, st, sort_items_for(ctx, count)),
                   "reinsertion sort");
-        OBVHS_TRY(hipMemcpyAsync(h, misc, 12, hipMemcpyDeviceToHost, st), "read reinsertion count");
-        OBVHS_TRY(hipStreamSynchronize(st), "reinsertion count sync");
-        if (h[0]) return device_error_to_status(h[0]);
-        const uint32_t npos = h[1];
-        const bool replay = h[2] != 0u;
-        if (npos == 0) continue;
-        const uint32_t pblk = (npos + T256 - 1) / T256;
+        // The conflict rounds run over all candidates' places (those beyond the positive ones end at once), so that one
+        // read brings the error, the count and what is left undecided.
+        const uint32_t pblk = (count + T256 - 1) / T256;
         k_fill_u32<<<std::min(nblk, 4096u), T256, 0, st>>>(reinterpret_cast<uint32_t*>(touched), 0u,
                                                           ((size_t)N + 3) / 4);
         k_mis_init<<<pblk, T256, 0, st>>>(Q.rvals.as<uint32_t>(), misc, Q.rfrom.as<uint32_t>(),
                                           Q.rto.as<uint32_t>(), parents, Q.conf.as<uint32_t>(),
                                           Q.state.as<uint8_t>());
         // every round accepts at least the best-ranked undecided reinsertion, so npos rounds always suffice
+        uint32_t npos = 0;
+        bool replay = false;
         for (uint32_t batch = 0;; ++batch) {
-            if ((uint64_t)batch * MIS_ROUNDS_PER_SYNC > (uint64_t)npos + MIS_ROUNDS_PER_SYNC) return OBVHS_ERR_DEVICE;
             for (uint32_t r = 0; r < MIS_ROUNDS_PER_SYNC; ++r) {
                 k_mis_claim<<<pblk, T256, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, r, owner);
                 k_mis_decide<<<pblk, T256, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, owner,
@@ -1991,18 +1988,24 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
                                                     touched);
             }
             OBVHS_TRY(hipGetLastError(), "conflict rounds launch");
-            OBVHS_TRY(hipMemcpyAsync(h, &misc->undecided[MIS_ROUNDS_PER_SYNC - 1], 4, hipMemcpyDeviceToHost, st),
-                      "read undecided");
+            OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(ReinsMisc), hipMemcpyDeviceToHost, st), "read reinsertion state");
             OBVHS_TRY(hipStreamSynchronize(st), "conflict rounds sync");
-            if (h[0] == 0u) break;
+            ReinsMisc hm;
+            memcpy(&hm, h, sizeof(hm));
+            if (hm.err) return device_error_to_status(hm.err);
+            npos = hm.positive;
+            replay = hm.negzero != 0u;
+            if (hm.undecided[MIS_ROUNDS_PER_SYNC - 1] == 0u) break;
+            if ((uint64_t)batch * MIS_ROUNDS_PER_SYNC > (uint64_t)npos) return OBVHS_ERR_DEVICE;
         }
+        if (npos == 0) continue;
         if (replay) {
             // leaves hold a -0: the crate's walks decide which zero bits each box keeps, so they run as written
             k_reins_replay<<<1, 64, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, nodes, parents);
         } else {
             // every zero coordinate is +0, so a value-equal box has equal bits and one full refit (deferred to the
             // next step or fused with the cost table) leaves exactly the boxes the crate's walks leave
-            k_reins_apply<<<pblk, T256, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, nodes);
+            k_reins_apply<<<(npos + T256 - 1) / T256, T256, 0, st>>>(Q.conf.as<uint32_t>(), Q.state.as<uint8_t>(), misc, nodes);
         }
         OBVHS_TRY(hipGetLastError(), "apply launch");
         s = walked_levels(ctx, bvh, meta, levels);
