@@ -147,8 +147,7 @@ def tune_step(ob, ctx, n_prims, step, reps=3, layouts=("triangle",)):
 def kernel_name(ctx, ob, n_prims, mode="closest"):
     t = ctx.tune_table()
     cls = ob.size_class(n_prims)
-    form = "k_traverse_chunk" if t["trav_chunk"][cls] else "k_traverse"
-    return f"{form}<{mode}, lds {t['trav_lds_depth'][cls]}>"
+    return f"k_traverse_chunk<{mode}, lds {t['trav_lds_depth'][cls]}>"
 
 
 def leg_counters(leg):

@@ -128,7 +128,8 @@ __global__ void __launch_bounds__(T256) k_dp_range(const Node32* __restrict__ no
 // workgroup lists their internal nodes in LDS with their heights above the finished slots (found pass by pass, LDS
 // only) and evaluates the entries by height (tail.hpp).  A chain of entries bounds it: pass by pass, each waiting for
 // the nodes' and then the records' loads, the last 36 passes of 1.29M triangles (from 4,096 slots a pass on) took 404
-// us; now 7 of them are launches of 4 us and the rest take 57 us.  hist[p] for p in [p0, passes] bounds the passes' slots; hist[passes] is 1.
+// us; now 7 of them are launches of 4 us and the rest take 57 us.  hist[p] for p in [p0, passes] bounds
+// the passes' slots; hist[passes] is 1.
 constexpr uint32_t TOP_NODES = 2048;
 __global__ void __launch_bounds__(1024) k_dp_top(const Node32* __restrict__ nodes, DpView dp,
                                                  const uint32_t* __restrict__ hist, uint32_t p0, uint32_t passes,
@@ -921,8 +922,8 @@ obvhs_status cwbvh_convert_batch(obvhs_context* ctx, const Node32* nodes, const 
 hipError_t launch_reorder_triangles(const obvhs_triangle* tris, const uint32_t* prim_indices, uint32_t n,
                                     obvhs_triangle* out, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    k_reorder_tris<<<xcd_grid((n + T256 - 1) / T256), T256, 0, stream>>>(reinterpret_cast<const float4*>(tris), prim_indices,
-                                                                n, reinterpret_cast<float4*>(out));
+    k_reorder_tris<<<xcd_grid((n + T256 - 1) / T256), T256, 0, stream>>>(
+        reinterpret_cast<const float4*>(tris), prim_indices, n, reinterpret_cast<float4*>(out));
     return hipGetLastError();
 }
 

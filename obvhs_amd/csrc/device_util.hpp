@@ -191,7 +191,8 @@ __device__ __forceinline__ uint2 scan_chunk_apply(uint2* __restrict__ counts, ui
 // Workgroups go round-robin to the 8 XCDs, each with its own L2.  The tile of a workgroup such that an XCD's
 // workgroups take one contiguous eighth of the tiles: for kernels whose neighbouring tiles read the same lines at
 // random (a 128-byte line holds four leaf records or parts of four triangles).  20M triangles in 4,096 meshes: leaf
-// gather 502 -> 471 us; 17.3M-triangle build with reordering 29.96 -> 29.54 ms.  The grid is xcd_grid(tiles) workgroups; those that get a tile >= tiles have none.
+// gather 502 -> 471 us; 17.3M-triangle build with reordering 29.96 -> 29.54 ms.  The grid is xcd_grid(tiles) workgroups;
+// those that get a tile >= tiles have none.
 constexpr uint32_t XCDS = 8;
 inline uint32_t xcd_grid(uint32_t tiles) { return (tiles + XCDS - 1) / XCDS * XCDS; }
 __device__ __forceinline__ uint32_t xcd_tile() {

@@ -1311,9 +1311,11 @@ static obvhs_status sort_gather(obvhs_context* ctx, const Node32* leaves, const 
               "radix sort (top words)");
     const uint32_t nblk = (n + T256 - 1) / T256;
     if (keys_hi)
-        k_gather_runs<true><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+        k_gather_runs<true><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur,
+                                                             order_out);
     else
-        k_gather_runs<false><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur, order_out);
+        k_gather_runs<false><<<xcd_grid(nblk), T256, 0, st>>>(leaves, tops, vals, n, keys, keys_hi, misc, cur,
+                                                              order_out);
     OBVHS_TRY(hipGetLastError(), "gather launch");
     return OBVHS_OK;
 }

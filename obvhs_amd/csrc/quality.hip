@@ -158,9 +158,9 @@ __global__ void __launch_bounds__(T256) k_refit_level(Node32* __restrict__ nodes
     store_node(&nodes[x], make_node(u, 0u, nd.first_index));
 }
 
-// Consecutive levels [lo, hi] of at most REFIT_RUN nodes each by one workgroup, deepest first; the next level's nodes are
-// loaded beside this one's children.  A launch of such a level waits 3 us for its three dependent loads and as long for
-// the next launch; a level here takes 1.3 us.
+// Consecutive levels [lo, hi] of at most REFIT_RUN nodes each by one workgroup, deepest first; the next level's nodes
+// are loaded beside this one's children.  A launch of such a level waits 3 us for its three dependent loads and as long
+// for the next launch; a level here takes 1.3 us.
 constexpr uint32_t REFIT_RUN = 1024;
 __global__ void __launch_bounds__(REFIT_RUN) k_refit_run(Node32* __restrict__ nodes, const uint32_t* __restrict__ list,
                                                          const uint32_t* __restrict__ meta, uint32_t lo, uint32_t hi) {

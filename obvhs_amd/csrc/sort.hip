@@ -13,8 +13,8 @@
 //               keys are reordered in LDS and written out coalesced per digit run, then its values through the same
 //               LDS (half the LDS of staging both at once, so twice the tiles per CU).
 // Up to FEW_TILES tiles the scan has no launch: the upsweep writes counts[tile][digit] and every tile of the downsweep
-// sums the digits' counts itself.  A sort of 26K keys (13 tiles) was 12 launches of 5 to 8 us, bound by latency; 32 such
-// sorts of a reinsertion: 2.0 -> 1.5 ms.  At 49 tiles both forms take 55 us a sort.
+// sums the digits' counts itself.  A sort of 26K keys (13 tiles) was 12 launches of 5 to 8 us, bound by latency; 32
+// such sorts of a reinsertion: 2.0 -> 1.5 ms.  At 49 tiles both forms take 55 us a sort.
 // Tiles are 256 threads x ITEMS keys (ITEMS = 4, 8 or 16, the sort tile the context's tuning table picks per size
 // class; 8 by default); each wave owns a contiguous 64 x ITEMS key segment.  Every tile size gives the same order.
 //
@@ -216,6 +216,100 @@ __global__ void __launch_bounds__(SORT_THREADS)
     }
 }
 
+// At most ONE_MAX u32 keys: the whole sort in one workgroup, keys and values in LDS between the passes (a wave owns 64 x
+// ITEMS consecutive keys, ranked as in the downsweep).  The ranking's instructions bound it: 2,048 keys 12 us, 4,096
+// 19, 8,192 30, against 46 us and eight launches at any of these sizes.
+constexpr int ONE_THREADS = 1024;
+constexpr int ONE_WAVES = ONE_THREADS / 64;
+constexpr uint32_t ONE_MAX = ONE_THREADS * 8;
+
+template <int ITEMS>
+__global__ void __launch_bounds__(ONE_THREADS)
+    k_radix_one(uint32_t* __restrict__ keys, uint32_t* __restrict__ values, uint32_t identity, uint32_t n,
+                uint32_t passes) {
+    __shared__ uint32_t sk[ONE_THREADS * ITEMS], sv[ONE_THREADS * ITEMS];
+    __shared__ uint32_t whist[ONE_WAVES][256];
+    __shared__ uint32_t wtot[4];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+    const uint32_t seg = wave * (64 * ITEMS);
+    const uint64_t lt = lanemask_lt();
+    uint32_t k[ITEMS], v[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t e = seg + j * 64 + lane;
+        k[j] = e < n ? keys[e] : 0u;
+        v[j] = e < n ? (identity ? e : values[e]) : 0u;
+    }
+    for (uint32_t pass = 0; pass < passes; ++pass) {
+        const uint32_t shift = pass * 8u;
+        for (uint32_t i = lane; i < 256u; i += 64u) whist[wave][i] = 0u;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const bool valid = seg + j * 64 + lane < n;
+            const uint32_t d = (k[j] >> shift) & 0xffu;
+            uint64_t peers = ballot64(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bm = ballot64(bit);
+                peers &= bit ? bm : ~bm;
+            }
+            const uint32_t below = (uint32_t)__popcll(peers & lt);
+            uint32_t base = 0;
+            if (valid) base = whist[wave][d];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0) whist[wave][d] = base + (uint32_t)__popcll(peers);
+            __builtin_amdgcn_wave_barrier();
+            rank[j] = base + below;
+        }
+        __syncthreads();
+        // digit tid: where its keys begin in each wave's share
+        uint32_t total = 0u, incl = 0u;
+        if (tid < 256u) {
+            for (int w = 0; w < ONE_WAVES; ++w) {
+                const uint32_t c = whist[w][tid];
+                whist[w][tid] = total;
+                total += c;
+            }
+            incl = wave_inclusive_scan(total);
+            if (lane == 63u) wtot[wave] = incl;
+        }
+        __syncthreads();
+        if (tid < 256u) {
+            uint32_t start = incl - total;
+            for (uint32_t w = 0; w < wave; ++w) start += wtot[w];
+            for (int w = 0; w < ONE_WAVES; ++w) whist[w][tid] += start;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            if (seg + j * 64 + lane < n) {
+                const uint32_t at = whist[wave][(k[j] >> shift) & 0xffu] + rank[j];
+                sk[at] = k[j];
+                sv[at] = v[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const uint32_t e = seg + j * 64 + lane;
+            if (e < n) {
+                k[j] = sk[e];
+                v[j] = sv[e];
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t e = seg + j * 64 + lane;
+        if (e < n) {
+            keys[e] = k[j];
+            values[e] = v[j];
+        }
+    }
+}
+
 }  // namespace
 
 size_t radix_sort_scratch_bytes(uint32_t n) {
@@ -296,7 +390,15 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identi
 
 hipError_t radix_sort_pairs32(uint32_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                               void* scratch, hipStream_t stream, int items) {
-    return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
+    if (n == 0 || n > ONE_MAX) return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
+    const uint32_t identity = values_identity ? 1u : 0u, passes = (uint32_t)(bits + 7) / 8u;
+    if (n <= ONE_THREADS * 2u)
+        k_radix_one<2><<<1, ONE_THREADS, 0, stream>>>(keys, values, identity, n, passes);
+    else if (n <= ONE_THREADS * 4u)
+        k_radix_one<4><<<1, ONE_THREADS, 0, stream>>>(keys, values, identity, n, passes);
+    else
+        k_radix_one<8><<<1, ONE_THREADS, 0, stream>>>(keys, values, identity, n, passes);
+    return hipGetLastError();
 }
 
 }  // namespace obvhs
