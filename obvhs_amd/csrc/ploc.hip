@@ -9,8 +9,7 @@
 //   radix sort     : stable (sort.hip); a U128 key is sorted by its low word, then stably by its high word
 //   k_gather       : sorted leaves become the first cluster array (ploc/mod.rs:829-846)
 //   per pass       : k_ploc_search_count (ploc/mod.rs:329-419, window in LDS, and the per-tile counts of emitted
-//                    clusters and merges), k_ploc_scan (their prefix sums; two launches over chunks for the largest
-//                    passes),
+//                    clusters and merges), their prefix sums in two launches over chunks for the largest passes,
 //                    k_ploc_compact (ploc/mod.rs:420-487: the parent of a mutual pair is emitted at the higher
 //                    index, its children go to nodes[insert - 2(s+1)] and [+1] where s is the merge's rank in the
 //                    pass); passes of at most 1,024 tiles are one launch each (k_ploc_pass)
@@ -46,13 +45,27 @@ constexpr int TAIL_THREADS = 1024;
 // Passes enqueued between host reads of the cluster count (1.29M-triangle build: 4 -> 1.97 ms, 8 -> 1.92, 16 -> 1.93).
 constexpr int PASSES_PER_SYNC = 8;
 
+// Passes of at most GROUP_MAX_TILES tiles need no scan between search and compaction: a tile's place is the sum of the
+// groups before its own and of the tiles before it in its group (k_ploc_compact).  Eight passes of up to 5,033 tiles: the
+// scans took 46 us; the search's atomics cost 8 of them with 16 tiles to a group, 46 with 64.
+constexpr uint32_t GROUP_TILES = 16;
+constexpr uint32_t TILE_GROUPS = 1024;
+constexpr uint32_t GROUP_MAX_TILES = GROUP_TILES * TILE_GROUPS;
+
 struct Misc {
     uint32_t bounds[6];  // order keys: min x,y,z (atomicMin) then max x,y,z (atomicMax)
     uint32_t err;
     uint32_t pad;
     PlocState state[2];
     CwRootInfo info;  // written by the tail of a build that evaluates the cost table
+    // Sums of the tiles' counts (emits in the low word, merges in the high one) by GROUP_TILES tiles, by slot; zero
+    // before a pass, the other slot's cleared by the pass's compaction.
+    unsigned long long groups[2][TILE_GROUPS];
 };
+
+__device__ __forceinline__ void clear_groups(Misc* misc) {
+    for (uint32_t g = threadIdx.x; g < 2u * TILE_GROUPS; g += blockDim.x) (&misc->groups[0][0])[g] = 0ull;
+}
 
 __global__ void k_init_misc(Misc* misc, uint32_t n, uint32_t* hist) {
     if (threadIdx.x == 0) {
@@ -65,6 +78,7 @@ __global__ void k_init_misc(Misc* misc, uint32_t n, uint32_t* hist) {
         misc->state[0] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
         misc->state[1] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
     }
+    clear_groups(misc);
 }
 
 // Reduces the leaf bounds of one block into the scene bounds.  Both the min and the max corner of every leaf go
@@ -343,6 +357,7 @@ __global__ void k_reset_state(Misc* misc, uint32_t n) {
         misc->state[0] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
         misc->state[1] = PlocState{n, 2u * n - 1u, 0u, 0u, 0ull};
     }
+    clear_groups(misc);
 }
 
 // The front of a build of at most SMALL_MAX leaves in one workgroup and one launch: leaf boxes, scene bounds, Morton
@@ -653,7 +668,7 @@ template <int R>
 __global__ void __launch_bounds__(SC_THREADS) k_ploc_search_count(const Node32* __restrict__ cur, Misc* misc,
                                                                   uint32_t slot, uint32_t r, uint32_t dist1,
                                                                   int8_t* __restrict__ merge,
-                                                                  uint2* __restrict__ blocksums) {
+                                                                  uint2* __restrict__ blocksums, uint32_t grouped) {
     __shared__ float s[6][SC_WINDOW];
     __shared__ int8_t mm[T256 + 2 * MAX_RADIUS];  // offsets of clusters [base - r, base + 256 + r)
     __shared__ uint32_t we[T256 / 64], wm[T256 / 64];
@@ -662,7 +677,7 @@ __global__ void __launch_bounds__(SC_THREADS) k_ploc_search_count(const Node32* 
     if (count <= 1 || base >= count) {  // workgroup-uniform
         if (threadIdx.x == 0)
             blocksums[blockIdx.x] = count == 1 && blockIdx.x == 0 ? make_uint2(1u, 0u) : make_uint2(0u, 0u);
-        return;
+        return;  // a single cluster's pass changes nothing: its group stays empty
     }
     const int wstart = (int)base - 2 * (int)r;
     const int wlen = T256 + 4 * (int)r;
@@ -743,66 +758,12 @@ __global__ void __launch_bounds__(SC_THREADS) k_ploc_search_count(const Node32* 
             M += wm[w];
         }
         blocksums[blockIdx.x] = make_uint2(E, M);
+        if (grouped) atomicAdd(&misc->groups[slot][blockIdx.x / GROUP_TILES], (unsigned long long)M << 32 | E);
     }
 }
 
-// Single workgroup: exclusive scan of the per-block (emit, merge) counts and the next pass's state.
-__global__ void __launch_bounds__(1024) k_ploc_scan(uint2* __restrict__ blocksums, uint32_t nblocks, Misc* misc,
-                                                    uint32_t slot, uint32_t* __restrict__ hist) {
-    __shared__ uint32_t se[16], sm[16];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t chunk = (nblocks + 1023u) / 1024u;
-    const uint32_t b0 = tid * chunk, b1 = min(nblocks, b0 + chunk);
-    uint32_t E = 0, M = 0;
-    // each thread's chunk is contiguous (the prefix order); unrolled so that several loads are in flight
-#pragma unroll 8
-    for (uint32_t b = b0; b < b1; ++b) {
-        uint2 v = blocksums[b];
-        E += v.x;
-        M += v.y;
-    }
-    uint32_t ie = wave_inclusive_scan(E), im = wave_inclusive_scan(M);
-    const uint32_t wave = tid >> 6, lane = tid & 63u;
-    if (lane == 63) {
-        se[wave] = ie;
-        sm[wave] = im;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        uint32_t re = 0, rm = 0;
-        for (int w = 0; w < 16; ++w) {
-            uint32_t te = se[w], tm = sm[w];
-            se[w] = re;
-            sm[w] = rm;
-            re += te;
-            rm += tm;
-        }
-        const PlocState st = misc->state[slot];
-        PlocState nx = st;
-        if (st.count > 1) {
-            nx.count = re;
-            nx.insert = st.insert - 2u * rm;
-            nx.depth = st.depth + 1u;
-            nx.cluster_sum = st.cluster_sum + st.count;
-            hist[nx.depth] = nx.insert;
-        }
-        misc->state[slot ^ 1u] = nx;
-    }
-    __syncthreads();
-    uint32_t ee = se[wave] + ie - E, em = sm[wave] + im - M;
-#pragma unroll 8
-    for (uint32_t b = b0; b < b1; ++b) {
-        uint2 v = blocksums[b];
-        blocksums[b] = make_uint2(ee, em);
-        ee += v.x;
-        em += v.y;
-    }
-}
-
-// Two-level scan of the tile counts for passes of more than SCAN_ONE_BLOCK tiles (one workgroup reading every count
-// twice takes ~50 us at 74K tiles): k_ploc_scan_chunks sums SCAN_CHUNK counts per workgroup, k_ploc_scan_apply
+// Two-level scan of the tile counts for passes of more than GROUP_MAX_TILES tiles: k_ploc_scan_chunks sums SCAN_CHUNK counts per workgroup, k_ploc_scan_apply
 // offsets each chunk by the chunks before it and scans it, and its workgroup 0 writes the next pass's state.
-constexpr uint32_t SCAN_ONE_BLOCK = 16384;   // passes of at most this many tiles use k_ploc_scan
 
 __global__ void __launch_bounds__(1024) k_ploc_scan_chunks(const uint2* __restrict__ blocksums, uint32_t nblocks,
                                                            uint2* __restrict__ chunk_tot) {
@@ -893,19 +854,57 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
     }
 }
 
+// Emits and merges of the first `n` groups, plus the lanes' own e and m, in every lane of the wave.
+__device__ __forceinline__ uint2 group_sums(const unsigned long long* groups, uint32_t n, uint32_t e, uint32_t m) {
+    for (uint32_t g = threadIdx.x & 63u; g < n; g += 64u) {
+        const unsigned long long x = groups[g];
+        e += (uint32_t)x;
+        m += (uint32_t)(x >> 32);
+    }
+    e = wave_inclusive_scan_dpp(e);
+    m = wave_inclusive_scan_dpp(m);
+    return make_uint2((uint32_t)__builtin_amdgcn_readlane((int)e, 63), (uint32_t)__builtin_amdgcn_readlane((int)m, 63));
+}
+
 __global__ void __launch_bounds__(T256) k_ploc_compact(const Node32* __restrict__ cur, Node32* __restrict__ next,
                                                        const int8_t* __restrict__ merge, Misc* misc, uint32_t slot,
-                                                       const uint2* __restrict__ offsets,
+                                                       const uint2* __restrict__ counts, uint32_t grouped,
                                                        Node32* __restrict__ bvh_nodes, DpView dp, uint32_t fused,
                                                        const uint32_t* __restrict__ slot_map, uint32_t vtop,
-                                                       uint32_t map_len) {
+                                                       uint32_t map_len, uint32_t* __restrict__ hist) {
     __shared__ uint32_t we[T256 / 64], wm[T256 / 64];
     const PlocState st = misc->state[slot];
+    if (grouped && blockIdx.x == 0) {  // the state after the pass; the other slot's groups for the next one
+        for (uint32_t g = threadIdx.x; g < TILE_GROUPS; g += T256) misc->groups[slot ^ 1u][g] = 0ull;
+        if (threadIdx.x < 64u) {
+            const uint2 all = group_sums(misc->groups[slot], (gridDim.x + GROUP_TILES - 1u) / GROUP_TILES, 0u, 0u);
+            if (threadIdx.x == 0) {
+                PlocState nx = st;
+                if (st.count > 1u) {
+                    nx.count = all.x;
+                    nx.insert = st.insert - 2u * all.y;
+                    nx.depth = st.depth + 1u;
+                    nx.cluster_sum = st.cluster_sum + st.count;
+                    hist[nx.depth] = nx.insert;
+                }
+                misc->state[slot ^ 1u] = nx;
+            }
+        }
+    }
+    if (blockIdx.x * T256 >= st.count) return;
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     Node32 a{};
     if (i < st.count) a = load_node(&cur[i]);
     const Cls k = classify(merge, i, st.count);
-    const uint2 off = offsets[blockIdx.x];
+    uint2 off;
+    if (grouped) {  // in every wave by itself: no barrier
+        const uint32_t g0 = blockIdx.x / GROUP_TILES, tile = g0 * GROUP_TILES + (threadIdx.x & 63u);  // those below its own
+        uint2 v = make_uint2(0u, 0u);
+        if (tile < blockIdx.x) v = counts[tile];
+        off = group_sums(misc->groups[slot], g0, v.x, v.y);
+    } else {
+        off = counts[blockIdx.x];
+    }
     compact_tile(cur, next, a, k.emit, k.mrg, k.b, st, off.x, off.y, bvh_nodes, dp, fused, slot_map, vtop, map_len,
                  &misc->err, we, wm);
 }
@@ -1344,7 +1343,7 @@ static obvhs_status resort_gather(obvhs_context* ctx, const Node32* leaves, uint
 static hipError_t read_state(const Misc* misc, uint32_t slot, void* pinned, hipStream_t st, PlocState& state,
                              uint32_t& err, CwRootInfo* info = nullptr) {
     const size_t lo = offsetof(Misc, err),
-                 hi = info ? sizeof(Misc) : offsetof(Misc, state) + (slot + 1u) * sizeof(PlocState);
+                 hi = info ? offsetof(Misc, info) + sizeof(CwRootInfo) : offsetof(Misc, state) + (slot + 1u) * sizeof(PlocState);
     hipError_t e = hipMemcpyAsync(pinned, reinterpret_cast<const char*>(misc) + lo, hi - lo, hipMemcpyDeviceToHost,
                                   st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1358,14 +1357,14 @@ static hipError_t read_state(const Misc* misc, uint32_t slot, void* pinned, hipS
 
 // The search-and-count kernel for the search distance (each allowed distance has its unrolled instance).
 static void launch_search_count(uint32_t blocks, hipStream_t st, const Node32* cur, Misc* misc, uint32_t slot,
-                                uint32_t r, uint32_t dist1, int8_t* merge, uint2* blocksums) {
+                                uint32_t r, uint32_t dist1, int8_t* merge, uint2* blocksums, uint32_t grouped) {
     switch (r) {
-        case 2: k_ploc_search_count<2><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
-        case 6: k_ploc_search_count<6><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
-        case 14: k_ploc_search_count<14><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
-        case 24: k_ploc_search_count<24><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
-        case 32: k_ploc_search_count<32><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
-        default: k_ploc_search_count<0><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums); break;
+        case 2: k_ploc_search_count<2><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
+        case 6: k_ploc_search_count<6><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
+        case 14: k_ploc_search_count<14><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
+        case 24: k_ploc_search_count<24><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
+        case 32: k_ploc_search_count<32><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
+        default: k_ploc_search_count<0><<<blocks, SC_THREADS, 0, st>>>(cur, misc, slot, r, dist1, merge, blocksums, grouped); break;
     }
 }
 
@@ -1454,10 +1453,9 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
         } else {
             for (int k = 0; k < PASSES_PER_SYNC; ++k) {
                 const uint32_t dist1 = (r == 1 || pass < search_depth_threshold) ? 1u : 0u;
-                launch_search_count(blocks, st, cur, misc, slot, r, dist1, merge, blocksums);
-                if (blocks <= SCAN_ONE_BLOCK) {
-                    k_ploc_scan<<<1, 1024, 0, st>>>(blocksums, blocks, misc, slot, hist);
-                } else {
+                const uint32_t grouped = blocks <= GROUP_MAX_TILES ? 1u : 0u;
+                launch_search_count(blocks, st, cur, misc, slot, r, dist1, merge, blocksums, grouped);
+                if (!grouped) {
                     // chunk totals after the counts, in the blocksums allocation's tail (dead during the passes)
                     uint2* chunk_tot = blocksums + blocks + 16;
                     const uint32_t nchunks = (blocks + SCAN_CHUNK - 1) / SCAN_CHUNK;
@@ -1465,8 +1463,8 @@ static obvhs_status run_passes(obvhs_context* ctx, Node32* cur, Node32* nxt, uin
                     k_ploc_scan_apply<<<nchunks, 1024, 0, st>>>(blocksums, blocks, chunk_tot, nchunks, misc, slot,
                                                                  hist);
                 }
-                k_ploc_compact<<<blocks, T256, 0, st>>>(cur, nxt, merge, misc, slot, blocksums, bvh_nodes, dp, fused,
-                                                       slot_map, vtop, map_len);
+                k_ploc_compact<<<blocks, T256, 0, st>>>(cur, nxt, merge, misc, slot, blocksums, grouped, bvh_nodes, dp,
+                                                       fused, slot_map, vtop, map_len, hist);
                 std::swap(cur, nxt);
                 slot ^= 1u;
                 pass++;
