@@ -46,8 +46,8 @@ constexpr int TAIL_THREADS = 1024;
 constexpr int PASSES_PER_SYNC = 8;
 
 // Passes of at most GROUP_MAX_TILES tiles need no scan between search and compaction: a tile's place is the sum of the
-// groups before its own and of the tiles before it in its group (k_ploc_compact).  Eight passes of up to 5,033 tiles: the
-// scans took 46 us; the search's atomics cost 8 of them with 16 tiles to a group, 46 with 64.
+// groups before its own and of the tiles before it in its group (k_ploc_compact).  Eight passes of up to 5,033 tiles:
+// the scans took 46 us; the search's atomics cost 8 of them with 16 tiles to a group, 46 with 64.
 constexpr uint32_t GROUP_TILES = 16;
 constexpr uint32_t TILE_GROUPS = 1024;
 constexpr uint32_t GROUP_MAX_TILES = GROUP_TILES * TILE_GROUPS;
@@ -762,9 +762,9 @@ __global__ void __launch_bounds__(SC_THREADS) k_ploc_search_count(const Node32* 
     }
 }
 
-// Two-level scan of the tile counts for passes of more than GROUP_MAX_TILES tiles: k_ploc_scan_chunks sums SCAN_CHUNK counts per workgroup, k_ploc_scan_apply
-// offsets each chunk by the chunks before it and scans it, and its workgroup 0 writes the next pass's state.
-
+// Two-level scan of the tile counts for passes of more than GROUP_MAX_TILES tiles: k_ploc_scan_chunks sums SCAN_CHUNK
+// counts per workgroup, k_ploc_scan_apply offsets each chunk by the chunks before it and scans it, and its workgroup 0
+// writes the next pass's state.
 __global__ void __launch_bounds__(1024) k_ploc_scan_chunks(const uint2* __restrict__ blocksums, uint32_t nblocks,
                                                            uint2* __restrict__ chunk_tot) {
     scan_chunk_total(blocksums, nblocks, chunk_tot);
