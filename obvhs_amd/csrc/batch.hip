@@ -562,7 +562,7 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     // The tile's merges, their cost-table entries evaluated by consecutive threads afterwards (a merge is counted at
     // its higher cluster; a partner lies within its mesh's distance, at most MAX_RADIUS: at most 128 + r / 2).
     constexpr uint32_t MAX_TILE_MERGES = (T256 + MAX_RADIUS) / 2;
-    __shared__ Node32 s_left[MAX_TILE_MERGES], s_right[MAX_TILE_MERGES];
+    __shared__ __align__(16) Node32 s_left[MAX_TILE_MERGES], s_right[MAX_TILE_MERGES];
     __shared__ uint32_t s_first[MAX_TILE_MERGES], s_kbase[MAX_TILE_MERGES];
     const uint32_t total = misc->total[q];
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
@@ -613,13 +613,26 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     }
     lds_barrier();  // the stores are not waited for
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
-    if (threadIdx.x < nm) {
-        const Node32 l = s_left[threadIdx.x], r = s_right[threadIdx.x];
-        DpView dpm = dp;
+    if (wave * 64u >= nm) return;
+    const bool entry = threadIdx.x < nm;
+    Node32 l{}, r{};
+    l.prim_count = r.prim_count = 1u;
+    DpView dpm = dp;
+    uint32_t first = 0u;
+    if (entry) {
+        l = s_left[threadIdx.x];
+        r = s_right[threadIdx.x];
         dpm.kbase = s_kbase[threadIdx.x];
-        const uint32_t e = dp_evaluate(dpm, box_union(node_box(l), node_box(r)), s_first[threadIdx.x], l, r);
-        if (e) atomicOr(&misc->err, e);
+        first = s_first[threadIdx.x];
     }
+    const Box box = box_union(node_box(l), node_box(r));
+    uint32_t e;
+    if (wave < 2u) {  // the wave's entries of s_left are in its lanes' registers now: 2 KB of LDS
+        e = dp_evaluate_wave(dpm, box, first, l, r, entry, reinterpret_cast<uint4*>(&s_left[wave * 64u]));
+    } else {
+        e = entry ? dp_evaluate(dpm, box, first, l, r) : 0u;
+    }
+    if (e) atomicOr(&misc->err, e);
 }
 
 // The remaining passes of every mesh of search distance r, one workgroup per mesh (tail.hpp), once no mesh has more

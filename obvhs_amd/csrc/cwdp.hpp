@@ -150,9 +150,8 @@ __device__ __forceinline__ ChildDp child_dp(const DpChild& c, const DpRaw& raw) 
 // from the records afterwards (up to 14 loads one after the other), 7.5K with the records loaded one after the other
 // and a branch per candidate pair (1.29M-triangle build: the tail 215 -> 182 us, the grid passes' compactions 376 ->
 // 338 us, the refit's table 792 -> 630 us).
-__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
-                                                const DpChild& r, const DpRaw& raw_l, const DpRaw& raw_r) {
-    DpRec* const rec = &dp.rec[dp_key(dp, first)];
+__device__ __forceinline__ uint32_t dp_entry(const DpView& dp, float ha, const DpChild& l, const DpChild& r,
+                                             const DpRaw& raw_l, const DpRaw& raw_r, uint4* e) {
     const bool ll = l.prim_count != 0u, rl = r.prim_count != 0u;
     const ChildDp L = child_dp(l, raw_l), R = child_dp(r, raw_r);
     const uint32_t num_primitives = L.nprims + R.nprims;
@@ -200,9 +199,7 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint
     const bool two = L.plist.w >= 2u, few = num_primitives <= 3u;
     const uint4 pl = make_uint4(few ? L.plist.x : 0u, few ? (two ? L.plist.y : R.plist.x) : 0u,
                                 few ? (two ? R.plist.x : R.plist.y) : 0u, few ? num_primitives : 0u);
-    // The whole 128-byte entry in eight 16-byte stores (the padding too, so that no 32-byte sector of the line is
-    // left partly written).
-    uint4* e = reinterpret_cast<uint4*>(rec);
+    // The whole 128-byte entry (the padding too, so that no 32-byte sector of the line is left partly written).
     e[0] = make_uint4(__float_as_uint(cost[0]), __float_as_uint(cost[1]), __float_as_uint(cost[2]),
                       __float_as_uint(cost[3]));
     e[1] = make_uint4(__float_as_uint(cost[4]), __float_as_uint(cost[5]), __float_as_uint(cost[6]), num_primitives);
@@ -215,6 +212,16 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint
     e[7] = make_uint4(0u, 0u, 0u, 0u);
     // checked last, so that the records' loads do not wait for the leaf counts (bvh2_to_cwbvh.rs:243-247)
     return l.prim_count > 1u || r.prim_count > 1u ? DERR_CW_NONUNIT_LEAF : 0u;
+}
+
+__device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint32_t first, const DpChild& l,
+                                                const DpChild& r, const DpRaw& raw_l, const DpRaw& raw_r) {
+    uint4 e[8];
+    const uint32_t err = dp_entry(dp, ha, l, r, raw_l, raw_r, e);
+    uint4* rec = reinterpret_cast<uint4*>(&dp.rec[dp_key(dp, first)]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) rec[k] = e[k];
+    return err;
 }
 
 // The record to load for a child.  A leaf has none: the table's first is read in its place (a line every lane shares)
@@ -241,6 +248,40 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, float ha, uint
 __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                 const Node32& r) {
     return dp_evaluate(dp, half_area(box), first, dp_child(l), dp_child(r));
+}
+
+// The same by a whole wave, the entries written eight lanes to a record through buf (2 KB of LDS of the wave's own): a
+// lane that stores its own record touches another line with every 16 bytes, 64 requests of a store instruction where
+// eight lanes a record make 16.  Lanes without an entry: valid false, any leaves.
+__device__ __forceinline__ uint32_t dp_evaluate_wave(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
+                                                     const Node32& r, bool valid, uint4* buf) {
+    const DpChild cl = dp_child(l), cr = dp_child(r);
+    const DpRaw raw_l = load_dp_raw(dp_child_record(dp, cl)), raw_r = load_dp_raw(dp_child_record(dp, cr));
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 e[8];
+    const uint32_t err = dp_entry(dp, half_area(box), cl, cr, raw_l, raw_r, e);
+    const uint32_t lane = __lane_id(), key = (uint32_t)dp_key(dp, first);
+    const uint64_t entries = __ballot(valid);
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q) {  // 16 records at a time
+        if (((entries >> (16u * q)) & 0xffffull) == 0ull) continue;
+        if ((lane >> 4) == q) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) buf[(lane & 15u) * 8u + (k ^ (lane & 7u))] = e[k];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h) {
+            const uint32_t rec = h * 8u + (lane >> 3), from = 16u * q + rec, part = lane & 7u;
+            const uint4 v = buf[rec * 8u + (part ^ (rec & 7u))];
+            const uint32_t to = (uint32_t)__shfl((int)key, (int)from);
+            if ((entries >> from) & 1ull) reinterpret_cast<uint4*>(&dp.rec[to])[part] = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    return valid ? err : 0u;
 }
 
 // The root's part of the evaluated table (1 and 1 for a single-leaf BVH2).

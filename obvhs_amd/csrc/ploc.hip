@@ -807,7 +807,7 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
                                              const DpView& dp, uint32_t fused, const uint32_t* __restrict__ slot_map,
                                              uint32_t vtop, uint32_t map_len, uint32_t* __restrict__ err,
                                              uint32_t* we, uint32_t* wm) {
-    __shared__ Node32 s_left[MAX_TILE_MERGES], s_right[MAX_TILE_MERGES];
+    __shared__ __align__(16) Node32 s_left[MAX_TILE_MERGES], s_right[MAX_TILE_MERGES];
     __shared__ uint32_t s_first[MAX_TILE_MERGES];
     const uint64_t be = __ballot(emit), bm = __ballot(mrg);
     const uint64_t lt = lanemask_lt();
@@ -847,11 +847,24 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
     if (!fused) return;  // uniform
     lds_barrier();
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
-    if (threadIdx.x < nm && s_first[threadIdx.x] != UINT32_MAX) {
-        const Node32 l = s_left[threadIdx.x], r = s_right[threadIdx.x];
-        const uint32_t e = dp_evaluate(dp, box_union(node_box(l), node_box(r)), s_first[threadIdx.x], l, r);
-        if (e) atomicOr(err, e);
+    if (wave * 64u >= nm) return;
+    const bool entry = threadIdx.x < nm && s_first[threadIdx.x] != UINT32_MAX;
+    Node32 l{}, r{};
+    l.prim_count = r.prim_count = 1u;
+    uint32_t first = 0u;
+    if (entry) {
+        l = s_left[threadIdx.x];
+        r = s_right[threadIdx.x];
+        first = s_first[threadIdx.x];
     }
+    const Box box = box_union(node_box(l), node_box(r));
+    uint32_t e;
+    if (wave < 2u) {  // the wave's entries of s_left are in its lanes' registers now: 2 KB of LDS
+        e = dp_evaluate_wave(dp, box, first, l, r, entry, reinterpret_cast<uint4*>(&s_left[wave * 64u]));
+    } else {
+        e = entry ? dp_evaluate(dp, box, first, l, r) : 0u;
+    }
+    if (e) atomicOr(err, e);
 }
 
 // Emits and merges of the first `n` groups, plus the lanes' own e and m, in every lane of the wave.
