@@ -595,9 +595,6 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
             const uint32_t s = offsets[blockIdx.x].y + tq - sg.mbase;
             const Node32 c = load_node(&cur[b]);
             const uint32_t first = sg.insert - 2u * (s + 1u);
-            Node32* mn = nodes + md.node_base;
-            store_node(&mn[first], a);
-            store_node(&mn[first + 1], c);
             store_node(&next[pos], make_node(box_union(node_box(a), node_box(c)), 0u, first));
             if (tq < MAX_TILE_MERGES) {
                 s_left[tq] = a;
@@ -614,6 +611,8 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     lds_barrier();  // the stores are not waited for
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
     if (wave * 64u >= nm) return;
+    store_pairs(s_left, s_right, wave, nm, nodes,
+                [&](uint32_t q) { return 2u * (size_t)s_kbase[q] + s_first[q]; });  // MeshDesc::node_base
     const bool entry = threadIdx.x < nm;
     Node32 l{}, r{};
     l.prim_count = r.prim_count = 1u;

@@ -188,6 +188,21 @@ __device__ __forceinline__ uint2 scan_chunk_apply(uint2* __restrict__ counts, ui
     return make_uint2(all_e, all_m);
 }
 
+// The children of a tile's merges [64 * wave, count) that are the wave's, 64 bytes each, from LDS to the child slots:
+// four lanes to a pair.  (A lane that stores its own pair touches another line with every 16 bytes.)  offset(q): the
+// slot of merge q's first child, SIZE_MAX for none.
+template <class Offset>
+__device__ __forceinline__ void store_pairs(const Node32* s_left, const Node32* s_right, uint32_t wave, uint32_t count,
+                                            Node32* __restrict__ nodes, Offset offset) {
+    const uint32_t lane = threadIdx.x & 63u, part = lane & 3u;
+    const uint32_t end = min(count, wave * 64u + 64u);
+    for (uint32_t q = wave * 64u + (lane >> 2); q < end; q += 16u) {
+        const float4* from = reinterpret_cast<const float4*>(part < 2u ? &s_left[q] : &s_right[q]);
+        const size_t at = offset(q);
+        if (at != SIZE_MAX) reinterpret_cast<float4*>(&nodes[at])[part] = from[part & 1u];
+    }
+}
+
 // Workgroups go round-robin to the 8 XCDs, each with its own L2.  The tile of a workgroup such that an XCD's
 // workgroups take one contiguous eighth of the tiles: for kernels whose neighbouring tiles read the same lines at
 // random (a 128-byte line holds four leaf records or parts of four triangles).  20M triangles in 4,096 meshes: leaf

@@ -833,8 +833,6 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
                 atomicOr(err, DERR_CAPACITY);
                 if (q < MAX_TILE_MERGES) s_first[q] = UINT32_MAX;
             } else {
-                store_node(&bvh_nodes[first], a);
-                store_node(&bvh_nodes[first + 1], c);
                 store_node(&next[pos], make_node(box_union(node_box(a), node_box(c)), 0u, first));
                 s_left[q] = a;
                 s_right[q] = c;
@@ -844,10 +842,12 @@ __device__ __forceinline__ void compact_tile(const Node32* __restrict__ cur, Nod
             store_node(&next[pos], a);
         }
     }
-    if (!fused) return;  // uniform
     lds_barrier();
     const uint32_t nm = min(wm[0] + wm[1] + wm[2] + wm[3], MAX_TILE_MERGES);
     if (wave * 64u >= nm) return;
+    store_pairs(s_left, s_right, wave, nm, bvh_nodes,
+                [&](uint32_t q) { return s_first[q] == UINT32_MAX ? SIZE_MAX : (size_t)s_first[q]; });
+    if (!fused) return;  // uniform
     const bool entry = threadIdx.x < nm && s_first[threadIdx.x] != UINT32_MAX;
     Node32 l{}, r{};
     l.prim_count = r.prim_count = 1u;
