@@ -1258,7 +1258,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_ploc_tail(const Node32* __rest
                            vtop, map_len, &misc->err);
     if (threadIdx.x == 0) {
         misc->state[slot] = st;
-        if (fused) misc->info = root_info(bvh_nodes, dp);
+        if (fused && st.insert == 1u) misc->info = root_info(bvh_nodes, dp);  // a finished tree
     }
 }
 
