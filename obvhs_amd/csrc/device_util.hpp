@@ -48,6 +48,14 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The same inside a wave, for lanes that read what other lanes of it wrote to LDS, or overwrite what they read: the
+// hardware keeps a wave's LDS accesses in order, and this keeps the compiler's.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // morton.rs:35-43
 __device__ __forceinline__ uint64_t split_by_3_u64(uint32_t a) {
     uint64_t x = (uint64_t)a & 0x1fffffull;

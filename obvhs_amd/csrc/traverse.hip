@@ -24,6 +24,7 @@
 
 #include "common.hpp"
 #include "cwdp.hpp"
+#include "device_util.hpp"
 #include "internal.hpp"
 
 #ifndef TRAV_LDS_STACK
@@ -630,6 +631,7 @@ __global__ void __launch_bounds__(TRAV_THREADS)
                 }
                 total += (uint32_t)__popcll(m);
             }
+            wave_lds_fence();  // the list is read by other lanes than wrote it
             for (uint32_t b = 0; b < total; b += TRAV_THREADS) {
                 const uint32_t e = b + lane < total ? tests[b + lane] : 0x80000000u;
                 const int owner = (int)(e & 63u);
@@ -647,6 +649,7 @@ __global__ void __launch_bounds__(TRAV_THREADS)
                     tests[b + lane] = __float_as_uint(t);
                 }
             }
+            wave_lds_fence();  // and so are the results
 #pragma unroll
             for (uint32_t k = 0; k < TESTS_PER_STEP; ++k) {
                 if (prim.y != 0u && !done) {
@@ -656,6 +659,7 @@ __global__ void __launch_bounds__(TRAV_THREADS)
                     if (t >= r.tmin) result(prim.x + local, t);
                 }
             }
+            wave_lds_fence();  // the next step writes its list over them
         }
         if (live) {
             if (!done) {
