@@ -20,6 +20,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "device_util.hpp"
 #include "internal.hpp"
 
 namespace obvhs {
@@ -263,6 +264,7 @@ __device__ __forceinline__ uint32_t dp_evaluate_wave(const DpView& dp, const Box
     const uint32_t err = dp_entry(dp, half_area(box), cl, cr, raw_l, raw_r, e);
     const uint32_t lane = __lane_id(), key = (uint32_t)dp_key(dp, first);
     const uint64_t entries = __ballot(valid);
+    wave_lds_fence();  // buf may hold what lanes of the wave have just read as something else
 #pragma unroll
     for (uint32_t q = 0; q < 4u; ++q) {  // 16 records at a time
         if (((entries >> (16u * q)) & 0xffffull) == 0ull) continue;
@@ -270,8 +272,7 @@ __device__ __forceinline__ uint32_t dp_evaluate_wave(const DpView& dp, const Box
 #pragma unroll
             for (uint32_t k = 0; k < 8u; ++k) buf[(lane & 15u) * 8u + (k ^ (lane & 7u))] = e[k];
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (uint32_t h = 0; h < 2u; ++h) {
             const uint32_t rec = h * 8u + (lane >> 3), from = 16u * q + rec, part = lane & 7u;
@@ -279,8 +280,7 @@ __device__ __forceinline__ uint32_t dp_evaluate_wave(const DpView& dp, const Box
             const uint32_t to = (uint32_t)__shfl((int)key, (int)from);
             if ((entries >> from) & 1ull) reinterpret_cast<uint4*>(&dp.rec[to])[part] = v;
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
     return valid ? err : 0u;
 }
