@@ -469,7 +469,7 @@ __global__ void __launch_bounds__(SMALL_THREADS)
         uint32_t key[SMALL_ITEMS], rank[SMALL_ITEMS];
         uint16_t val[SMALL_ITEMS];
         for (uint32_t d = lane; d < 256u; d += 64u) whist[wave][d] = 0u;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int j = 0; j < SMALL_ITEMS; ++j) {
             const uint32_t p = wave * (64u * SMALL_ITEMS) + (uint32_t)j * 64u + lane;
@@ -487,9 +487,9 @@ __global__ void __launch_bounds__(SMALL_THREADS)
             const uint32_t below = (uint32_t)__popcll(peers & lt);
             uint32_t at = 0u;
             if (valid) at = whist[wave][d];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             if (valid && below == 0u) whist[wave][d] = at + (uint32_t)__popcll(peers);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             rank[j] = at + below;
         }
         __syncthreads();
@@ -1111,7 +1111,7 @@ __global__ void __launch_bounds__(PASS_THREADS)
         }
     }
     if ((t & 63u) == 0u) w_nan[t >> 6] = 0u;
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_fence();
     if (nan_here) w_nan[t >> 6] = 1u;
     lds_barrier();
     uint32_t any_nan = 0u;

@@ -165,9 +165,9 @@ __global__ void __launch_bounds__(SORT_THREADS)
         uint32_t below = (uint32_t)__popcll(peers & lt);
         uint32_t base = 0;
         if (valid) base = whist[wave][d];
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         if (valid && below == 0) whist[wave][d] = base + (uint32_t)__popcll(peers);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         rank[j] = base + below;
     }
     __syncthreads();
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(ONE_THREADS)
     for (uint32_t pass = 0; pass < passes; ++pass) {
         const uint32_t shift = pass * 8u;
         for (uint32_t i = lane; i < 256u; i += 64u) whist[wave][i] = 0u;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
             const bool valid = seg + j * 64 + lane < n;
@@ -258,9 +258,9 @@ __global__ void __launch_bounds__(ONE_THREADS)
             const uint32_t below = (uint32_t)__popcll(peers & lt);
             uint32_t base = 0;
             if (valid) base = whist[wave][d];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             if (valid && below == 0) whist[wave][d] = base + (uint32_t)__popcll(peers);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             rank[j] = base + below;
         }
         __syncthreads();

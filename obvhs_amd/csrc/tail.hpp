@@ -382,7 +382,7 @@ __device__ __forceinline__ void ploc_tail(const Node32* __restrict__ cur, PlocSt
             uint32_t ah = ht[lane];
             const float4 blo = lo[b], bhi = hi[b];
             const uint32_t bh = ht[b];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             const uint32_t nm = (uint32_t)__popcll(bm);
             if (mrg) {
                 const uint32_t pm = (uint32_t)__popcll(bm & lt);
@@ -397,7 +397,7 @@ __device__ __forceinline__ void ploc_tail(const Node32* __restrict__ cur, PlocSt
                 ht[pe] = (uint16_t)ah;
             }
             if (lane < MAX_RADIUS) lo[count + lane] = hi[count + lane] = nan4();
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             merges += nm;
             insert -= 2u * nm;
             depth += 1u;
