@@ -1656,6 +1656,9 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     uint64_t* keys = S.keys.as<uint64_t>();
     uint64_t* keys_hi = u128 ? S.keys_hi.as<uint64_t>() : nullptr;
     uint32_t* hist = bvh->hist.as<uint32_t>();
+    // From here on the nodes change: a rebuild that fails leaves no tree in pass order, and no cost table.
+    bvh->pass_ordered = false;
+    bvh->dp_max_prims = 0;
     // The clusters are copied out first: merges may overwrite the freed slots they came from.
     k_gather<<<nblk, T256, 0, st>>>(bvh_nodes, d_src_slots, k, leaves);
     k_init_misc<<<1, 64, 0, st>>>(misc, k, hist);
