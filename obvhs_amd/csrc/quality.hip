@@ -358,7 +358,11 @@ __global__ void __launch_bounds__(T256) k_depths(const Node32* __restrict__ node
     if (i < n) {
         const bool inner = load_node(&nodes[i]).prim_count == 0u;
         uint32_t d = 0u;
-        for (uint32_t x = i; x != 0u && d < MAX_WALK; ++d) x = parents[x];
+        // a slot that no node refers to has no parent: what stands there may lead nowhere
+        for (uint32_t x = i; x != 0u && d < MAX_WALK; ++d) {
+            x = parents[x];
+            if (x >= n) d = MAX_WALK - 1u;
+        }
         if (inner && d < MAX_WALK) atomicAdd(&count[d], 1u);
         atomicMax(&deepest, d);
         depths[i] = (uint16_t)(inner ? d : MAX_WALK);
