@@ -228,8 +228,9 @@ __global__ void __launch_bounds__(T256) k_b_gather(const Node32* __restrict__ le
 // a leaf among others of the same top word ranks itself among them by the whole codes, ties in sorted (leaf) order.
 // The leaf records read at random bound it.  20M triangles in 4,096 icospheres (20 bits of code each): this sort and
 // gather 1.23 ms, against 3.27 for the sorts of 63-bit codes and of mesh numbers, the mesh keys between them and
-// k_b_gather.  A run longer than RUN_MAX on one side of a member sets DERR_RESORT and leaves no cluster to the
-// passes that are already enqueued.
+// k_b_gather.  A run longer than RUN_MAX on one side of a member sets DERR_RESORT and leaves no cluster to the passes
+// that are already enqueued; all meshes are then sorted by their whole codes (one such mesh among those icospheres:
+// build 8.2 -> 11.5 ms).
 constexpr uint32_t RUN_MAX = 64;
 
 __global__ void __launch_bounds__(T256) k_b_gather_runs(const Node32* __restrict__ leaves,
@@ -240,13 +241,16 @@ __global__ void __launch_bounds__(T256) k_b_gather_runs(const Node32* __restrict
     constexpr uint32_t WIN = T256 + 2 * RUN_MAX;
     __shared__ uint32_t tk[WIN];
     __shared__ uint64_t code[WIN];  // of the members of runs
+    __shared__ bool flagged;
     const uint32_t base = xcd_tile() * T256;
     if (base >= n) return;
     // window slot w holds sorted position base - RUN_MAX + w
     const uint32_t w0 = base < RUN_MAX ? RUN_MAX - base : 0u;  // first slot inside the array
     const uint32_t w1 = min(WIN, n - base + RUN_MAX);          // end of the slots inside it
     for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) tk[w] = tops[base + w - RUN_MAX];
+    if (threadIdx.x == 0) flagged = resort_flagged(&misc->err);
     __syncthreads();
+    if (flagged) return;  // the host sorts again
     for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) {
         const uint32_t t = tk[w];
         if ((w > w0 && tk[w - 1] == t) || (w + 1 < w1 && tk[w + 1] == t)) code[w] = keys[order[base + w - RUN_MAX]];
@@ -260,8 +264,7 @@ __global__ void __launch_bounds__(T256) k_b_gather_runs(const Node32* __restrict
     uint32_t a = me, b = me;  // the run's first and last slot
     while (a > w0 && me - a < RUN_MAX && tk[a - 1] == t) --a;
     while (b + 1 < w1 && b - me < RUN_MAX && tk[b + 1] == t) ++b;
-    if (me - a == RUN_MAX || b - me == RUN_MAX) {
-        atomicOr(&misc->err, DERR_RESORT);
+    if (flag_resort(me - a == RUN_MAX || b - me == RUN_MAX, &misc->err)) {
         misc->total[0] = 0u;
         return;
     }

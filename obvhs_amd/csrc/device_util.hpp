@@ -211,6 +211,17 @@ __device__ __forceinline__ void store_pairs(const Node32* s_left, const Node32* 
     }
 }
 
+// Whether DERR_RESORT is set in the word (by some workgroup, as far as this one sees).
+__device__ __forceinline__ bool resort_flagged(const uint32_t* err) {
+    return (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & DERR_RESORT) != 0u;
+}
+// Sets it if one of the calling lanes asks for it (`mine`): one atomic a wave at most.  Returns `mine`.
+__device__ __forceinline__ bool flag_resort(bool mine, uint32_t* err) {
+    const uint64_t lanes = __ballot(mine);
+    if (mine && (lanes & lanemask_lt()) == 0ull && !resort_flagged(err)) atomicOr(err, DERR_RESORT);
+    return mine;
+}
+
 // Workgroups go round-robin to the 8 XCDs, each with its own L2.  The tile of a workgroup such that an XCD's
 // workgroups take one contiguous eighth of the tiles: for kernels whose neighbouring tiles read the same lines at
 // random (a 128-byte line holds four leaf records or parts of four triangles).  20M triangles in 4,096 meshes: leaf

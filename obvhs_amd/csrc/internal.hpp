@@ -118,6 +118,9 @@ struct obvhs_bvh2 {
     // Children are stored in PLOC pass order (the pass ranges in hist order the nodes bottom-up); false after
     // reinsertion, when bottom-up sweeps use the level lists instead.
     bool pass_ordered = true;
+    // The leaves' codes had long runs of equal tops when the tree was last built (ploc.hip): its rebuilds, over the same
+    // leaves or some of their ancestors, sort by whole codes at once.
+    bool long_runs = false;
 };
 
 struct obvhs_cwbvh {

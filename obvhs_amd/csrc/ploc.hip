@@ -6,7 +6,7 @@
 //                    order-preserving keys; the zero sign of the bounds cannot change a Morton code)
 //   k_morton       : 63-bit Morton code of the f32 centre normalised in f64 (ploc/mod.rs:287-288, 782-785;
 //                    morton.rs:35-58), or the 126-bit code of SortPrecision::U128 (morton.rs:63-89) as two words
-//   radix sort     : stable (sort.hip); a U128 key is sorted by its low word, then stably by its high word
+//   radix sort     : stable (sort.hip), by the code's top 32 bits
 //   k_gather       : sorted leaves become the first cluster array (ploc/mod.rs:829-846)
 //   per pass       : k_ploc_search_count (ploc/mod.rs:329-419, window in LDS, and the per-tile counts of emitted
 //                    clusters and merges), their prefix sums in two launches over chunks for the largest passes,
@@ -264,12 +264,13 @@ __global__ void __launch_bounds__(T256) k_morton(const Node32* __restrict__ leav
     tops[i] = top_of_u64(code);
 }
 
-__global__ void __launch_bounds__(T256) k_gather_u64(const uint64_t* __restrict__ src,
-                                                     const uint32_t* __restrict__ order, uint32_t n,
-                                                     uint64_t* __restrict__ out) {
+// `bits` bits of the codes' words from `shift` up, in the given order (NULL: leaf order).
+__global__ void __launch_bounds__(T256) k_code_words(const uint64_t* __restrict__ src,
+                                                     const uint32_t* __restrict__ order, uint32_t n, uint32_t shift,
+                                                     uint32_t bits, uint32_t* __restrict__ out) {
     const uint32_t i = blockIdx.x * T256 + threadIdx.x;
     if (i >= n) return;
-    out[i] = src[order[i]];
+    out[i] = (uint32_t)(src[order ? order[i] : i] >> shift) & (0xffffffffu >> (32u - bits));
 }
 
 __global__ void __launch_bounds__(T256) k_gather(const Node32* __restrict__ leaves,
@@ -286,7 +287,10 @@ __global__ void __launch_bounds__(T256) k_gather(const Node32* __restrict__ leav
 // whole codes.  Runs are short (the tops are cells of 10 or 11 bits per axis: 1 to 12 leaves a run on the benchmark's
 // heightfields of 1.3M and 17.3M triangles).  A run longer than RUN_MAX (or that long on one side of a member) sets
 // DERR_RESORT and leaves one cluster in the pass state, which turns the passes behind this launch into no-ops; the
-// host then sorts the whole codes.
+// host then sorts the whole codes.  Such a scene (a dense object in a large extent, duplicated geometry) pays for the
+// first sort, the launches without work and a host wait: 16.8M leaves in a 500th of their box 7.5 ms against 5.9 for
+// an evenly filled one (20.1 when every member of a run set the flag by an atomic of its own, which a workgroup that
+// finds it set now skips with all its work), 1M 1.24 ms, 65,536 0.68 (0.53 evenly filled).
 // Bound by the random 32-byte leaf reads.  1,288,352 leaves: 23 us against the plain gather's 16, and with it the sort
 // takes 4 passes of 20 bytes per key instead of 8 of 32 (198 -> 98 us).
 // order_out (may be NULL): the final permutation.
@@ -303,13 +307,16 @@ __global__ void __launch_bounds__(T256) k_gather_runs(const Node32* __restrict__
     __shared__ uint32_t tk[WIN];
     __shared__ uint32_t rest[WIN];                  // the bits below the top: 31, or 30 of the high word
     __shared__ uint64_t low[WIDE ? WIN : 1];        // the low word of a 126-bit code
+    __shared__ bool flagged;
     const uint32_t base = xcd_tile() * T256;
     if (base >= n) return;
     // window slot w holds sorted position base - RUN_MAX + w
     const uint32_t w0 = base < RUN_MAX ? RUN_MAX - base : 0u;             // first slot inside the array
     const uint32_t w1 = min(WIN, n - base + RUN_MAX);                     // end of the slots inside it
     for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) tk[w] = tops[base + w - RUN_MAX];
+    if (threadIdx.x == 0) flagged = resort_flagged(&misc->err);
     __syncthreads();
+    if (flagged) return;  // the host sorts again
     for (uint32_t w = w0 + threadIdx.x; w < w1; w += T256) {
         const uint32_t t = tk[w];
         if ((w > w0 && tk[w - 1] == t) || (w + 1 < w1 && tk[w + 1] == t)) {
@@ -329,8 +336,7 @@ __global__ void __launch_bounds__(T256) k_gather_runs(const Node32* __restrict__
     uint32_t a = me, b = me;  // the run's first and last slot
     while (a > w0 && me - a < RUN_MAX && tk[a - 1] == t) --a;
     while (b + 1 < w1 && b - me < RUN_MAX && tk[b + 1] == t) ++b;
-    if (me - a == RUN_MAX || b - me == RUN_MAX) {
-        atomicOr(&misc->err, DERR_RESORT);
+    if (flag_resort(me - a == RUN_MAX || b - me == RUN_MAX, &misc->err)) {
         misc->state[0].count = 1u;
         return;
     }
@@ -1290,23 +1296,30 @@ void DevBuf::release() {
         if (_e != hipSuccess) return set_hip_error(ctx, _e, where);         \
     } while (0)
 
-// Sorts the leaf indices vals[0..n) (identity on entry) by their Morton codes, ties in leaf order
-// (ploc/mod.rs:811-827).  U64: one sort of the 63-bit codes in keys.  U128 (keys_hi != NULL): LSD over the whole
-// 126-bit key as a stable sort of the low words followed by a stable sort of the high words (62 bits) gathered in
-// that order; keys ends up holding the sorted high words.
-static obvhs_status sort_codes(obvhs_context* ctx, uint64_t* keys, const uint64_t* keys_hi, uint32_t* vals,
+// Sorts the leaf indices vals[0..n) by their whole Morton codes, ties in leaf order (ploc/mod.rs:811-827): stable sorts
+// by 32 bits of the code at a time, the lowest first, the words gathered in the order so far.  The codes stay in leaf
+// order.  Eight passes of 20 bytes a key and two gathers (16.8M leaves: 1.23 ms) where a sort of 64-bit keys makes
+// eight of 32 bytes.
+static obvhs_status sort_codes(obvhs_context* ctx, const uint64_t* keys, const uint64_t* keys_hi, uint32_t* vals,
                                uint32_t n) {
     hipStream_t st = ctx->stream;
-    void* scratch = ctx->scratch.sort_scratch.ptr;
-    const int items = sort_items_for(ctx, n);
-    if (!keys_hi) {
-        OBVHS_TRY(radix_sort_pairs(keys, vals, true, n, 63, scratch, st, items), "radix sort");
-        return OBVHS_OK;
+    BuildScratch& S = ctx->scratch;
+    uint32_t* words = S.tops.as<uint32_t>();
+    struct Word {
+        const uint64_t* from;
+        uint32_t shift, bits;
+    };
+    const Word u64[2] = {{keys, 0u, 31u}, {keys, 31u, 32u}};
+    const Word u128[4] = {{keys, 0u, 32u}, {keys, 32u, 32u}, {keys_hi, 0u, 30u}, {keys_hi, 30u, 32u}};
+    const Word* const w = keys_hi ? u128 : u64;
+    for (int k = 0; k < (keys_hi ? 4 : 2); ++k) {
+        k_code_words<<<(n + T256 - 1) / T256, T256, 0, st>>>(w[k].from, k ? vals : nullptr, n, w[k].shift, w[k].bits,
+                                                             words);
+        OBVHS_TRY(hipGetLastError(), "code words");
+        OBVHS_TRY(radix_sort_pairs32(words, vals, k == 0, n, (int)w[k].bits, S.sort_scratch.ptr, st,
+                                     sort_items_for(ctx, n)),
+                  "radix sort (whole codes)");
     }
-    OBVHS_TRY(radix_sort_pairs(keys, vals, true, n, 64, scratch, st, items), "radix sort (low words)");
-    k_gather_u64<<<(n + T256 - 1) / T256, T256, 0, st>>>(keys_hi, vals, n, keys);
-    OBVHS_TRY(hipGetLastError(), "gather high words");
-    OBVHS_TRY(radix_sort_pairs(keys, vals, false, n, 62, scratch, st, items), "radix sort (high words)");
     return OBVHS_OK;
 }
 
@@ -1333,7 +1346,7 @@ static obvhs_status sort_gather(obvhs_context* ctx, const Node32* leaves, const 
 }
 
 // The same by a sort of the whole codes, after sort_gather met a long run (DERR_RESORT): the pass state starts over.
-static obvhs_status resort_gather(obvhs_context* ctx, const Node32* leaves, uint64_t* keys, const uint64_t* keys_hi,
+static obvhs_status resort_gather(obvhs_context* ctx, const Node32* leaves, const uint64_t* keys, const uint64_t* keys_hi,
                                   uint32_t n, Node32* cur, uint32_t* order_out) {
     hipStream_t st = ctx->stream;
     BuildScratch& S = ctx->scratch;
@@ -1608,6 +1621,7 @@ obvhs_status ploc_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const 
     bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, n, search_distance, search_depth_threshold, bvh_nodes, hist, dp,
                                  fused, nullptr, 0u, 0u, fin, resort, info);
+    bvh->long_runs = resort;
     if (ps == OBVHS_OK && resort) {
         ps = resort_gather(ctx, leaves, keys, keys_hi, n, cur, order_out);
         if (ps == OBVHS_OK)
@@ -1667,13 +1681,17 @@ obvhs_status ploc_rebuild(obvhs_context* ctx, obvhs_bvh2* bvh, const uint32_t* d
     OBVHS_TRY(hipGetLastError(), "rebuild morton launch");
     Node32* cur = S.clusters_a.as<Node32>();
     Node32* nxt = S.clusters_b.as<Node32>();
-    const obvhs_status ss = sort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
+    // A tree that met long runs is not tried by its tops again: 1M leaves in a thousandth of their box, 2% of the leaves
+    // rebuilt 884 -> 747 us, all 949 -> 757.
+    const obvhs_status ss = bvh->long_runs ? resort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr)
+                                           : sort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
     if (ss != OBVHS_OK) return ss;
     PlocState fin{};
     bool resort = false;
     obvhs_status ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist,
                                  DpView{}, 0u, d_slot_map, 2u * k - 3u, k - 1u, fin, resort, nullptr);
     if (ps == OBVHS_OK && resort) {
+        bvh->long_runs = true;
         ps = resort_gather(ctx, leaves, keys, keys_hi, k, cur, nullptr);
         if (ps == OBVHS_OK)
             ps = run_passes(ctx, cur, nxt, k, search_distance, search_depth_threshold, bvh_nodes, hist, DpView{}, 0u,

@@ -210,6 +210,7 @@ obvhs_status run_update(obvhs_server* S, obvhs_context* ctx, Scene* sc, Req* r, 
         d->ploc_iterations = b->ploc_iterations;
         d->cluster_sum = b->cluster_sum;
         d->pass_ordered = b->pass_ordered;
+        d->long_runs = b->long_runs;
         d->dp_max_prims = 0;
         s = bvh2_refit_from_triangles(ctx, d, dst.tris.as<obvhs_triangle>());
         uint32_t mp = sc->params.max_prims_per_leaf;
