@@ -23,11 +23,11 @@
 #include <new>
 #include <vector>
 
+#include "batch.hpp"
 #include "common.hpp"
 #include "cwdp.hpp"
 #include "device_util.hpp"
 #include "internal.hpp"
-#include "tail.hpp"
 
 struct obvhs_batch {
     obvhs::DevBuf tri_offsets;    // u32[m+1]
@@ -50,26 +50,6 @@ namespace {
 constexpr int T256 = 256;
 // Passes between host reads; 8 and 16 measured slower here (16.1 -> 16.8 and 18.3 ms): grids sized at the last read.
 constexpr int PASSES_PER_SYNC = 4;
-// Clusters of a mesh that one workgroup takes over (k_b_tail).
-constexpr int B_TAIL_MAX = 1024;
-
-struct SegState {
-    uint32_t start;   // first cluster of the mesh in the current cluster array
-    uint32_t count;   // clusters of the mesh
-    uint32_t insert;  // next free child slot + 1 (mesh-local), ploc/mod.rs:283-284
-    uint32_t mbase;   // global exclusive merge count at the segment's first cluster (current pass)
-};
-
-// The cluster count is double-buffered by pass parity q: pass p reads total[p & 1] and its scan writes the next
-// pass's count into total[(p + 1) & 1], so no launch is needed between passes to move it.
-struct BatchMisc {
-    uint32_t err;
-    uint32_t total[2];   // clusters in the current array (by pass parity)
-    uint32_t large;      // 1 if a mesh has more than B_TAIL_MAX clusters after the last pass, else 0
-    uint32_t totals[2];  // emits, merges of the pass
-    uint32_t passes;     // of the mesh that took most
-};
-
 __device__ __forceinline__ uint32_t mesh_in(const uint32_t* __restrict__ offsets, uint32_t lo, uint32_t hi,
                                             uint32_t g) {
     // offsets[lo] <= g < offsets[hi]
@@ -640,34 +620,6 @@ __global__ void __launch_bounds__(T256) k_b_compact(const Node32* __restrict__ c
     if (e) atomicOr(&misc->err, e);
 }
 
-// The remaining passes of every mesh of search distance r, one workgroup per mesh (tail.hpp), once no mesh has more
-// than B_TAIL_MAX clusters; its last cluster goes to the mesh's node 0 (ploc/mod.rs:495-499).  R: r if that distance
-// has an unrolled search, else 0.
-// A mesh's chain of passes bounds a workgroup, not any throughput; two of them fit a CU's LDS.  4,096 icospheres of up
-// to 20,480 triangles: passes 16 to 48 in 321 us, about 0.8 ms as launches over all meshes (build 10.17 -> 9.69 ms).
-template <int R>
-__global__ void __launch_bounds__(B_TAIL_MAX / 2, 4) k_b_tail(const Node32* __restrict__ cur,
-                                                           const SegState* __restrict__ seg, BatchMisc* misc,
-                                                           const MeshDesc* __restrict__ meshes, uint32_t r,
-                                                           uint32_t first_pass, uint32_t depth_threshold,
-                                                           Node32* __restrict__ nodes, DpView dp, uint32_t q) {
-    const MeshDesc md = meshes[blockIdx.x];
-    const SegState sg = seg[blockIdx.x];
-    if (md.prim_count == 0u || md.radius != r || misc->total[q] == 0u) return;  // total 0: DERR_RESORT
-    if (sg.count == 0u || sg.count > (uint32_t)B_TAIL_MAX) {
-        if (threadIdx.x == 0) atomicOr(&misc->err, DERR_CAPACITY);
-        return;
-    }
-    dp.kbase = md.prim_base;
-    PlocState st{sg.count, sg.insert, first_pass, 0u, 0ull};
-    ploc_tail<R, B_TAIL_MAX>(cur + sg.start, st, first_pass, r, r == 1u ? 1u : 0u, depth_threshold,
-                             nodes + md.node_base, nullptr, dp, 1u, nullptr, 0u, 0u, &misc->err);
-    if (threadIdx.x == 0) {
-        if (st.count != 1u || st.insert != 1u) atomicOr(&misc->err, DERR_SELF_MERGE);
-        atomicMax(&misc->passes, st.depth);
-    }
-}
-
 // Root box of every mesh's BVH2 (the BLAS bounds a TLAS is built over), as Aabb records.
 __global__ void __launch_bounds__(T256) k_b_root_boxes(const Node32* __restrict__ nodes,
                                                        const MeshDesc* __restrict__ meshes, uint32_t m,
@@ -686,23 +638,6 @@ __global__ void __launch_bounds__(T256) k_b_root_boxes(const Node32* __restrict_
         hipError_t _e = (expr);                                     \
         if (_e != hipSuccess) return set_hip_error(ctx, _e, where); \
     } while (0)
-
-// The tail for the search distance (each allowed distance has its unrolled instance).
-static void launch_tail(hipStream_t st, const Node32* cur, const SegState* seg, BatchMisc* misc,
-                        const MeshDesc* meshes, uint32_t m, uint32_t r, uint32_t pass, uint32_t threshold,
-                        Node32* nodes, const DpView& dp, uint32_t q) {
-#define OBVHS_TAIL(RR) \
-    k_b_tail<RR><<<m, B_TAIL_MAX / 2, 0, st>>>(cur, seg, misc, meshes, r, pass, threshold, nodes, dp, q)
-    switch (r) {
-        case 2: OBVHS_TAIL(2); break;
-        case 6: OBVHS_TAIL(6); break;
-        case 14: OBVHS_TAIL(14); break;
-        case 24: OBVHS_TAIL(24); break;
-        case 32: OBVHS_TAIL(32); break;
-        default: OBVHS_TAIL(0); break;
-    }
-#undef OBVHS_TAIL
-}
 
 static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris, const uint32_t* h_offsets,
                                 uint32_t m, uint32_t r, uint32_t sdt, uint32_t max_prims, obvhs_batch* B) {
@@ -809,10 +744,10 @@ static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris
         if (ss != OBVHS_OK) return ss;
     }
 
-    // The search distances of the meshes, for the tail's launches.
-    bool has_radius[MAX_RADIUS + 1] = {};
+    // The meshes by search distance and class, for the tail's launches.
+    uint32_t has[MAX_RADIUS + 1][B_TAIL_CLASSES] = {};
     for (const MeshDesc& md : B->meshes)
-        if (md.prim_count) has_radius[md.radius] = true;
+        if (md.prim_count) has[md.radius][(md.prim_count > B_TAIL_SIZES[0]) + (md.prim_count > B_TAIL_SIZES[1])]++;
     uint32_t* h = static_cast<uint32_t*>(ctx->pinned);
     for (;;) {
         uint32_t known = n;
@@ -856,9 +791,22 @@ static obvhs_status batch_build(obvhs_context* ctx, const obvhs_triangle* d_tris
             known = now;
         }
         if (err == 0u) {
-            for (uint32_t rr = 1; rr <= MAX_RADIUS; ++rr)
-                if (has_radius[rr])
-                    launch_tail(st, cur, seg[cs], misc, d_meshes, m, rr, pass, sdt, nodes, dp, pass & 1u);
+            for (uint32_t rr = 1; rr <= MAX_RADIUS; ++rr) {
+                uint32_t above = 0u, waiting = 0u;  // meshes of more triangles than `above` have no launch yet
+                for (int c = 0; c < B_TAIL_CLASSES; ++c) {
+                    waiting += has[rr][c];
+                    uint32_t larger = 0u;
+                    for (int l = c + 1; l < B_TAIL_CLASSES; ++l) larger += has[rr][l];
+                    if (waiting == 0u || (larger != 0u && waiting < B_TAIL_OWN)) continue;
+                    const uint32_t upto = c + 1 < B_TAIL_CLASSES ? B_TAIL_SIZES[c] : UINT32_MAX;
+                    const BatchTail t{st, cur, seg[cs], misc, d_meshes, m, above, upto, rr, pass, sdt, nodes, dp,
+                                      pass & 1u};
+                    if (c + 1 < B_TAIL_CLASSES) launch_tail_small(c, t);
+                    else launch_tail<B_TAIL_MAX>(t);
+                    above = upto;
+                    waiting = 0u;
+                }
+            }
             OBVHS_TRY(hipGetLastError(), "batch tail launch");
             OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(BatchMisc), hipMemcpyDeviceToHost, st), "read batch state");
             OBVHS_TRY(hipStreamSynchronize(st), "batch tail sync");
