@@ -491,7 +491,10 @@ __device__ __forceinline__ bool row_coherent(const float4* __restrict__ rays, ui
 // flags; an owner without rows and a row that is not its workgroup's leave at once.  The line: primary rays whose
 // directions were spread, refilled against one lane per ray in us at a smallest cosine of 0.995 / 0.982 / 0.93 / 0.59
 // within the rows: heightfield 266 / 261 / 268 / 257 against 276 / 310 / 440 / 560, soup 276 / 293 / 316 / 296
-// against 252 / 293 / 515 / 950.
+// against 252 / 293 / 515 / 950.  The price on launches whose rows are all coherent, against one lane per ray alone:
+// 2.07M primary rays of 500 triangles 52.5 -> 57.9 us, of the soup 237 -> 249, of the heightfield 238 -> 237,
+// watertight (88 registers for 79) 293 -> 304; 2M incoherent rays of the heightfield gain 396 -> 215.  (Four samples a
+// row: 56.4, 247, 239, 301, but 1M shadow rays 185 -> 191.)
 // SRC_MESHES: as in k_traverse, each ray's mesh (ray_mesh) selects its CWBVH and triangle slices; node_count_in is
 // then the mesh count.
 template <int MODE, int LDS, int SRC = SRC_PLAIN>
