@@ -117,7 +117,8 @@ obvhs_status obvhs_context_set_trace(obvhs_context* ctx, int enable);
  *   ploc_radius[c]    : the PlocSearchDistance a build with search distance 0 ("auto") uses for a BVH of class c;
  *                       batched builds resolve it per mesh.  Changes the tree (each result equals the build with
  *                       that distance).  Default 14.
- *   sort_items[c]     : keys per thread of the radix sort's tiles (4, 8 or 16) for a sort of class c.  Default 8.
+ *   sort_items[c]     : keys per thread of the radix sort's tiles (4, 8 or 16) for a sort of class c.  Default 8.  Sorts
+ *                       of at most 8,192 32-bit keys (builds of as many leaves) have no tiles.
  *   trav_lds_depth[c] : traversal stack entries kept in LDS (4, 8 or 16) for a BVH of class c.  Default 8.
  *   trav_chunk[c]     : 1: a single-BVH traversal launch of at least 1.25 rows of 64 rays per resident wave gives each
  *                       wave interleaved rows of rays and refills a lane as soon as its ray ends; 0: only the rows
@@ -133,7 +134,8 @@ typedef struct obvhs_tune_table {
 uint32_t obvhs_size_class(uint64_t n);
 obvhs_status obvhs_tune_get(const obvhs_context* ctx, obvhs_tune_table* out);
 obvhs_status obvhs_tune_set(obvhs_context* ctx, const obvhs_tune_table* table); /* rejects values out of range */
-/* Times the radix sort of n seeded 63-bit keys with each tile size and stores the fastest in sort_items[class(n)]. */
+/* Times the radix sort of n seeded 32-bit keys, the builds' form, with each tile size and stores the fastest in
+ * sort_items[class(n)].  For n <= 8,192 there is nothing to time: the entry stays and is returned. */
 obvhs_status obvhs_tune_sort(obvhs_context* ctx, uint32_t n, uint32_t* out_items);
 /* Times closest-hit (any_hit = 0) or occlusion traversal of the given rays with each LDS depth, one lane per ray
  * and chunked, and stores the fastest in trav_lds_depth[class(prim count)] and trav_chunk[class(prim count)]. */

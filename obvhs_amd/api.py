@@ -792,7 +792,8 @@ def size_class(n):
 
 
 def tune_sort(ctx, n):
-    """Times the radix sort of n keys with each tile size; stores and returns the fastest (keys per thread)."""
+    """Times the radix sort of n keys with each tile size; stores and returns the fastest (keys per thread).  For n of
+    at most 8,192, sorted without tiles, the table's entry stays and is returned."""
     out = C.c_uint32()
     check(lib().obvhs_tune_sort(ctx.handle, int(n), C.byref(out)), ctx.handle)
     return out.value

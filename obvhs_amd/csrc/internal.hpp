@@ -140,6 +140,7 @@ hipError_t launch_iota(uint32_t* p, uint32_t n, hipStream_t stream);
 size_t radix_sort_scratch_bytes(uint32_t n);
 hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                             void* scratch, hipStream_t stream, int items);
+constexpr uint32_t SORT_ONE_MAX = 8192;  // u32 keys that one workgroup sorts, whatever the tile size
 hipError_t radix_sort_pairs32(uint32_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                               void* scratch, hipStream_t stream, int items);
 // Size class of n primitives or keys (the tuning table's index).

@@ -27,15 +27,15 @@ namespace obvhs {
 
 namespace {
 
-// Seeded 63-bit keys (an integer hash of the index), the shape of Morton codes for the sort timing.
-__global__ void k_tune_keys(uint64_t* keys, uint32_t n) {
+// Seeded 32-bit keys (an integer hash of the index), what the builds sort by (the codes' top words) for the sort timing.
+__global__ void k_tune_keys(uint32_t* keys, uint32_t n) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
     uint64_t x = (uint64_t)i * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
     x ^= x >> 31;
     x *= 0xBF58476D1CE4E5B9ull;
     x ^= x >> 29;
-    keys[i] = x >> 1;
+    keys[i] = (uint32_t)(x >> 32);
 }
 
 constexpr uint32_t CANDIDATE_TILES[3] = {4u, 8u, 16u};
@@ -101,13 +101,18 @@ obvhs_status obvhs_tune_sort(obvhs_context* ctx, uint32_t n, uint32_t* out_items
     if (!ctx || n == 0) return OBVHS_ERR_INVALID_ARG;
     TUNE_TRY(hipSetDevice(ctx->device), "set device");
     hipStream_t st = ctx->stream;
-    const size_t kb = ((size_t)n * 8 + 255) & ~(size_t)255, vb = ((size_t)n * 4 + 255) & ~(size_t)255;
-    TUNE_TRY(ctx->tune_scratch.ensure(2 * kb + vb + radix_sort_scratch_bytes(n)), "alloc tuning scratch");
+    const uint32_t cls = size_class(n);
+    if (n <= SORT_ONE_MAX) {  // one workgroup sorts them, without tiles: nothing to choose
+        if (out_items) *out_items = ctx->tune.sort_items[cls];
+        return OBVHS_OK;
+    }
+    const size_t kb = ((size_t)n * 4 + 255) & ~(size_t)255;
+    TUNE_TRY(ctx->tune_scratch.ensure(3 * kb + radix_sort_scratch_bytes(n)), "alloc tuning scratch");
     char* base = ctx->tune_scratch.as<char>();
-    uint64_t* keys0 = reinterpret_cast<uint64_t*>(base);
-    uint64_t* keys = reinterpret_cast<uint64_t*>(base + kb);
+    uint32_t* keys0 = reinterpret_cast<uint32_t*>(base);
+    uint32_t* keys = reinterpret_cast<uint32_t*>(base + kb);
     uint32_t* vals = reinterpret_cast<uint32_t*>(base + 2 * kb);
-    void* scratch = base + 2 * kb + vb;
+    void* scratch = base + 3 * kb;
     k_tune_keys<<<(n + 255) / 256, 256, 0, st>>>(keys0, n);
     TUNE_TRY(hipGetLastError(), "tuning keys");
     uint32_t best = 8u;
@@ -118,8 +123,8 @@ obvhs_status obvhs_tune_sort(obvhs_context* ctx, uint32_t n, uint32_t* out_items
             ctx,
             [&]() -> obvhs_status {
                 // the copy belongs to every candidate alike; the sort dominates
-                TUNE_TRY(hipMemcpyAsync(keys, keys0, (size_t)n * 8, hipMemcpyDeviceToDevice, st), "copy keys");
-                TUNE_TRY(radix_sort_pairs(keys, vals, true, n, 63, scratch, st, (int)items), "sort");
+                TUNE_TRY(hipMemcpyAsync(keys, keys0, (size_t)n * 4, hipMemcpyDeviceToDevice, st), "copy keys");
+                TUNE_TRY(radix_sort_pairs32(keys, vals, true, n, 32, scratch, st, (int)items), "sort");
                 return OBVHS_OK;
             },
             &ms);
@@ -129,7 +134,7 @@ obvhs_status obvhs_tune_sort(obvhs_context* ctx, uint32_t n, uint32_t* out_items
             best = items;
         }
     }
-    ctx->tune.sort_items[size_class(n)] = best;
+    ctx->tune.sort_items[cls] = best;
     if (out_items) *out_items = best;
     return OBVHS_OK;
 }
