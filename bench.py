@@ -144,10 +144,14 @@ def tune_step(ob, ctx, n_prims, step, reps=3, layouts=("triangle",)):
             "step_ms_by_lds_depth_chunked_layout": {f"{d}/{c}/{l}": round(v, 4) for (d, c, l), v in ms_by.items()}}
 
 
-def kernel_name(ctx, ob, n_prims, mode="closest"):
+CHUNK_MIN_RAYS = 256 * 16 * 64  # the MI355X's compute units x 16 waves: traversal launches of fewer rays are k_traverse
+
+
+def kernel_name(ctx, ob, n_prims, n_rays, mode="closest"):
     t = ctx.tune_table()
     cls = ob.size_class(n_prims)
-    return f"k_traverse_chunk<{mode}, lds {t['trav_lds_depth'][cls]}>"
+    form = "k_traverse" if (n_rays + 63) // 64 * 64 < CHUNK_MIN_RAYS else "k_traverse_chunk"
+    return f"{form}<{mode}, lds {t['trav_lds_depth'][cls]}>"
 
 
 def leg_counters(leg):
@@ -387,7 +391,7 @@ def bench_batch(args, ob, ctx):
             C.c_void_p(tv.ptr.value + i * rpm * 4)), ctx.handle)
     node_tests, tri_tests = int(nv.to_host().astype(np.int64).sum()), int(tv.to_host().astype(np.int64).sum())
     result["roofline"] = roofline(40 * n_rays + 80 * node_tests + 36 * tri_tests, trace_s * 1e3, None,
-                                  kernel_name(ctx, ob, n_tris // m), node_tests=node_tests, tri_tests=tri_tests,
+                                  kernel_name(ctx, ob, n_tris // m, n_rays), node_tests=node_tests, tri_tests=tri_tests,
                                   bytes_model="40 B per ray + 80 B per node test + 36 B per triangle test",
                                   timing="wall time per batched launch (one kernel), not HIP events")
     t0 = time.perf_counter()
@@ -540,7 +544,7 @@ def bench_large(args, ob, ctx):
         closest()
         ctx.synchronize()
         print(json.dumps({"pmc_probe": "large", "copy_bytes": PMC_COPY_BYTES, "closest_rays": nr,
-                          "kernel": kernel_name(ctx, ob, leaves)}), flush=True)
+                          "kernel": kernel_name(ctx, ob, leaves, nr)}), flush=True)
         return None
     # per-ray node / triangle test counts for the byte model (instrumented launch, not timed)
     _, nv, tv = cw.ray_traverse(d_rays, d_bvh_tris, counted=True)
@@ -562,7 +566,7 @@ def bench_large(args, ob, ctx):
         closest()
         kms.append(ctx.timer_stop())
     kernel_ms = float(np.mean(kms))
-    closest_kernel = kernel_name(ctx, ob, leaves, "closest, RtTriangle" if layout["value"] == "rt" else "closest")
+    closest_kernel = kernel_name(ctx, ob, leaves, nr, "closest, RtTriangle" if layout["value"] == "rt" else "closest")
 
     for _ in range(args.warmup):
         anyhit()
@@ -680,7 +684,7 @@ def bench_heightfield(args, ob, ctx):
         step()
         ctx.synchronize()
         print(json.dumps({"pmc_probe": "heightfield", "copy_bytes": PMC_COPY_BYTES, "primary_rays": len(prim_rays),
-                          "bounce_rays": len(bounce), "kernel": kernel_name(ctx, ob, n_tris)}), flush=True)
+                          "bounce_rays": len(bounce), "kernel": kernel_name(ctx, ob, n_tris, len(bounce))}), flush=True)
         return None
     _, nv_p, tv_p = cw.ray_traverse(d_prim, d_bvh_tris, counted=True)
     _, nv_b, tv_b = cw.ray_traverse(d_bounce, d_bvh_tris, counted=True)
@@ -709,7 +713,7 @@ def bench_heightfield(args, ob, ctx):
            "closest_mrays_per_s": round(n_rays * args.steps / wall / 1e6, 2),
            "ms_per_step": round(wall / args.steps * 1e3, 4),
            "roofline": roofline(algo_bytes / 2.0, kernel_ms, traffic_per_launch("heightfield"),
-                                kernel_name(ctx, ob, n_tris), counters=leg_counters("heightfield"),
+                                kernel_name(ctx, ob, n_tris, len(bounce)), counters=leg_counters("heightfield"),
                                 avg_kernel_ms_by_launch={"primary": round(float(np.mean(kp)), 4),
                                                          "bounce": round(float(np.mean(kb)), 4)},
                                 node_tests=node_tests, tri_tests=tri_tests),
