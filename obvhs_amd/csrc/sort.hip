@@ -14,7 +14,8 @@
 //               LDS (half the LDS of staging both at once, so twice the tiles per CU).
 // Up to FEW_TILES tiles the scan has no launch: the upsweep writes counts[tile][digit] and every tile of the downsweep
 // sums the digits' counts itself.  A sort of 26K keys (13 tiles) was 12 launches of 5 to 8 us, bound by latency; 32
-// such sorts of a reinsertion: 2.0 -> 1.5 ms.  At 49 tiles both forms take 55 us a sort.
+// such sorts of a reinsertion: 2.0 -> 1.5 ms.  At 49, 57 and 64 tiles the kernels take as long in either form (63 to
+// 65 us a sort), and four launches of twelve are spared.
 // Tiles are 256 threads x ITEMS keys (ITEMS = 4, 8 or 16, the sort tile the context's tuning table picks per size
 // class; 8 by default); each wave owns a contiguous 64 x ITEMS key segment.  Every tile size gives the same order.
 //
@@ -216,8 +217,8 @@ __global__ void __launch_bounds__(SORT_THREADS)
     }
 }
 
-// At most SORT_ONE_MAX u32 keys: the whole sort in one workgroup, keys and values in LDS between the passes (a wave owns 64 x
-// ITEMS consecutive keys, ranked as in the downsweep).  The ranking's instructions bound it: 2,048 keys 12 us, 4,096
+// At most SORT_ONE_MAX u32 keys: the whole sort in one workgroup, keys and values in LDS between the passes (a wave owns
+// 64 x ITEMS consecutive keys, ranked as in the downsweep).  The ranking's instructions bound it: 2,048 keys 12 us, 4,096
 // 19, 8,192 30, against 46 us and eight launches at any of these sizes.
 constexpr int ONE_THREADS = 1024;
 constexpr int ONE_WAVES = ONE_THREADS / 64;

@@ -12,3 +12,9 @@ pytestmark = pytest.mark.gpu
 def test_tile_merges(ctx, sd, sdt):
     """Distance-1 passes merge up to half of a tile's clusters: every wave of a tile has table entries to write."""
     check_build(ctx, scenes.soup(300001, seed=sd), sd, sdt, 3, 64)
+
+
+@pytest.mark.parametrize("n", [4194304, 4194305])
+def test_group_limit(ctx, n):
+    """16,384 tiles and one more: the first round of passes goes by group sums, or by the scan and later ones by sums."""
+    check_build(ctx, scenes.soup(n, seed=n), 14, 0, 3, 64)
