@@ -117,8 +117,8 @@ obvhs_status obvhs_context_set_trace(obvhs_context* ctx, int enable);
  *   ploc_radius[c]    : the PlocSearchDistance a build with search distance 0 ("auto") uses for a BVH of class c;
  *                       batched builds resolve it per mesh.  Changes the tree (each result equals the build with
  *                       that distance).  Default 14.
- *   sort_items[c]     : keys per thread of the radix sort's tiles (4, 8 or 16) for a sort of class c.  Default 8.  Sorts
- *                       of at most 8,192 32-bit keys (builds of as many leaves) have no tiles.
+ *   sort_items[c]     : keys per thread of the radix sort's tiles (4, 8 or 16) for a sort of class c.  Default 8.
+ *                       Sorts of at most 8,192 32-bit keys (builds of as many leaves) have no tiles.
  *   trav_lds_depth[c] : traversal stack entries kept in LDS (4, 8 or 16) for a BVH of class c.  Default 8.
  *   trav_chunk[c]     : 1: a single-BVH traversal launch of at least 1.25 rows of 64 rays per resident wave gives each
  *                       wave interleaved rows of rays and refills a lane as soon as its ray ends; 0: only the rows

@@ -19,7 +19,7 @@
 //                before, 20K now at 2.4 GHz): the walk's 3 to 5 dependent loads 8K, the octant assignment 8.7K -> 5.7K
 //                (costs as order keys, the round's pick by two group minima instead of three-word butterflies), the
 //                primitives' gather 2.1K -> 1.1K (stored last), the level count and the items loaded side by side.
-//                1.29M triangles, 11 levels: 213 -> 191 us.
+//                1.29M triangles, 11 levels: 207 us.
 // The exponent exp2(ceil(log2(x))) (bvh2_to_cwbvh.rs:85-88) goes through the host libm's log2f in the reference;
 // a 256-entry table of per-exponent mantissa thresholds, generated from that same log2f when the context is
 // created, reproduces it with integer compares.

@@ -27,7 +27,6 @@ struct DevBuf {
     }
 };
 
-// PLOC per-pass state, double buffered on the device (pass k reads slot k&1, writes slot (k+1)&1).
 constexpr size_t PINNED_BYTES = 4096;
 
 // What a conversion's launches depend on: the BVH2 root's box, and the size and depth of the CWBVH subtree it roots.
@@ -36,6 +35,7 @@ struct CwRootInfo {
     uint32_t size, depth;
 };
 
+// PLOC per-pass state, double buffered on the device (pass k reads slot k&1, writes slot (k+1)&1).
 struct PlocState {
     uint32_t count;
     uint32_t insert;
@@ -118,8 +118,8 @@ struct obvhs_bvh2 {
     // Children are stored in PLOC pass order (the pass ranges in hist order the nodes bottom-up); false after
     // reinsertion, when bottom-up sweeps use the level lists instead.
     bool pass_ordered = true;
-    // The leaves' codes had long runs of equal tops when the tree was last built (ploc.hip): its rebuilds, over the same
-    // leaves or some of their ancestors, sort by whole codes at once.
+    // The leaves' codes had long runs of equal tops when the tree was last built (ploc.hip): its rebuilds, over the
+    // same leaves or some of their ancestors, sort by whole codes at once.
     bool long_runs = false;
 };
 

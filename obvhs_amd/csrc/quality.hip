@@ -2005,8 +2005,8 @@ obvhs_status bvh2_reinsertion(obvhs_context* ctx, obvhs_bvh2* bvh, float batch_s
                   "reinsertion sort");
         // The conflict rounds run over all candidates' places (those beyond the positive ones end at once), so that one
         // read brings the error, the count and what is left undecided.  After a step without a move the count is read
-        // first: a tree that has settled spares the rounds' 24 launches in every further step (16
-        // steps of 0.15 on settled trees: 530K triangles 4.44 -> 3.87 ms, 3,000 triangles 1.80 -> 0.94).
+        // first: a tree that has settled spares the rounds' 24 launches in every further step (16 steps of 0.15 on
+        // settled trees: 530K triangles 4.44 -> 3.87 ms, 3,000 triangles 1.80 -> 0.94).
         ReinsMisc hm;
         auto read_misc = [&]() -> obvhs_status {
             OBVHS_TRY(hipMemcpyAsync(h, misc, sizeof(ReinsMisc), hipMemcpyDeviceToHost, st), "read reinsertion state");

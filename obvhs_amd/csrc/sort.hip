@@ -217,9 +217,9 @@ __global__ void __launch_bounds__(SORT_THREADS)
     }
 }
 
-// At most SORT_ONE_MAX u32 keys: the whole sort in one workgroup, keys and values in LDS between the passes (a wave owns
-// 64 x ITEMS consecutive keys, ranked as in the downsweep).  The ranking's instructions bound it: 2,048 keys 12 us, 4,096
-// 19, 8,192 30, against 46 us and eight launches at any of these sizes.
+// At most SORT_ONE_MAX u32 keys: the whole sort in one workgroup, keys and values in LDS between the passes (a wave
+// owns 64 x ITEMS consecutive keys, ranked as in the downsweep).  The ranking's instructions bound it: 2,048 keys 12
+// us, 4,096 19, 8,192 30, against 46 us and eight launches at any of these sizes.
 constexpr int ONE_THREADS = 1024;
 constexpr int ONE_WAVES = ONE_THREADS / 64;
 static_assert(SORT_ONE_MAX == ONE_THREADS * 8, "eight keys per thread");
@@ -391,7 +391,8 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* values, bool values_identi
 
 hipError_t radix_sort_pairs32(uint32_t* keys, uint32_t* values, bool values_identity, uint32_t n, int bits,
                               void* scratch, hipStream_t stream, int items) {
-    if (n == 0 || n > SORT_ONE_MAX) return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
+    if (n == 0 || n > SORT_ONE_MAX)
+        return radix_sort_items(keys, values, values_identity, n, bits, scratch, stream, items);
     const uint32_t identity = values_identity ? 1u : 0u, passes = (uint32_t)(bits + 7) / 8u;
     if (n <= ONE_THREADS * 2u)
         k_radix_one<2><<<1, ONE_THREADS, 0, stream>>>(keys, values, identity, n, passes);

@@ -223,7 +223,7 @@ __device__ __forceinline__ bool tail_merge(float4& alo, float4& ahi, uint32_t& h
 // entries are evaluated after the last pass by height above the tail's first clusters: an entry needs only entries of
 // lower height, and there are fewer heights than passes (1,135 clusters: 14 against 29).
 // A chain of passes and entries bounds the kernel, not any throughput.  1.29M-triangle build (1,135 clusters): 182 ->
-// 120 us; of the 16.8K cycles of a late pass 9.7K had been the entries of the pass before it, 4.5K a lane's search,
+// 114 us; of the 16.8K cycles of a late pass 9.7K had been the entries of the pass before it, 4.5K a lane's search,
 // 2.9K the scan with a serial step and 3.4K a barrier that waited for the node stores.
 // R > 0: the search distance, known at compile time (the unrolled search over NaN-padded arrays); R = 0: any r.
 template <int R, int MAX>

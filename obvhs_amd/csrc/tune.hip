@@ -27,7 +27,7 @@ namespace obvhs {
 
 namespace {
 
-// Seeded 32-bit keys (an integer hash of the index), what the builds sort by (the codes' top words) for the sort timing.
+// Seeded 32-bit keys (an integer hash of the index) for the sort timing: builds sort by the codes' top words.
 __global__ void k_tune_keys(uint32_t* keys, uint32_t n) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;

@@ -28,8 +28,8 @@ def test_sizes(ctx, sd):
         check(ctx, [n] * 5, sd, range(5))
 
 
-@pytest.mark.parametrize("small,middle,large", [(4095, 3, [1]), (4096, 3, []), (4097, 4096, [1024]), (4100, 4200, [5000]),
-                                                (100, 4200, [600]), (5000, 0, [3000])])
+@pytest.mark.parametrize("small,middle,large", [(4095, 3, [1]), (4096, 3, []), (4097, 4096, [1024]),
+                                                (4100, 4200, [5000]), (100, 4200, [600]), (5000, 0, [3000])])
 def test_mixed(ctx, small, middle, large):
     rng = np.random.default_rng(small + middle)
     counts = np.concatenate([rng.integers(0, 7, small - 2), [128, 127], rng.integers(129, 140, max(middle - 2, 0)),

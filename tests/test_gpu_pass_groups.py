@@ -16,5 +16,5 @@ def test_tile_merges(ctx, sd, sdt):
 
 @pytest.mark.parametrize("n", [4194304, 4194305])
 def test_group_limit(ctx, n):
-    """16,384 tiles and one more: the first round of passes goes by group sums, or by the scan and later ones by sums."""
+    """16,384 tiles and one more: the first passes go by group sums, or by the scan and later ones by sums."""
     check_build(ctx, scenes.soup(n, seed=n), 14, 0, 3, 64)
