@@ -883,17 +883,25 @@ __global__ void __launch_bounds__(T256) k_split_prepare(const float4* __restrict
 // one workgroup that jumps over the blocks without a stop, and steps through ties in place, since a tie keeps the
 // binade and so the block totals).  A pass ends at a binade crossing, and the host starts the next one.  The split
 // thresholds of split_aabbs_preset follow.
-// A stop costs a step of the workgroup, so the head (a doubling every few elements) is added one by one and the tiles are
-// small: 57K elements 613 -> 210 us (head 4,096: 326 with 16K tiles, 240 with 8K, 210 with 4K).  19M elements: the
+// A stop costs a step of the workgroup, so the head (a doubling every few elements) is added one by one and the tiles
+// are small: 57K elements 613 -> 210 us (head 4,096: 326 with 16K tiles, 240 with 8K, 210 with 4K).  19M elements: the
 // serial launches 1.0 ms -> 0.36, the passes 0.31 -> 0.47 (span 2^18 -> 2^16).
+// A pass costs two launches and a host wait, so after one that ended within 2 * SUM_SOON elements the next span goes
+// serially again, and after two in a row that ended within SUM_DENSE (but not within SUM_SOON) the next SUM_DENSE_SPAN,
+// there in tiles of 16K, which hold few stops.  2M areas that grow over 120 octaves (a stop every 17K elements): 5,140 us
+// by the first rule alone, 3,690 with the second.  One short pass, as any scene has, is no such stretch (2M soup: 589
+// us, 861 if it were taken for one).
 constexpr int SUM_THREADS = 1024;
-constexpr int SUM_ITEMS = 4;  // serial tile: 4K elements
-constexpr uint32_t SUM_TILE = SUM_THREADS * SUM_ITEMS;
+constexpr int SUM_ITEMS = 4;         // elements per thread of a serial tile at the start
+constexpr int SUM_DENSE_ITEMS = 16;  // and in a dense stretch after it
 constexpr uint32_t SUM_CAP = 1u << 24;
 constexpr uint32_t SUM_NONE = 0xffffffffu;
 constexpr uint32_t SUM_SERIAL_SPAN = 1u << 16;
+constexpr uint32_t SUM_SOON = 1u << 13;
+constexpr uint32_t SUM_DENSE = 1u << 16;
+constexpr uint32_t SUM_DENSE_SPAN = 1u << 18;
 constexpr uint32_t SUM_HEAD = 4096;  // elements added one by one
-static_assert(SUM_HEAD <= SUM_TILE, "the head comes from the first tile");
+static_assert(SUM_HEAD <= SUM_THREADS * SUM_ITEMS, "the head comes from the first tile");
 constexpr int PASS_ITEMS = 16;
 constexpr uint32_t PASS_BLOCK = T256 * PASS_ITEMS;  // elements per k_sum_blocks workgroup
 constexpr int PASS_TILE_ITEMS = PASS_BLOCK / SUM_THREADS;
@@ -1043,28 +1051,30 @@ __device__ __forceinline__ void split_finish(SplitMisc* misc, float s, uint32_t 
     misc->thresh_high = fmaxf(avg * 4.0f, avg * 0.9f + largest * 0.1f);  // splits.rs:28
 }
 
-// From the state (misc->sum, misc->sum_pos), 4K-element tiles until the position reaches `limit` (or the sum turns
-// NaN).  The tiles go through LDS, one pad word after every SUM_ITEMS elements: filled by lane-contiguous loads and
-// read back as each thread's SUM_ITEMS consecutive elements (thread stride SUM_ITEMS + 1 words); the next tile is
-// loaded while the current one is scanned.
+// From the state (misc->sum, misc->sum_pos), tiles of 1,024 x ITEMS elements until the position reaches `limit` (or the
+// sum turns NaN).  The tiles go through LDS, one pad word after every ITEMS elements: filled by lane-contiguous loads
+// and read back as each thread's ITEMS consecutive elements (thread stride ITEMS + 1 words); the next tile is loaded
+// while the current one is scanned.
+template <int ITEMS>
 __global__ void __launch_bounds__(SUM_THREADS) k_sum_serial(const float* __restrict__ ha, uint32_t n, uint32_t limit,
                                                            SplitMisc* misc) {
-    __shared__ float tile[SUM_TILE + SUM_TILE / SUM_ITEMS];
+    constexpr uint32_t SUM_TILE = SUM_THREADS * ITEMS;
+    __shared__ float tile[SUM_TILE + SUM_TILE / ITEMS];
     __shared__ SumShared sh;
     const uint32_t tid = threadIdx.x;
-    float nxt[SUM_ITEMS];
+    float nxt[ITEMS];
     auto load_tile = [&](uint32_t base) {
 #pragma unroll
-        for (int r = 0; r < SUM_ITEMS; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint64_t k = (uint64_t)base + (uint32_t)r * SUM_THREADS + tid;
             nxt[r] = k < n ? ha[k] : 0.0f;
         }
     };
     auto store_tile = [&]() {
 #pragma unroll
-        for (int r = 0; r < SUM_ITEMS; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint32_t e = (uint32_t)r * SUM_THREADS + tid;
-            tile[e + e / SUM_ITEMS] = nxt[r];
+            tile[e + e / ITEMS] = nxt[r];
         }
     };
     float s = misc->sum;  // the running sum, identical in every thread
@@ -1078,12 +1088,12 @@ __global__ void __launch_bounds__(SUM_THREADS) k_sum_serial(const float* __restr
         const uint32_t head = min(SUM_HEAD, n);
         if (tid < 64u) {
             uint32_t e = 0u;
-            for (; e + SUM_ITEMS <= head; e += SUM_ITEMS) {
-                const float* const v = &tile[e + e / SUM_ITEMS];
+            for (; e + ITEMS <= head; e += ITEMS) {
+                const float* const v = &tile[e + e / ITEMS];
 #pragma unroll
-                for (int r = 0; r < SUM_ITEMS; ++r) s += v[r];
+                for (int r = 0; r < ITEMS; ++r) s += v[r];
             }
-            for (; e < head; ++e) s += tile[e + e / SUM_ITEMS];
+            for (; e < head; ++e) s += tile[e + e / ITEMS];
             if (tid == 0) sh.s_after = s;
         }
         __syncthreads();
@@ -1100,7 +1110,7 @@ __global__ void __launch_bounds__(SUM_THREADS) k_sum_serial(const float* __restr
         if (tile_len < n - pos) load_tile(pos + SUM_TILE);  // the next tile when this one has no stop
         const SumMode md = sum_mode(s);
         const SumStep o =
-            sum_step<SUM_ITEMS>(md, 0ull, tile_len, [&](uint32_t e) { return tile[e + e / SUM_ITEMS]; }, sh);
+            sum_step<ITEMS>(md, 0ull, tile_len, [&](uint32_t e) { return tile[e + e / ITEMS]; }, sh);
         const uint32_t prev = pos;
         if (o.idx == SUM_NONE) {
             s = sum_value(md, o.total);
@@ -2117,12 +2127,13 @@ obvhs_status presplit_leaves(obvhs_context* ctx, const obvhs_triangle* d_tris, u
     k_split_prepare<<<std::min(nblk, PREPARE_MAX_BLOCKS), T256, 0, st>>>(tris, n, Q.split_aabbs.as<float4>(), Q.split_indices.as<uint32_t>(),
                                            Q.ha.as<float>(), misc);
     {  // the exact running sum: one workgroup over its first SUM_SERIAL_SPAN elements, then passes over all CUs
-        k_sum_serial<<<1, SUM_THREADS, 0, st>>>(Q.ha.as<float>(), n, std::min(n, SUM_SERIAL_SPAN), misc);
+        k_sum_serial<SUM_ITEMS><<<1, SUM_THREADS, 0, st>>>(Q.ha.as<float>(), n, std::min(n, SUM_SERIAL_SPAN), misc);
         OBVHS_TRY(hipGetLastError(), "sum launch");
         unsigned long long* bsum = Q.sums.as<unsigned long long>();
         uint32_t* bstop = reinterpret_cast<uint32_t*>(bsum + max_nb);
         uint32_t start = 0;
         bool last_pass = false;
+        uint32_t shorts = 0;  // passes in a row that ended within SUM_DENSE elements
         while (n > SUM_SERIAL_SPAN) {
             OBVHS_TRY(hipMemcpyAsync(h, &misc->sum, 8, hipMemcpyDeviceToHost, st), "read sum");
             OBVHS_TRY(hipStreamSynchronize(st), "sum sync");
@@ -2131,17 +2142,22 @@ obvhs_status presplit_leaves(obvhs_context* ctx, const obvhs_triangle* d_tris, u
             memcpy(&sum, h, 4);
             memcpy(&pos, h + 1, 4);
             if (pos >= n || std::isnan(sum)) break;
-            const bool dense = last_pass && pos - start < SUM_SERIAL_SPAN / 4;  // the last pass ended soon
+            if (last_pass) shorts = pos - start < SUM_DENSE ? shorts + 1 : 0;
+            const bool soon = last_pass && pos - start < (shorts > 1 ? SUM_SOON : 2 * SUM_SOON);
+            const bool dense = last_pass && shorts > 1;
             start = pos;
-            if (dense) {
-                k_sum_serial<<<1, SUM_THREADS, 0, st>>>(
+            if (soon) {
+                k_sum_serial<SUM_ITEMS><<<1, SUM_THREADS, 0, st>>>(
                     Q.ha.as<float>(), n, (uint32_t)std::min<uint64_t>(n, (uint64_t)pos + SUM_SERIAL_SPAN), misc);
+            } else if (dense) {
+                k_sum_serial<SUM_DENSE_ITEMS><<<1, SUM_THREADS, 0, st>>>(
+                    Q.ha.as<float>(), n, (uint32_t)std::min<uint64_t>(n, (uint64_t)pos + SUM_DENSE_SPAN), misc);
             } else {
                 const uint32_t nb = (n - pos + PASS_BLOCK - 1) / PASS_BLOCK;
                 k_sum_blocks<<<nb, T256, 0, st>>>(Q.ha.as<float>(), n, pos, sum, bsum, bstop);
                 k_sum_pass<<<1, SUM_THREADS, 0, st>>>(Q.ha.as<float>(), n, pos, sum, nb, bsum, bstop, misc);
             }
-            last_pass = !dense;
+            last_pass = !soon && !dense;
             OBVHS_TRY(hipGetLastError(), "sum pass launch");
         }
     }
