@@ -888,9 +888,9 @@ __global__ void __launch_bounds__(T256) k_split_prepare(const float4* __restrict
 // serial launches 1.0 ms -> 0.36, the passes 0.31 -> 0.47 (span 2^18 -> 2^16).
 // A pass costs two launches and a host wait, so after one that ended within 2 * SUM_SOON elements the next span goes
 // serially again, and after two in a row that ended within SUM_DENSE (but not within SUM_SOON) the next SUM_DENSE_SPAN,
-// there in tiles of 16K, which hold few stops.  2M areas that grow over 120 octaves (a stop every 17K elements): 5,140 us
-// by the first rule alone, 3,690 with the second.  One short pass, as any scene has, is no such stretch (2M soup: 589
-// us, 861 if it were taken for one).
+// there in tiles of 16K, which hold few stops.  2M areas that grow over 120 octaves (a stop every 17K elements): 5,140
+// us by the first rule alone, 3,690 with the second.  One short pass, as any scene has, is no such stretch (2M soup:
+// 589 us, 861 if it were taken for one).
 constexpr int SUM_THREADS = 1024;
 constexpr int SUM_ITEMS = 4;         // elements per thread of a serial tile at the start
 constexpr int SUM_DENSE_ITEMS = 16;  // and in a dense stretch after it

@@ -1,6 +1,6 @@
-"""Pre-splits of triangles whose areas grow along the array: the running sum leaves its binade every few thousand elements
-to the end, so it goes serially in small tiles, in large ones, or in passes by the distance of the stops.  Split boxes
-and indices equal the oracle's, whose thresholds come from the sum in order."""
+"""Pre-splits of triangles whose areas grow along the array: the running sum leaves its binade every few thousand
+elements to the end, so it goes serially in small tiles, in large ones, or in passes by the distance of the stops.
+Split boxes and indices equal the oracle's, whose thresholds come from the sum in order."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,8 @@ from test_gpu_parity import assert_same_bytes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,octaves", [(150000, 75), (200000, 20), (400000, 30), (400000, 13), (600001, 10), (600001, 0)])
+@pytest.mark.parametrize("n,octaves", [(150000, 75), (200000, 20), (400000, 30), (400000, 13), (600001, 10),
+                                       (600001, 0)])
 def test_growing_areas(ctx, n, octaves):
     rng = np.random.default_rng(n + octaves)
     size = 1e-4 * np.exp2(np.arange(n) * (octaves / 2 / n))
